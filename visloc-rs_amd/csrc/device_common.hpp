@@ -167,57 +167,155 @@ __device__ __forceinline__ void sym6_mul(const double* U, const double* x, doubl
     }
 }
 
-// Sum over the terms k = first, first + stride, ... of block b's term list
-// (landmark l, edge of p, edge of q) of the Schur terms
-// W_p V_l^-1 W_q^T = [[C, -C K], [K C, -K C K]], C = G_p V_l^-1 G_q,
-// K = [X_l]x, into acc (row-major 6x6, zeroed here).
-__device__ __forceinline__ void schur_block_terms(const DevProblem& P, const DensePairs& D, int b, int first,
-                                                  int stride, double acc[36]) {
+__device__ __forceinline__ double from_halves(unsigned lo, unsigned hi) {
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The value of the partner lane under DPP control CTRL (within a row).
+template <int CTRL>
+__device__ __forceinline__ double dpp_partner(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xf, 0xf, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+    return from_halves(lo, hi);
+}
+
+// One halving step of wave_sum36: the lane and its partner sum a where the
+// lane's `upper` is false and b where it is true.
+template <int CTRL>
+__device__ __forceinline__ double halve_dpp(double a, double b, bool upper) {
+    return (upper ? b : a) + dpp_partner<CTRL>(upper ? a : b);
+}
+__device__ __forceinline__ double halve_rows(double a, double b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a),
+                             y = (unsigned long long)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return from_halves(lo[0], hi[0]) + from_halves(lo[1], hi[1]);
+}
+__device__ __forceinline__ double halve_wave(double a, double b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a),
+                             y = (unsigned long long)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return from_halves(lo[0], hi[0]) + from_halves(lo[1], hi[1]);
+}
+
+// Sums of 36 values over a wave, one sum per lane: a lane of each pair keeps
+// half of the values and takes the partner's part of them (halves of the
+// wave, row pairs, then mirror and neighbour lanes: 36, 18, 9, 5, 3, 2, 1
+// values), in 38 exchanges where a butterfly that leaves every sum in every
+// lane takes 216. Fixed order; all lanes must be active. The lane's sum is
+// entry wave_entry36(lane); lanes with -1 hold none.
+__device__ __forceinline__ double wave_sum36(const double v[36], int lane) {
+    double a[18], b[9], c[5], d[3], e[2];
+#pragma unroll
+    for (int i = 0; i < 18; ++i) a[i] = halve_wave(v[i], v[i + 18]);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) b[i] = halve_rows(a[i], a[i + 9]);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) c[i] = halve_dpp<0x140>(b[i], i < 4 ? b[i + 5] : 0.0, lane & 8);  // row_mirror
+#pragma unroll
+    for (int i = 0; i < 3; ++i) d[i] = halve_dpp<0x141>(c[i], i < 2 ? c[i + 3] : 0.0, lane & 4);  // row_half_mirror
+    e[0] = halve_dpp<0x4E>(d[0], d[2], lane & 2);  // quad_perm [2,3,0,1]
+    e[1] = halve_dpp<0x4E>(d[1], 0.0, lane & 2);
+    return halve_dpp<0xB1>(e[0], e[1], lane & 1);  // quad_perm [1,0,3,2]
+}
+__device__ __forceinline__ int wave_entry36(int lane) {
+    const int t = (lane & 2) + (lane & 1);                 // of 3 (0, 1; 2)
+    const int u = ((lane & 4) ? 3 : 0) + t;                // of 5 (0..2; 3, 4)
+    const int w = ((lane & 8) ? 5 : 0) + u;                // of 9 (0..4; 5..8)
+    if (t > 2 || ((lane & 4) && t > 1) || ((lane & 8) && u > 3)) return -1;
+    return ((lane & 32) ? 18 : 0) + ((lane & 16) ? 9 : 0) + w;
+}
+
+// Block b of sum_l W_p V_l^-1 W_q^T over its term list (landmark l, edge of
+// p, edge of q), W_p V_l^-1 W_q^T = [[C, -C K], [K C, -K C K]] with
+// C = G_p V_l^-1 G_q and K = [X_l]x, by one wave: entry wave_entry36(lane)
+// (row-major 6x6) in each lane. Lane t adds terms t, t + 64, ... in order.
+//
+// A term is a chain of two dependent gathers (its indices, then 168 bytes of
+// blocks) and 126 FP64 operations, so what bounds the sum is how many terms
+// are in flight: a whole wave per block, the next term's indices loaded with
+// this term's blocks, 16-byte loads. Consecutive terms' landmarks and edges
+// lie near one another in storage, so the lanes of a gather share lines.
+// Eight lanes per block, each walking an eighth of the list, took 594 us for
+// the 50-camera circle's 6.4M terms against 103 us here, 821 us for 64 stereo
+// windows (longest list about 1,200 terms) against 158 us, and 635 us for a
+// 2.3M-observation loop's 17M terms against 576 us: that one reads 2.9 GB of
+// blocks through L1 and is bound there.
+__device__ __forceinline__ double schur_block_wave(const DevProblem& P, const DensePairs& D, int b, int lane) {
+    double acc[36];
 #pragma unroll
     for (int i = 0; i < 36; ++i) acc[i] = 0.0;
-    for (int k = D.block_ptr[b] + first; k < D.block_ptr[b + 1]; k += stride) {
-        const int l = D.terms[3 * (size_t)k], ep = D.terms[3 * (size_t)k + 1], eq = D.terms[3 * (size_t)k + 2];
-        const double* Vi = P.Vinv64 + 6 * (size_t)l;
-        const double vi[9] = {Vi[0], Vi[1], Vi[2], Vi[1], Vi[3], Vi[4], Vi[2], Vi[4], Vi[5]};
-        const double* A = P.Gl64 + 6 * (size_t)ep;
-        const double* B = P.Gl64 + 6 * (size_t)eq;
-        const double a[9] = {A[0], A[1], A[2], A[1], A[3], A[4], A[2], A[4], A[5]};
-        const double bb[9] = {B[0], B[1], B[2], B[1], B[3], B[4], B[2], B[4], B[5]};
-        double T[9], C[9];
+    const int end = D.block_ptr[b + 1];
+    int k = D.block_ptr[b] + lane;
+    if (k < end) {
+        const int32_t* t = D.terms + 3 * (size_t)k;
+        int l = t[0], ep = t[1], eq = t[2];
+        while (true) {
+            const double2* v2 = (const double2*)(P.Vinv64 + 6 * (size_t)l);
+            const double2* a2 = (const double2*)(P.Gl64 + 6 * (size_t)ep);
+            const double2* b2 = (const double2*)(P.Gl64 + 6 * (size_t)eq);
+            const double* X = P.lms + 3 * (size_t)l;
+            const double2 v01 = v2[0], v23 = v2[1], v45 = v2[2];
+            const double2 p01 = a2[0], p23 = a2[1], p45 = a2[2];
+            const double2 q01 = b2[0], q23 = b2[1], q45 = b2[2];
+            const double x0 = X[0], x1 = X[1], x2 = X[2];
+            k += 64;
+            const int32_t* tn = D.terms + 3 * (size_t)min(k, end - 1);
+            l = tn[0];
+            ep = tn[1];
+            eq = tn[2];
+            const double vi[9] = {v01.x, v01.y, v23.x, v01.y, v23.y, v45.x, v23.x, v45.x, v45.y};
+            const double gp[9] = {p01.x, p01.y, p23.x, p01.y, p23.y, p45.x, p23.x, p45.x, p45.y};
+            const double gq[9] = {q01.x, q01.y, q23.x, q01.y, q23.y, q45.x, q23.x, q45.x, q45.y};
+            double T[9], C[9], CK[9];
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+            for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) T[3 * i + j] = a[3 * i] * vi[j] + a[3 * i + 1] * vi[3 + j] + a[3 * i + 2] * vi[6 + j];
+                for (int j = 0; j < 3; ++j)
+                    T[3 * i + j] = fma(gp[3 * i + 2], vi[6 + j], fma(gp[3 * i + 1], vi[3 + j], gp[3 * i] * vi[j]));
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+            for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) C[3 * i + j] = T[3 * i] * bb[j] + T[3 * i + 1] * bb[3 + j] + T[3 * i + 2] * bb[6 + j];
-        const double* X = P.lms + 3 * (size_t)l;
-        const double K[9] = {0.0, -X[2], X[1], X[2], 0.0, -X[0], -X[1], X[0], 0.0};
-        double CK[9], KC[9], KCK[9];
+                for (int j = 0; j < 3; ++j)
+                    C[3 * i + j] = fma(T[3 * i + 2], gq[6 + j], fma(T[3 * i + 1], gq[3 + j], T[3 * i] * gq[j]));
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                CK[3 * i + j] = C[3 * i] * K[j] + C[3 * i + 1] * K[3 + j] + C[3 * i + 2] * K[6 + j];
-                KC[3 * i + j] = K[3 * i] * C[j] + K[3 * i + 1] * C[3 + j] + K[3 * i + 2] * C[6 + j];
+            for (int i = 0; i < 3; ++i) {
+                CK[3 * i] = fma(C[3 * i + 1], x2, -(C[3 * i + 2] * x1));
+                CK[3 * i + 1] = fma(C[3 * i + 2], x0, -(C[3 * i] * x2));
+                CK[3 * i + 2] = fma(C[3 * i], x1, -(C[3 * i + 1] * x0));
             }
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) KCK[3 * i + j] = KC[3 * i] * K[j] + KC[3 * i + 1] * K[3 + j] + KC[3 * i + 2] * K[6 + j];
-        // [[C, -C K], [K C, -K C K]]
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
             for (int j = 0; j < 3; ++j) {
-                acc[6 * i + j] += C[3 * i + j];
-                acc[6 * i + 3 + j] -= CK[3 * i + j];
-                acc[6 * (3 + i) + j] += KC[3 * i + j];
-                acc[6 * (3 + i) + 3 + j] -= KCK[3 * i + j];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    acc[6 * i + j] += C[3 * i + j];
+                    acc[6 * i + 3 + j] -= CK[3 * i + j];
+                }
+                // K C and -K (C K), row by row of K
+                acc[18 + j] = fma(x1, C[6 + j], fma(-x2, C[3 + j], acc[18 + j]));
+                acc[24 + j] = fma(x2, C[j], fma(-x0, C[6 + j], acc[24 + j]));
+                acc[30 + j] = fma(x0, C[3 + j], fma(-x1, C[j], acc[30 + j]));
+                acc[21 + j] = fma(-x1, CK[6 + j], fma(x2, CK[3 + j], acc[21 + j]));
+                acc[27 + j] = fma(-x2, CK[j], fma(x0, CK[6 + j], acc[27 + j]));
+                acc[33 + j] = fma(-x0, CK[3 + j], fma(x1, CK[j], acc[33 + j]));
             }
+            if (k >= end) break;
+        }
     }
+    return wave_sum36(acc, lane);
 }
+
+// The block of this wave of a kBlock launch over block_grid(num_blocks), one block per wave, neighbouring blocks
+// (which share edges) on one XCD.
+__device__ __forceinline__ int block_of_wave(int num_blocks) {
+    constexpr int kWaves = kBlock / 64;
+    const int wg = xcd_tile(blockIdx.x, (num_blocks + kWaves - 1) / kWaves);
+    return __builtin_amdgcn_readfirstlane(wg * kWaves + (int)(threadIdx.x >> 6));
+}
+inline int block_grid(int num_blocks) { return xcd_grid(blocks_for(num_blocks, kBlock / 64)); }
 
 // 6x6 Cholesky inverse; false for a non-positive or non-finite pivot.
 // Every loop is unrolled, so that L and y stay in registers (dynamic

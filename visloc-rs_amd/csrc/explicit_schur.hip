@@ -7,10 +7,9 @@
 // one assembly per LM iteration each PCG product reads 36 values per stored
 // block instead of streaming every edge's G.
 //
-// Assembly: a group of 8 lanes per upper block sums the block's term list
-// (one term per landmark the two poses share, in landmark order) with a
-// fixed-order butterfly, then writes S_pq and its transpose S_qp. Products:
-// one wave per block row, 48 lanes as 6 rows x 8 column-block groups.
+// Assembly: one wave per upper block sums the block's term list (one term per
+// landmark the two poses share, in landmark order) in a fixed order, then
+// writes S_pq and its transpose S_qp. Products: one wave per block row, 48 lanes as 6 rows x 8 column-block groups.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -22,51 +21,31 @@ namespace vba {
 
 namespace {
 
-constexpr int kTermLanes = 8;  // lanes per block in the assembly
-
-// One upper block per 8-lane group: S_pq = [p == q](U_p + lambda I) - sum of
-// its terms, stored row-major at block_pos[2b] and transposed at
+// One upper block per wave: S_pq = [p == q](U_p + lambda I) - sum of its
+// terms, stored row-major at block_pos[2b] and transposed at
 // block_pos[2b + 1]. The diagonal block keeps its upper triangle and mirrors
 // it, so that it is exactly symmetric.
-__global__ __launch_bounds__(kBlock) void k_explicit_assemble(DevProblem P, DensePairs D, ExplicitDev X,
+__global__ __launch_bounds__(kBlock, 4) void k_explicit_assemble(DevProblem P, DensePairs D, ExplicitDev X,
                                                                double lambda) {
-    const int b = blockIdx.x * (kBlock / kTermLanes) + (int)threadIdx.x / kTermLanes;
+    const int b = block_of_wave(D.num_blocks);
     if (b >= D.num_blocks) return;
-    const int g = threadIdx.x % kTermLanes;
-    double acc[36];
-    schur_block_terms(P, D, b, g, kTermLanes, acc);
-#pragma unroll
-    for (int off = 1; off < kTermLanes; off <<= 1)
-#pragma unroll
-        for (int i = 0; i < 36; ++i) acc[i] += __shfl_xor(acc[i], off, kTermLanes);
+    const int lane = threadIdx.x & 63;
+    double v = -schur_block_wave(P, D, b, lane);
     const int sp = D.block_pq[2 * b], sq = D.block_pq[2 * b + 1];
-    const int pos = X.block_pos[2 * b], pos_t = X.block_pos[2 * b + 1];
-    const double* U = P.U + 21 * (size_t)sp;
-#pragma unroll
-    for (int idx0 = 0; idx0 < 36; idx0 += kTermLanes) {
-        const int idx = idx0 + g;
-        if (idx < 36) {
-            const int i = idx / 6, j = idx % 6;
-            double v = 0.0;
-            if (sp == sq) {
-                const int src = i <= j ? idx : 6 * j + i;
-#pragma unroll
-                for (int t = 0; t < 36; ++t)
-                    if (t == src) v = acc[t];
-                v = U[i <= j ? up6(i, j) : up6(j, i)] + (i == j && lambda > 0.0 ? lambda : 0.0) - v;
-            } else {
-#pragma unroll
-                for (int t = 0; t < 36; ++t)
-                    if (t == idx) v = acc[t];
-                v = -v;
-            }
-            X.S64[36 * (size_t)pos + idx] = v;
-            if (X.S32) X.S32[36 * (size_t)pos + idx] = (float)v;
-            if (pos_t >= 0) {
-                X.S64[36 * (size_t)pos_t + 6 * j + i] = v;
-                if (X.S32) X.S32[36 * (size_t)pos_t + 6 * j + i] = (float)v;
-            }
-        }
+    const int pos = X.block_pos[2 * b], idx = wave_entry36(lane);
+    if (idx < 0) return;
+    const int i = idx / 6, j = idx % 6, tidx = 6 * j + i;
+    int pos_t = X.block_pos[2 * b + 1];
+    if (sp == sq) {
+        if (i > j) return;
+        v = P.U[21 * (size_t)sp + up6(i, j)] + (i == j && lambda > 0.0 ? lambda : 0.0) + v;
+        pos_t = i < j ? pos : -1;
+    }
+    X.S64[36 * (size_t)pos + idx] = v;
+    if (X.S32) X.S32[36 * (size_t)pos + idx] = (float)v;
+    if (pos_t >= 0) {
+        X.S64[36 * (size_t)pos_t + tidx] = v;
+        if (X.S32) X.S32[36 * (size_t)pos_t + tidx] = (float)v;
     }
 }
 
@@ -198,8 +177,7 @@ __global__ __launch_bounds__(kBlock) void k_explicit_true_pose(DevProblem P, Exp
 void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, double lambda,
                               hipStream_t s) {
     if (D.num_blocks)
-        hipLaunchKernelGGL(k_explicit_assemble, dim3(blocks_for(D.num_blocks, kBlock / kTermLanes)), dim3(kBlock), 0,
-                           s, P, D, X, lambda);
+        hipLaunchKernelGGL(k_explicit_assemble, dim3(block_grid(D.num_blocks)), dim3(kBlock), 0, s, P, D, X, lambda);
     hipLaunchKernelGGL(k_explicit_precond, dim3(blocks_for(P.num_pose_slots, kBlock)), dim3(kBlock), 0, s, P, X);
 }
 

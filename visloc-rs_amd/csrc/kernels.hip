@@ -503,51 +503,31 @@ __global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, 
 // one-work-group Cholesky with an LU fallback (pose_graph.rs:2259-2270).
 // ---------------------------------------------------------------------------
 // One 6x6 block (p, q) of S = U + lambda I - W V^-1 W^T, written at the
-// variable indices local to its system (and mirrored when p != q).
-// Lanes that assemble one 6x6 block of S together.
-constexpr int kBlockLanes = 8;
-
-// One 6x6 block (p, q) of S = U + lambda I - W V^-1 W^T, written at the
-// variable indices local to its system (and mirrored when p != q), by a
-// group of kBlockLanes lanes: each sums a strided share of the block's terms,
-// a butterfly within the group combines them in a fixed order.
-__device__ void dense_assemble_group(const DevProblem& P, const DensePairs& D, int b, double* S, int n, int var_begin,
-                                     double lambda, int g) {
+// variable indices local to its system (and mirrored when p != q), by one
+// wave: every lane with an entry of the block's sum writes it.
+__device__ __forceinline__ void dense_assemble_wave(const DevProblem& P, const DensePairs& D, int b, double* S, int n,
+                                                    int var_begin, double lambda, int lane) {
     const int sp = D.block_pq[2 * b], sq = D.block_pq[2 * b + 1];
+    const double v = schur_block_wave(P, D, b, lane);
+    const int idx = wave_entry36(lane);
+    if (idx < 0) return;
     const int vp = P.pose_var[sp] - var_begin, vq = P.pose_var[sq] - var_begin;
-    double acc[36];
-    schur_block_terms(P, D, b, g, kBlockLanes, acc);
-#pragma unroll
-    for (int off = 1; off < kBlockLanes; off <<= 1)
-#pragma unroll
-        for (int i = 0; i < 36; ++i) acc[i] += __shfl_xor(acc[i], off, kBlockLanes);
-    // every lane holds the sum; lane g writes entries g, g + 8, ...
-    const double* U = P.U + 21 * (size_t)sp;
-#pragma unroll
-    for (int idx0 = 0; idx0 < 36; idx0 += kBlockLanes) {
-        const int idx = idx0 + g;
-        if (idx < 36) {
-            const int i = idx / 6, j = idx % 6;
-            double v = 0.0;
-#pragma unroll
-            for (int t = 0; t < 36; ++t)
-                if (t == idx) v = acc[t];
-            if (sp == sq) {
-                const double u = U[i <= j ? up6(i, j) : up6(j, i)] + (i == j && lambda > 0.0 ? lambda : 0.0);
-                S[(size_t)(6 * vp + i) * n + 6 * vq + j] = u - v;
-            } else {
-                S[(size_t)(6 * vp + i) * n + 6 * vq + j] = -v;
-                S[(size_t)(6 * vq + j) * n + 6 * vp + i] = -v;
-            }
-        }
+    const int i = idx / 6, j = idx % 6;
+    if (sp == sq) {
+        const double* U = P.U + 21 * (size_t)sp;
+        const double u = U[i <= j ? up6(i, j) : up6(j, i)] + (i == j && lambda > 0.0 ? lambda : 0.0);
+        S[(size_t)(6 * vp + i) * n + 6 * vq + j] = u - v;
+    } else {
+        S[(size_t)(6 * vp + i) * n + 6 * vq + j] = -v;
+        S[(size_t)(6 * vq + j) * n + 6 * vp + i] = -v;
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_dense_assemble(DevProblem P, DensePairs D, double* S, int n,
+__global__ __launch_bounds__(kBlock, 4) void k_dense_assemble(DevProblem P, DensePairs D, double* S, int n,
                                                            double lambda) {
-    const int b = blockIdx.x * (kBlock / kBlockLanes) + (int)threadIdx.x / kBlockLanes;
+    const int b = block_of_wave(D.num_blocks);
     if (b >= D.num_blocks) return;
-    dense_assemble_group(P, D, b, S, n, 0, lambda, threadIdx.x % kBlockLanes);
+    dense_assemble_wave(P, D, b, S, n, 0, lambda, threadIdx.x & 63);
 }
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -1048,15 +1028,15 @@ __global__ __launch_bounds__(kSmallBlock) void k_dense_solve_plain(double* S, do
 // every window at once, with per-window lambda, cost and accept/reject kept
 // on the device (no host round trip per iteration).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_batch_dense_assemble(DevProblem P, DensePairs D, BatchDev B) {
-    const int b = blockIdx.x * (kBlock / kBlockLanes) + (int)threadIdx.x / kBlockLanes;
+__global__ __launch_bounds__(kBlock, 4) void k_batch_dense_assemble(DevProblem P, DensePairs D, BatchDev B) {
+    const int b = block_of_wave(D.num_blocks);
     if (b >= D.num_blocks) return;
     const int w = P.pose_win[D.block_pq[2 * b]];
     const WindowState& st = B.state[w];
     if (!st.active) return;
     const WindowLayout L = B.layout[w];
-    dense_assemble_group(P, D, b, B.S + L.s_offset, 6 * (L.var_end - L.var_begin), L.var_begin, st.lambda,
-                         threadIdx.x % kBlockLanes);
+    dense_assemble_wave(P, D, b, B.S + L.s_offset, 6 * (L.var_end - L.var_begin), L.var_begin, st.lambda,
+                        threadIdx.x & 63);
 }
 
 __global__ __launch_bounds__(kBlock) void k_batch_dense_zero(DevProblem P, BatchDev B) {
@@ -1636,8 +1616,7 @@ size_t joint_part_size(const DevProblem& P) {
 void launch_dense_assemble(const DevProblem& P, const DensePairs& D, double* S, int32_t n, double lambda,
                            hipStream_t s) {
     if (D.num_blocks)
-        hipLaunchKernelGGL(k_dense_assemble, dim3(blocks_for(D.num_blocks, kBlock / kBlockLanes)), dim3(kBlock), 0, s, P,
-                           D, S, n, lambda);
+        hipLaunchKernelGGL(k_dense_assemble, dim3(block_grid(D.num_blocks)), dim3(kBlock), 0, s, P, D, S, n, lambda);
 }
 namespace {
 // The device-wide factor and the finishing solve (n > kDenseOneGroupMax).
@@ -1683,8 +1662,7 @@ hipError_t launch_dense_solve_plain(double* S, double* work, const double* b, do
 }
 void launch_batch_dense_assemble(const DevProblem& P, const DensePairs& D, const BatchDev& B, hipStream_t s) {
     if (D.num_blocks)
-        hipLaunchKernelGGL(k_batch_dense_assemble, dim3(blocks_for(D.num_blocks, kBlock / kBlockLanes)), dim3(kBlock),
-                           0, s, P, D, B);
+        hipLaunchKernelGGL(k_batch_dense_assemble, dim3(block_grid(D.num_blocks)), dim3(kBlock), 0, s, P, D, B);
 }
 void launch_batch_dense_zero(const DevProblem& P, const BatchDev& B, hipStream_t s) {
     if (B.num_windows) hipLaunchKernelGGL(k_batch_dense_zero, dim3(16, B.num_windows), dim3(kBlock), 0, s, P, B);
