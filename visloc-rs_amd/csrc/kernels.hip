@@ -788,19 +788,14 @@ __device__ void lu_fallback_body(double* A2, double* y, int n, int* fail_sh, dou
 
 // Cholesky (blocked, MFMA trailing updates), then forward/back
 // substitution; on a non-positive pivot an LU with partial pivoting on the
-// saved copy (allow_lu, solve_normal_equations), or singular (the Sparse
-// solver's block Cholesky has no fallback). Solves S x = b for the n
-// unknowns of `io`. One work-group of NT threads.
+// copy saved first. Solves S x = b for the n unknowns of `io`. One work-group
+// of NT threads.
 template <int NT>
 __device__ void dense_solve_body(const DenseRows& io, double* S, double* work, int n, int* status, int* fail_sh,
-                                 double* piv_val, int* piv_idx, double* dblk, bool copied = false,
-                                 bool allow_lu = true) {
+                                 double* piv_val, int* piv_idx, double* dblk) {
     double* A2 = work;                 // n*n copy for the LU fallback
     double* y = work + (size_t)n * n;  // n
-    // the saved copy for the LU fallback, unless the whole device made it
-    // before this work-group started
-    if (!copied && allow_lu)
-        for (size_t k = threadIdx.x; k < (size_t)n * n; k += NT) A2[k] = S[k];
+    for (size_t k = threadIdx.x; k < (size_t)n * n; k += NT) A2[k] = S[k];
     for (int i = threadIdx.x; i < n; i += NT) y[i] = io.rhs(i);
     if (threadIdx.x == 0) *fail_sh = 0;
     __syncthreads();
@@ -808,18 +803,232 @@ __device__ void dense_solve_body(const DenseRows& io, double* S, double* work, i
     __syncthreads();
     if (!*fail_sh) {
         chol_blocked_solve<NT>(S, n, y, dblk);
-    } else if (allow_lu) {
+    } else {
         // LU with partial pivoting on A2; y holds b again.
         for (int i = threadIdx.x; i < n; i += NT) y[i] = io.rhs(i);
         __syncthreads();
         lu_fallback_body<NT>(A2, y, n, fail_sh, piv_val, piv_idx);
-    } else {
-        if (threadIdx.x == 0) *fail_sh = 2;
     }
     __syncthreads();
     const int f = *fail_sh;
     for (int i = threadIdx.x; i < n; i += NT) io.put(i, (f != 2) ? y[i] : 0.0);
     if (threadIdx.x == 0) *status = (f == 2) ? 1 : 0;
+}
+
+// One wave, one row of 16 columns per lane: lanes 0..15 hold the rows of a
+// diagonal block A_kk, every other lane a row A_r of the panel below it. On
+// return lanes 0..15 hold L_kk (their upper parts are not defined) and the
+// others A_r L_kk^-T, and lane j < 16 gets 1 / L_kk[j][j] in *rinv. False on
+// a pivot that is not positive and finite (the same in every lane).
+//
+// The chain pivot -> reciprocal root -> column -> next pivot bounds it: the
+// root is v_rsq_f64 with two Newton steps (each squares the relative error,
+// below 2^-52 after the second), and pivots and column entries come by lane
+// reads, which need no LDS and no barrier.
+__device__ __forceinline__ bool chol16_rows(double a[16], int lane, double* rinv) {
+    double ri = 0.0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const double d = lane_value(a[j], j);
+        if (!(d > 0.0) || !isfinite(d)) return false;
+        double y = __builtin_amdgcn_rsq(d);
+        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+        if (lane == j) ri = y;
+        a[j] = a[j] * y;
+#pragma unroll
+        for (int c = j + 1; c < 16; ++c) a[c] = fma(-a[j], lane_value(a[j], c), a[c]);
+    }
+    *rinv = ri;
+    return true;
+}
+
+// Dense solves of at most kDenseOneGroupMax unknowns by one work-group of
+// kSmallWaves waves: Cholesky with the matrix in registers.
+//
+// Such a solve moves little (n = 234: 0.4 MB) and computes little (4 MFLOP);
+// what bounds it is the chain of n / 16 steps, each a diagonal factor, its
+// panel and the update that the next step waits for. So the lower 16 x 16
+// tiles stay in the waves' registers (tile t of wave w: number w + kSmallWaves
+// t in column order, MFMA result layout) and a step has two barriers:
+//   1. every wave factors the diagonal tile for itself, with 47 panel rows in
+//      its other lanes (chol16_rows) and the right-hand side's 16 entries in
+//      lane 63, whose result is this step's y = L^-1 b; the row lanes then
+//      take their part of y from the right-hand side below;
+//   2. tiles to the right subtract L_i L_j^T on FP64 MFMA with operands from
+//      the LDS panel, the step's column keeps L in its tiles, and the next
+//      column's tiles go to the other panel buffer.
+// Back substitution walks the columns backwards: wave 0 solves with L_kk^T,
+// then each tile (k, j) takes its part from y_j (one tile per j, so one
+// writer). S is only read; the LU fallback overwrites it.
+// Tiles in global memory with the diagonal factored in LDS, three barriers a
+// column: 17.7 us at 6 unknowns (8.4 us here), 124 us at 72 (30 us), 474 us
+// for 64 windows of up to 234 (109 us).
+constexpr int kSmallWaves = 8;
+constexpr int kSmallTiles = 17;  // of the 136 lower tiles of 256 unknowns, per wave
+constexpr int kSmallRows = 47;   // panel rows per wave in chol16_rows
+struct SmallSolveLds {
+    double panel[2][kDenseOneGroupMax * 17];
+    double diag[kDenseOneGroupMax / 16][16 * 17];
+    double b[kDenseOneGroupMax];     // right-hand side, what is left of it
+    double y[kDenseOneGroupMax];     // L^-1 b, then the solution
+    double rinv[kDenseOneGroupMax];  // reciprocal pivots
+    double piv_val[64 * kSmallWaves];  // LU fallback
+    int piv_idx[64 * kSmallWaves];
+    int fail;
+};
+
+__device__ void dense_solve_small(const DenseRows& io, double* S, double* work, int n, int* status, int allow_lu,
+                                  SmallSolveLds& sh) {
+    constexpr int NT = 64 * kSmallWaves;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int nb = (n + 15) >> 4;
+    for (int i = tid; i < 16 * nb; i += NT) sh.b[i] = i < n ? io.rhs(i) : 0.0;
+    if (tid == 0) sh.fail = 0;
+    // this wave's tiles, row and column packed in one scalar (column nb past
+    // the last tile); reading one hides its value from the compiler, which
+    // would otherwise keep every tile's addresses in registers across steps
+    int tile[kSmallTiles];
+    auto tile_at = [&](int t, int* i, int* j) {
+        int v = tile[t];
+        asm volatile("" : "+s"(v));
+        *i = v >> 8;
+        *j = v & 255;
+    };
+    v4d acc[kSmallTiles];
+    {
+        int col = 0, first = 0;  // first tile number of column col
+#pragma unroll
+        for (int t = 0; t < kSmallTiles; ++t) {
+            const int id = wave + kSmallWaves * t;
+            while (col < nb && id >= first + nb - col) {
+                first += nb - col;
+                ++col;
+            }
+            const int row = col + id - first;
+            tile[t] = __builtin_amdgcn_readfirstlane(col < nb ? row << 8 | col : nb);
+            if (col < nb) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[t][q] = padded_at(S, n, 16 * row + 4 * q + g, 16 * col + c);
+                if (col == 0)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) sh.panel[0][(16 * row + 4 * q + g) * 17 + c] = acc[t][q];
+            }
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < nb; ++k) {
+        double* panel = sh.panel[k & 1];
+        double* next = sh.panel[(k + 1) & 1];
+        const int below = 16 * (nb - k - 1);  // panel rows
+        if (kSmallRows * wave < below || wave == 0) {
+            const int rr = kSmallRows * wave + lane - 16;  // this lane's panel row (lanes 16..62)
+            const bool mine = lane >= 16 && lane < 63 && rr < below;
+            const int row = lane < 16 ? 16 * k + lane : 16 * (k + 1) + (mine ? rr : 0);
+            double a[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) a[j] = lane == 63 ? sh.b[16 * k + j] : below || lane < 16 ? panel[row * 17 + j] : 0.0;
+            double ri;
+            if (!chol16_rows(a, lane, &ri)) {
+                if (lane == 0) sh.fail = 1;
+            } else {
+                if (mine) {
+                    double bb = sh.b[row];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) panel[row * 17 + j] = a[j];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) bb = fma(-a[j], lane_value(a[j], 63), bb);
+                    sh.b[row] = bb;
+                }
+                if (wave == 0) {
+                    if (lane < 16) {
+                        sh.rinv[16 * k + lane] = ri;
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) sh.diag[k][lane * 17 + j] = a[j];
+                    } else if (lane == 63) {
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) sh.y[16 * k + j] = a[j];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (sh.fail) break;
+#pragma unroll
+        for (int t = 0; t < kSmallTiles; ++t) {
+            int i, j;
+            tile_at(t, &i, &j);
+            if (j >= nb || j < k) continue;
+            if (j == k) {
+                if (i > k)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[t][q] = panel[(16 * i + 4 * q + g) * 17 + c];
+                continue;
+            }
+            double av[4], bv[4];
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                av[kk] = -panel[(16 * i + c) * 17 + 4 * kk + g];
+                bv[kk] = panel[(16 * j + c) * 17 + 4 * kk + g];
+            }
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[kk], bv[kk], acc[t], 0, 0, 0);
+            if (j == k + 1)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) next[(16 * i + 4 * q + g) * 17 + c] = acc[t][q];
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    if (!sh.fail) {
+        for (int k = nb - 1; k >= 0; --k) {  // backward: L^T x = y
+            if (wave == 0) {
+                double col[16];  // column c of L_kk
+#pragma unroll
+                for (int j = 0; j < 16; ++j) col[j] = sh.diag[k][j * 17 + c];
+                const double ri = sh.rinv[16 * k + c];
+                double v = sh.y[16 * k + c];
+#pragma unroll
+                for (int j = 15; j >= 0; --j) {
+                    const double xj = lane_value(v * ri, j);
+                    if (c == j) v = xj;
+                    else if (c < j) v = fma(-col[j], xj, v);
+                }
+                if (lane < 16) sh.y[16 * k + c] = v;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < kSmallTiles; ++t) {
+                int i, j;
+                tile_at(t, &i, &j);
+                if (i != k || j >= k) continue;
+                double v = 0.0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v = fma(acc[t][q], sh.y[16 * k + 4 * q + g], v);
+                v += __shfl_xor(v, 16, 64);
+                v += __shfl_xor(v, 32, 64);
+                if (g == 0) sh.y[16 * j + c] -= v;
+            }
+            __syncthreads();
+        }
+        for (int i = tid; i < n; i += NT) io.put(i, sh.y[i]);
+        if (tid == 0) *status = 0;
+        return;
+    }
+    double* y = work + (size_t)n * n;
+    if (allow_lu) {
+        for (int i = tid; i < n; i += NT) y[i] = io.rhs(i);
+        __syncthreads();
+        lu_fallback_body<NT>(S, y, n, &sh.fail, sh.piv_val, sh.piv_idx);
+    } else if (tid == 0) {
+        sh.fail = 2;
+    }
+    __syncthreads();
+    const int f = sh.fail;
+    for (int i = tid; i < n; i += NT) io.put(i, f != 2 ? y[i] : 0.0);
+    if (tid == 0) *status = f == 2 ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1002,25 +1211,18 @@ __global__ __launch_bounds__(kSmallBlock) void k_dense_finish(DenseRows io, doub
     if (threadIdx.x == 0) flags[0] = (f == 2) ? 1 : 0;
 }
 
-__global__ __launch_bounds__(kSmallBlock) void k_dense_solve(DevProblem P, DensePairs D, double* S, double* work,
-                                                             int n, int* status, int allow_lu) {
-    __shared__ int fail;
-    __shared__ double piv_val[kSmallBlock];
-    __shared__ int piv_idx[kSmallBlock];
-    __shared__ double dblk[16 * 17];
-    dense_solve_body<kSmallBlock>(pose_rows(P, D.var_slot, n), S, work, n, status, &fail, piv_val, piv_idx, dblk,
-                                  true, allow_lu != 0);
+__global__ __launch_bounds__(64 * kSmallWaves) void k_dense_solve(DevProblem P, DensePairs D, double* S, double* work,
+                                                                  int n, int* status, int allow_lu) {
+    __shared__ SmallSolveLds sh;
+    dense_solve_small(pose_rows(P, D.var_slot, n), S, work, n, status, allow_lu, sh);
 }
 
 // S x = b for a caller's row-major S (overwritten); work holds n * n + n.
-__global__ __launch_bounds__(kSmallBlock) void k_dense_solve_plain(double* S, double* work, const double* b,
-                                                                   double* x, int n, int* status) {
-    __shared__ int fail;
-    __shared__ double piv_val[kSmallBlock];
-    __shared__ int piv_idx[kSmallBlock];
-    __shared__ double dblk[16 * 17];
+__global__ __launch_bounds__(64 * kSmallWaves) void k_dense_solve_plain(double* S, double* work, const double* b,
+                                                                        double* x, int n, int* status) {
+    __shared__ SmallSolveLds sh;
     const DenseRows io{b, x, nullptr, n, nullptr, nullptr};
-    dense_solve_body<kSmallBlock>(io, S, work, n, status, &fail, piv_val, piv_idx, dblk, true);
+    dense_solve_small(io, S, work, n, status, 1, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -1048,22 +1250,30 @@ __global__ __launch_bounds__(kBlock) void k_batch_dense_zero(DevProblem P, Batch
     for (size_t k = blockIdx.x * (size_t)kBlock + threadIdx.x; k < n * n; k += (size_t)gridDim.x * kBlock) S[k] = 0.0;
 }
 
-__global__ __launch_bounds__(kBlock) void k_batch_dense_solve(DevProblem P, DensePairs D, BatchDev B) {
-    __shared__ int fail;
-    __shared__ double piv_val[kBlock];
-    __shared__ int piv_idx[kBlock];
+// One work-group per window. Windows of at most kDenseOneGroupMax unknowns as
+// a single solve of that size; kLarge takes the others (up to 256 poses), by
+// the factor in global memory with the LU fallback's copy saved first.
+template <bool kLarge>
+__global__ __launch_bounds__(64 * kSmallWaves) void k_batch_dense_solve(DevProblem P, DensePairs D, BatchDev B) {
+    __shared__ SmallSolveLds sh;
     const int w = blockIdx.x;
     WindowState& st = B.state[w];
     if (!st.active) return;
     const WindowLayout L = B.layout[w];
     const int n = 6 * (L.var_end - L.var_begin);
+    if ((n > kDenseOneGroupMax) != kLarge) return;
     if (n == 0) {
         if (threadIdx.x == 0) st.solve_status = 0;
         return;
     }
-    __shared__ double dblk[16 * 17];
-    dense_solve_body<kBlock>(pose_rows(P, D.var_slot + L.var_begin, n), B.S + L.s_offset, B.work + B.work_offset[w],
-                             n, &st.solve_status, &fail, piv_val, piv_idx, dblk);
+    const DenseRows io = pose_rows(P, D.var_slot + L.var_begin, n);
+    double* S = B.S + L.s_offset;
+    double* work = B.work + B.work_offset[w];
+    if constexpr (kLarge)
+        dense_solve_body<64 * kSmallWaves>(io, S, work, n, &st.solve_status, &sh.fail, sh.piv_val, sh.piv_idx,
+                                           sh.diag[0]);
+    else
+        dense_solve_small(io, S, work, n, &st.solve_status, 1, sh);
 }
 
 // Per window: compensated cost and non-projectable count over its camera
@@ -1622,6 +1832,11 @@ namespace {
 // The device-wide factor and the finishing solve (n > kDenseOneGroupMax).
 hipError_t dense_solve_device_wide(const DenseRows& io, double* S, double* work, int32_t n, int32_t* status,
                                    bool allow_lu, hipStream_t s) {
+    // the LU fallback's copy of S at full device bandwidth
+    if (allow_lu) {
+        const hipError_t e = hipMemcpyAsync(work, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, s);
+        if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL(k_dense_flags_clear, dim3(1), dim3(64), 0, s, status);
     for (int k0 = 0; k0 < n; k0 += kPanel) {
         const int below = n - k0 - kPanel;
@@ -1640,25 +1855,22 @@ hipError_t dense_solve_device_wide(const DenseRows& io, double* S, double* work,
 
 hipError_t launch_dense_solve(const DevProblem& P, const DensePairs& D, double* S, double* work, int32_t n,
                               int32_t* status, hipStream_t s, bool allow_lu) {
-    allow_lu = allow_lu && n <= kLuFallbackMax;
-    // the LU fallback's copy of S at full device bandwidth
-    if (allow_lu) {
-        const hipError_t e = hipMemcpyAsync(work, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, s);
-        if (e != hipSuccess) return e;
+    if (n <= kDenseOneGroupMax) {
+        hipLaunchKernelGGL(k_dense_solve, dim3(1), dim3(64 * kSmallWaves), 0, s, P, D, S, work, n, status,
+                           (int)allow_lu);
+        return hipGetLastError();
     }
-    if (n > kDenseOneGroupMax) return dense_solve_device_wide(pose_rows(P, D.var_slot, n), S, work, n, status, allow_lu, s);
-    hipLaunchKernelGGL(k_dense_solve, dim3(1), dim3(kSmallBlock), 0, s, P, D, S, work, n, status, (int)allow_lu);
-    return hipGetLastError();
+    return dense_solve_device_wide(pose_rows(P, D.var_slot, n), S, work, n, status, allow_lu && n <= kLuFallbackMax,
+                                   s);
 }
 hipError_t launch_dense_solve_plain(double* S, double* work, const double* b, double* x, int32_t n, int32_t* status,
                                     hipStream_t s) {
-    const hipError_t e = hipMemcpyAsync(work, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) return e;
-    if (n > kDenseOneGroupMax)
-        return dense_solve_device_wide(DenseRows{b, x, nullptr, n, nullptr, nullptr}, S, work, n, status,
-                                       n <= kLuFallbackMax, s);
-    hipLaunchKernelGGL(k_dense_solve_plain, dim3(1), dim3(kSmallBlock), 0, s, S, work, b, x, n, status);
-    return hipGetLastError();
+    if (n <= kDenseOneGroupMax) {
+        hipLaunchKernelGGL(k_dense_solve_plain, dim3(1), dim3(64 * kSmallWaves), 0, s, S, work, b, x, n, status);
+        return hipGetLastError();
+    }
+    return dense_solve_device_wide(DenseRows{b, x, nullptr, n, nullptr, nullptr}, S, work, n, status,
+                                   n <= kLuFallbackMax, s);
 }
 void launch_batch_dense_assemble(const DevProblem& P, const DensePairs& D, const BatchDev& B, hipStream_t s) {
     if (D.num_blocks)
@@ -1668,7 +1880,10 @@ void launch_batch_dense_zero(const DevProblem& P, const BatchDev& B, hipStream_t
     if (B.num_windows) hipLaunchKernelGGL(k_batch_dense_zero, dim3(16, B.num_windows), dim3(kBlock), 0, s, P, B);
 }
 void launch_batch_dense_solve(const DevProblem& P, const DensePairs& D, const BatchDev& B, hipStream_t s) {
-    if (B.num_windows) hipLaunchKernelGGL(k_batch_dense_solve, dim3(B.num_windows), dim3(kBlock), 0, s, P, D, B);
+    if (!B.num_windows) return;
+    hipLaunchKernelGGL(k_batch_dense_solve<false>, dim3(B.num_windows), dim3(64 * kSmallWaves), 0, s, P, D, B);
+    if (B.max_unknowns > kDenseOneGroupMax)
+        hipLaunchKernelGGL(k_batch_dense_solve<true>, dim3(B.num_windows), dim3(64 * kSmallWaves), 0, s, P, D, B);
 }
 void launch_batch_scalars(const DevProblem& P, const BatchDev& B, hipStream_t s) {
     if (B.num_windows) hipLaunchKernelGGL(k_batch_scalars, dim3(B.num_windows), dim3(kBlock), 0, s, P, B);

@@ -273,9 +273,10 @@ void launch_dense_assemble(const DevProblem& P, const DensePairs& D, double* S, 
 // Solve S x = b (Cholesky, then an LU fallback with allow_lu, else singular)
 // for the variable poses; writes x and sets status[0] (0 ok, 1 singular);
 // status holds two words (the second records a failed pivot). S is
-// overwritten; `work` (n * n + n) receives a copy of S for the LU fallback.
-// Systems of more than kDenseOneGroupMax unknowns are factored across the
-// device (two launches per 64 columns), smaller ones by one work-group.
+// overwritten; `work` holds n * n + n. Systems of more than kDenseOneGroupMax
+// unknowns are factored across the device (two launches per 64 columns, a
+// copy of S for the LU fallback in `work`), smaller ones by one work-group
+// that reads S and overwrites it only in the LU fallback.
 // Returns the error of the copy or of a launch.
 // The same solve for a plain system: S row-major n x n (overwritten), b and x
 // n long, always with the LU fallback.
@@ -296,6 +297,7 @@ struct BatchDev {
     WindowState* state;
     vba_iteration_stats* stats;  // num_windows x stats_capacity
     int32_t stats_capacity;
+    int32_t max_unknowns;  // of the largest window's dense system
     double* S;      // dense systems, WindowLayout::s_offset
     double* work;   // per window: n*n + n doubles at s_offset + s_offset/... (see solver)
     const int64_t* work_offset;

@@ -108,8 +108,8 @@ int32_t dense_solve_noalloc(Context& ctx, uint32_t n, const double* h, const dou
     };
     hipError_t e;
     // H arrives column-major in the work region; the transpose writes the
-    // row-major S, and the solve launcher then copies S back over the work
-    // region as the LU fallback's saved copy.
+    // row-major S, and the solve launcher then has the work region for the
+    // LU fallback.
     if ((e = hipMemcpyAsync(dwork, h, nn * sizeof(double), hipMemcpyHostToDevice, s)) != hipSuccess)
         return fail(e, "upload of H");
     if ((e = hipMemcpyAsync(db, b, n * sizeof(double), hipMemcpyHostToDevice, s)) != hipSuccess)

@@ -1385,6 +1385,8 @@ int32_t run_batch(Context& ctx, PreparedBatch& pb, const vba_options& o, vba_ite
         B.state = dstate;
         B.stats_capacity = (int32_t)std::max<uint32_t>(cap, 1);
         B.stats = (vba_iteration_stats*)ensure(pb, BB_STATS, (size_t)W * B.stats_capacity * sizeof(vba_iteration_stats));
+        B.max_unknowns = 0;
+        for (const WindowLayout& L : pb.layout) B.max_unknowns = std::max(B.max_unknowns, 6 * (L.var_end - L.var_begin));
         B.S = buf<double>(pb, BB_S);
         B.work = buf<double>(pb, BB_WORK);
         B.work_offset = buf<int64_t>(pb, BB_WORK_OFFSET);
