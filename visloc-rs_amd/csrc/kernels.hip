@@ -821,26 +821,29 @@ __device__ void dense_solve_body(const DenseRows& io, double* S, double* work, i
 // others A_r L_kk^-T, and lane j < 16 gets 1 / L_kk[j][j] in *rinv. False on
 // a pivot that is not positive and finite (the same in every lane).
 //
-// The chain pivot -> reciprocal root -> column -> next pivot bounds it: the
-// root is v_rsq_f64 with two Newton steps (each squares the relative error,
-// below 2^-52 after the second), and pivots and column entries come by lane
-// reads, which need no LDS and no barrier.
+// The chain pivot -> reciprocal root -> column -> next pivot bounds it, so it
+// is kept short: v_rsq_f64 and one third-order step (y(1 + e/2 + 3e^2/8) with
+// e = 1 - d y^2 leaves 5e^3/16 of the 2^-20 or better that the instruction
+// gives), pivots and column entries by lane reads (no LDS, no barrier), and
+// one test of all pivots at the end (a bad one only makes values that the
+// caller drops).
 __device__ __forceinline__ bool chol16_rows(double a[16], int lane, double* rinv) {
     double ri = 0.0;
+    bool bad = false;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const double d = lane_value(a[j], j);
-        if (!(d > 0.0) || !isfinite(d)) return false;
-        double y = __builtin_amdgcn_rsq(d);
-        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
-        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+        bad = bad || !(d > 0.0 && d < __builtin_inf());
+        const double y0 = __builtin_amdgcn_rsq(d);
+        const double e = fma(-(d * y0), y0, 1.0);
+        const double y = fma(y0 * e, fma(0.375, e, 0.5), y0);
         if (lane == j) ri = y;
         a[j] = a[j] * y;
 #pragma unroll
         for (int c = j + 1; c < 16; ++c) a[c] = fma(-a[j], lane_value(a[j], c), a[c]);
     }
     *rinv = ri;
-    return true;
+    return !bad;
 }
 
 // Dense solves of at most kDenseOneGroupMax unknowns by one work-group of
@@ -908,13 +911,24 @@ __device__ void dense_solve_small(const DenseRows& io, double* S, double* work, 
             }
             const int row = col + id - first;
             tile[t] = __builtin_amdgcn_readfirstlane(col < nb ? row << 8 | col : nb);
-            if (col < nb) {
+            if (col < nb)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[t][q] = padded_at(S, n, 16 * row + 4 * q + g, 16 * col + c);
-                if (col == 0)
+                for (int q = 0; q < 4; ++q)
+                    acc[t][q] = S[(size_t)min(16 * row + 4 * q + g, n - 1) * n + min(16 * col + c, n - 1)];
+        }
+    }
+    // every tile's loads are in flight (clamped above); now the identity past
+    // the end, and column 0 into the panel
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) sh.panel[0][(16 * row + 4 * q + g) * 17 + c] = acc[t][q];
-            }
+    for (int t = 0; t < kSmallTiles; ++t) {
+        int i, j;
+        tile_at(t, &i, &j);
+        if (j >= nb) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * i + 4 * q + g, cc = 16 * j + c;
+            if (r >= n || cc >= n) acc[t][q] = r == cc ? 1.0 : 0.0;
+            if (j == 0) sh.panel[0][r * 17 + c] = acc[t][q];
         }
     }
     __syncthreads();
@@ -1033,177 +1047,386 @@ __device__ void dense_solve_small(const DenseRows& io, double* S, double* work, 
 
 // ---------------------------------------------------------------------------
 // The same solve across the whole device, for systems larger than one
-// work-group factors quickly: a right-looking Cholesky over 64-column
-// panels, two launches per panel. k_chol_panel: every work-group factors the
-// 64 x 64 diagonal block in LDS (the same arithmetic in each, so every one
-// sees the same pivots) and solves its 256 rows of the panel below,
-// L_R = A_R L_kk^-T; work-group 0 writes the diagonal block back.
-// k_chol_update: the trailing lower triangle A_ij -= L_i L_j^T in 16 x 16
-// tiles, one wave each, on FP64 MFMA. flags[1] records a failed pivot (set
-// by work-group 0; later launches exit at once); k_dense_finish then solves
-// with the factor, or runs the LU fallback on the saved copy, in one
-// work-group.
+// work-group holds: a right-looking Cholesky over 64-column panels, two
+// launches per panel, and a back substitution of one launch per panel.
+//
+// k_chol_step, one launch per panel. Its first work-groups own 64 panel rows
+// each: they take the previous panel's part from the 64 x 64 diagonal block
+// and from their rows, factor the block in LDS (the same arithmetic in each,
+// so every one sees the same pivots) with the rows of the identity below it,
+// which become L_kk^-T, and form X = A L_kk^-T on FP64 MFMA; the right-hand
+// side is carried along: y_k = L_kk^-1 b_k, b -= X y_k. The other work-groups
+// take the previous panel's part from the 64 x 64 tiles of the columns
+// further right, A_ij -= X_i X_j^T. k_chol_back: x_k = L_kk^-T y_k and
+// y_j -= X_kj^T x_k for every earlier column. Nothing that a launch's
+// work-groups read is written by another of them: the diagonal block's lower
+// triangle stays as it is, L_kk^-T goes to its strict upper triangle with the
+// diagonal in `rdiag`, y_k to `y`. flags[1] records a failed pivot (later
+// launches exit at once); k_dense_finish then runs the LU fallback on the
+// saved copy in one work-group.
+//
+// A panel step is a chain of latencies (loads, 64 pivots, three MFMA products
+// that use a few CUs), so its pieces are kept short and the update is off the
+// chain. Before: one wave holding a whole row per lane (64 square roots and
+// divisions in a row, then the inverse: 65-73 us a panel), one 16 x 16 update
+// tile a wave in its own launch (17.3 us at 2,394 unknowns), and both
+// substitutions in one work-group (2.9 ms): 6.4 ms a solve of 2,394 unknowns,
+// 1.2 ms here (26 us a panel step, 4.7 us a back substitution step). Of a
+// step's 22 us at 294 unknowns the loads take 2, the previous panel's part 5,
+// the four 16-column factors 7 and what follows each 3, and X 4.
 // ---------------------------------------------------------------------------
 constexpr int kPanel = 64;
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // rows of an odd n are 8-byte aligned
 
-
-__global__ void k_dense_flags_clear(int* flags) {
-    if (threadIdx.x < 2) flags[threadIdx.x] = 0;
+// b = the right-hand side, flags = 0.
+__global__ __launch_bounds__(256) void k_dense_start(DenseRows io, double* b, int n, int* flags) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 2) flags[i] = 0;
+    if (i < n) b[i] = io.rhs(i);
 }
 
-__global__ __launch_bounds__(256) void k_chol_panel(double* S, int n, int k0, int* flags) {
-    if (__hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-    __shared__ double L[kPanel][kPanel + 1];
-    const int w = min(kPanel, n - k0);
-    for (int t = threadIdx.x; t < kPanel * kPanel; t += 256) {
-        const int r = t / kPanel, c = t % kPanel;
-        L[r][c] = (r < w && c < w) ? S[(size_t)(k0 + r) * n + k0 + c] : (r == c ? 1.0 : 0.0);
-    }
-    __syncthreads();
-    // the diagonal block's factor by wave 0, lane i holding row i in registers:
-    // column j's pivot and entries come from lane j and lane c by lane reads.
-    // Then lane c forms column c of L^-1 the same way, into LDS (Li).
-    __shared__ int failed;
-    __shared__ double Li[kPanel][kPanel + 1];
-    if (threadIdx.x < kPanel) {
-        const int i = threadIdx.x;
-        double a[kPanel];
+// Sum over the 16 lanes of a row, in every one of them.
+__device__ __forceinline__ double row16_sum(double v) {
+    v = v + dpp_partner<0xB1>(v);   // quad_perm [1,0,3,2]
+    v = v + dpp_partner<0x4E>(v);   // quad_perm [2,3,0,1]
+    v = v + dpp_partner<0x141>(v);  // row_half_mirror
+    return v + dpp_partner<0x140>(v);  // row_mirror
+}
+
+// Sixteen columns of a 64-column operand row per step m: this lane's four are
+// 16 m + 4 g + (0..3), 32 consecutive bytes. MFMA number e of the step takes
+// element e from both operands, so its four k values are 16 m + 4 g + e.
+__device__ __forceinline__ void load_row4(const double* row, int m, int g, double v[4]) {
+    const d2u* p = (const d2u*)(row + 16 * m + 4 * g);
+    const d2u a = p[0], b = p[1];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+
+// The previous panel's part of a 64 x 64 tile (rows bi.., columns bj..; its
+// columns are kp..kp+63), a 32 x 32 quarter per wave (the quarter above the
+// diagonal of a diagonal tile has nothing to do). Rows and columns past the
+// end read the last row and are not written.
+__device__ __forceinline__ void chol_update_tile(double* S, int n, int kp, int bi, int bj, int wave, int c, int g) {
+    if (bi == bj && wave == 1) return;
+    bi += 32 * (wave >> 1);
+    bj += 32 * (wave & 1);
+    if (bi >= n || bj >= n) return;
+    double av[2][4][4], bv[2][4][4];
+    v4d acc[2][2];
 #pragma unroll
-        for (int c = 0; c < kPanel; ++c) a[c] = L[i][c];
-        int bad = 0;
+    for (int u = 0; u < 2; ++u) {
+        const double* ra = S + (size_t)min(bi + 16 * u + c, n - 1) * n + kp;
+        const double* rb = S + (size_t)min(bj + 16 * u + c, n - 1) * n + kp;
 #pragma unroll
-        for (int j = 0; j < kPanel; ++j) {
-            const double d = lane_value(a[j], j);
-            if (!(d > 0.0) || !isfinite(d)) {  // the same in every lane and work-group
-                bad = 1;
-                break;
-            }
-            const double ljj = sqrt(d);
-            if (i == j) a[j] = ljj;
-            else if (i > j) a[j] = a[j] / ljj;
-            const double lij = a[j];
-#pragma unroll
-            for (int c = j + 1; c < kPanel; ++c) {
-                const double lcj = lane_value(a[j], c);
-                if (c <= i) a[c] -= lij * lcj;
-            }
-        }
-        if (i == 0) failed = bad;
-        if (!bad) {
-            if (blockIdx.x == 0 && i < w)
-#pragma unroll
-                for (int c = 0; c < kPanel; ++c)
-                    if (c <= i) S[(size_t)(k0 + i) * n + k0 + c] = a[c];
-            if (k0 + kPanel < n) {
-                // column c = i of L^-1: y_r = (e_c - sum_{k<r} L[r][k] y_k) / L[r][r]
-                const int c = i;
-                double yv[kPanel];
-#pragma unroll
-                for (int r = 0; r < kPanel; ++r) {
-                    double t0 = 0.0, t1 = 0.0;
-#pragma unroll
-                    for (int k = 0; k < r; ++k) {
-                        const double lrk = lane_value(a[k], r);
-                        if (k & 1) t1 += lrk * yv[k];
-                        else t0 += lrk * yv[k];
-                    }
-                    const double lrr = lane_value(a[r], r);
-                    yv[r] = r < c ? 0.0 : ((r == c ? 1.0 : 0.0) - (t0 + t1)) / lrr;
-                }
-#pragma unroll
-                for (int r = 0; r < kPanel; ++r) Li[r][c] = yv[r];
-            }
+        for (int m = 0; m < 4; ++m) {
+            load_row4(ra, m, g, av[u][m]);
+            load_row4(rb, m, g, bv[u][m]);
         }
     }
-    __syncthreads();
-    if (failed) {
-        if (blockIdx.x == 0 && threadIdx.x == 0)
-            __hip_atomic_store(&flags[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                acc[u][v][q] = S[(size_t)min(bi + 16 * u + 4 * q + g, n - 1) * n + min(bj + 16 * v + c, n - 1)];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int v = 0; v < 2; ++v)
+                    acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(-av[u][m][e], bv[v][m][e], acc[u][v], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = bi + 16 * u + 4 * q + g, cc = bj + 16 * v + c;
+                if (r < n && cc < n) S[(size_t)r * n + cc] = acc[u][v][q];
+            }
+}
+
+// Panel k0: work-groups 0 .. panel_groups - 1 are its rows, the others the
+// tiles of the columns from k0 + 64 on. LDS allows two work-groups a CU.
+__global__ __launch_bounds__(256) void k_chol_step(double* S, int n, int k0, int panel_groups, double* b, double* y,
+                                                   double* rdiag, int* flags) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int kp = k0 - kPanel;  // the previous panel's columns
+    if ((int)blockIdx.x >= panel_groups) {
+        if (__hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+        const int bb = (int)blockIdx.x - panel_groups;
+        int i = (int)((sqrtf(8.0f * (float)bb + 1.0f) - 1.0f) * 0.5f);
+        while ((i + 1) * (i + 2) / 2 <= bb) ++i;
+        while (i * (i + 1) / 2 > bb) --i;
+        const int j = bb - i * (i + 1) / 2;
+        chol_update_tile(S, n, kp, k0 + kPanel + 64 * i, k0 + kPanel + 64 * j, wave, c, g);
         return;
     }
-    if (k0 + kPanel >= n) return;  // no panel rows below
-    // panel rows: X = A_R L_kk^-T on FP64 MFMA, 16 x 16 output tiles; each
-    // wave holds the B operands (L^-1 transposed) of all 4 column tiles and
-    // takes the rows of its 64-row slice of this work-group's 256 rows.
-    // Operand lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; result
-    // register q holds C[4q + l / 16][l % 16].
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    double bop[4][kPanel / 4];
+    // rows 0..63: the block, later this work-group's rows; 64..127: the
+    // previous panel's rows of the block, then the identity, then L^-T
+    __shared__ double M[2 * kPanel][kPanel + 1];
+    __shared__ double sb[kPanel], sy[kPanel];
+    const int w = min(kPanel, n - k0);
+    const int r0 = k0 + kPanel + (int)blockIdx.x * kPanel + 16 * wave;  // this wave's 16 panel rows
+    const bool rows = r0 < n;
+    // Every load is issued before any is used, with no branch around one
+    // (indices clamped to the last row and column, values past the end
+    // replaced after): rows 16 i + 4 wave.. of the block and of the previous
+    // panel, one element a lane, and this wave's panel rows.
+    const int stop = __hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double bk = b[min(k0 + lane, n - 1)];
+    double blk[16], prev[16];
+    const int kq = k0 > 0 ? kp : 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const size_t r = (size_t)min(k0 + 4 * i + wave, n - 1) * n;
+        blk[i] = S[r + min(k0 + lane, n - 1)];
+        prev[i] = S[r + kq + lane];
+    }
+    v4d arow[4];
+    double xr[4][4];
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-        for (int kk = 0; kk < kPanel / 4; ++kk) bop[ct][kk] = Li[16 * ct + (lane & 15)][4 * kk + (lane >> 4)];
-    const int rbase = k0 + kPanel + (int)blockIdx.x * 256 + 64 * wave;
+        for (int q = 0; q < 4; ++q)
+            arow[ct][q] = S[(size_t)min(r0 + 4 * q + g, n - 1) * n + min(k0 + 16 * ct + c, n - 1)];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int r0 = rbase + 16 * rt;
-        if (r0 >= n) break;
-        const int ra = r0 + (lane & 15);
-        double aop[kPanel / 4];
+    for (int m = 0; m < 4; ++m) load_row4(S + (size_t)min(r0 + c, n - 1) * n + kq, m, g, xr[m]);
+    if (stop) return;
 #pragma unroll
-        for (int kk = 0; kk < kPanel / 4; ++kk)
-            aop[kk] = ra < n ? S[(size_t)ra * n + k0 + 4 * kk + (lane >> 4)] : 0.0;
-        v4d acc[4];
+    for (int i = 0; i < 16; ++i) {
+        const int r = 4 * i + wave;
+        M[r][lane] = r < w && lane <= r ? blk[i] : (r == lane ? 1.0 : 0.0);
+        M[kPanel + r][lane] = k0 > 0 ? (r < w ? prev[i] : 0.0) : (r == lane ? 1.0 : 0.0);
+    }
+    if (tid < kPanel) sb[tid] = tid < w ? bk : 0.0;
+    __syncthreads();
+    if (k0 > 0) {
+        // row tile `wave` of the block (the columns past the diagonal are
+        // not read again) and this wave's panel rows, less X X_k^T: two
+        // independent MFMA chains over operands read ahead
+        double av[4][4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) av[m][e] = -M[kPanel + 16 * wave + c][16 * m + 4 * g + e];
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct) {
-            acc[ct] = v4d{0.0, 0.0, 0.0, 0.0};
+            double bv[4][4];
 #pragma unroll
-            for (int kk = 0; kk < kPanel / 4; ++kk)
-                acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[kk], bop[ct][kk], acc[ct], 0, 0, 0);
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bv[m][e] = M[kPanel + 16 * ct + c][16 * m + 4 * g + e];
+            v4d acc;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[q] = M[16 * wave + 4 * q + g][16 * ct + c];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[m][e], bv[m][e], acc, 0, 0, 0);
+                    arow[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(-xr[m][e], bv[m][e], arow[ct], 0, 0, 0);
+                }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) M[16 * wave + 4 * q + g][16 * ct + c] = acc[q];
         }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) M[kPanel + 4 * i + wave][lane] = 4 * i + wave == lane ? 1.0 : 0.0;
+        __syncthreads();
+    }
+#pragma unroll 1
+    for (int s = 0; s < 4; ++s) {
+        const int k1 = 16 * s;
+        // 16 diagonal rows in each of two waves, 48 rows of the block below
+        // them and of the identity's non-zero ones (64 in all) in the rest
+        double a[16];
+        int row = k1 + lane;
+        const int p = 48 * wave + lane - 16;
+        const bool mine = lane >= 16 && p < 64;
+        if (lane >= 16) row = !mine ? k1 : p < 48 - k1 ? k1 + 16 + p : kPanel + p - (48 - k1);
+        if (wave < 2)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) a[j] = M[row][k1 + j];
+        __syncthreads();
+        bool ok = true;
+        if (wave < 2) {
+            double ri;
+            ok = chol16_rows(a, lane, &ri);
+            if (mine || (wave == 0 && lane < 16))
+#pragma unroll
+                for (int j = 0; j < 16; ++j) M[row][k1 + j] = a[j];
+        }
+        if (__syncthreads_or(!ok)) {
+            if (blockIdx.x == 0 && tid == 0)
+                __hip_atomic_store(&flags[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+        // columns to the right: lower tiles of the block, and the identity's
+        // non-zero row tiles 0..s
+        const int m = 3 - s, na = m * (m + 1) / 2, nt = na + (s + 1) * m;
+        for (int t = wave; t < nt; t += 4) {
+            int ri, cj;  // first row in M, first column
+            if (t < na) {
+                const int i = t == 0 ? 0 : t < 3 ? 1 : 2;
+                ri = k1 + 16 + 16 * i;
+                cj = k1 + 16 + 16 * (t - i * (i + 1) / 2);
+            } else {
+                ri = kPanel + 16 * ((t - na) / m);
+                cj = k1 + 16 + 16 * ((t - na) % m);
+            }
+            v4d acc;
+            double av[4], bv[4];
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                av[kk] = -M[ri + c][k1 + 4 * kk + g];
+                bv[kk] = M[cj + c][k1 + 4 * kk + g];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[q] = M[ri + 4 * q + g][cj + c];
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[kk], bv[kk], acc, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) M[ri + 4 * q + g][cj + c] = acc[q];
+        }
+        __syncthreads();
+    }
+    // the block's rows are done with: this work-group's rows in operand
+    // order, and y_k = L^-1 b_k, row by row of (L^-T)^T
+    if (rows)
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int r = r0 + 4 * q + (lane >> 4);
-                if (r < n) S[(size_t)r * n + k0 + 16 * ct + (lane & 15)] = acc[ct][q];
-            }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_chol_update(double* S, int n, int k0, const int* flags) {
-    if (__hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-    const int k1 = k0 + kPanel;
-    const int m = (n - k1 + 15) >> 4;
-    const int lane = threadIdx.x & 63;
-    const long long bb = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (m <= 0 || bb >= (long long)m * (m + 1) / 2) return;
-    long long i = (long long)((sqrt(8.0 * (double)bb + 1.0) - 1.0) * 0.5);
-    while ((i + 1) * (i + 2) / 2 <= bb) ++i;
-    while (i * (i + 1) / 2 > bb) --i;
-    const int j = (int)(bb - i * (i + 1) / 2);
-    const int bi = k1 + 16 * (int)i, bj = k1 + 16 * j;
-    v4d acc;
+            for (int q = 0; q < 4; ++q) M[16 * wave + 4 * q + g][16 * ct + c] = arow[ct][q];
+    if (wave == 3) {
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = padded_at(S, n, bi + 4 * q + (lane >> 4), bj + (lane & 15));
+        for (int q = 0; q < kPanel; q += 4)
 #pragma unroll
-    for (int kk = 0; kk < kPanel / 4; ++kk) {
-        const double a = -padded_at(S, n, bi + (lane & 15), k0 + 4 * kk + (lane >> 4));
-        const double bv = padded_at(S, n, bj + (lane & 15), k0 + 4 * kk + (lane >> 4));
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv, acc, 0, 0, 0);
+            for (int u = 0; u < 4; ++u) v[u] = fma(M[kPanel + q + u][lane], sb[q + u], v[u]);
+        const double yl = (v[0] + v[1]) + (v[2] + v[3]);
+        sy[lane] = yl;
+        if (blockIdx.x == 0 && lane < w) {
+            y[k0 + lane] = yl;
+            rdiag[k0 + lane] = M[kPanel + lane][lane];
+        }
     }
+    if (blockIdx.x == 0) {
+        double lt[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) lt[i] = M[kPanel + 4 * i + wave][lane];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = 4 * i + wave;
+            if (lane > r && lane < w) S[(size_t)(k0 + r) * n + k0 + lane] = lt[i];
+        }
+    }
+    __syncthreads();
+    if (!rows) return;
+    v4d acc[4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) acc[ct] = v4d{0.0, 0.0, 0.0, 0.0};
+    double av[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) av[m][e] = M[16 * wave + c][16 * m + 4 * g + e];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        double bv[4][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int ct = m; ct < 4; ++ct) bv[e][ct] = M[kPanel + 16 * m + 4 * g + e][16 * ct + c];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int ct = m; ct < 4; ++ct)  // L^-1 is lower triangular
+                acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[m][e], bv[e][ct], acc[ct], 0, 0, 0);
+    }
+    double yc[4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) yc[ct] = sy[16 * ct + c];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int r = bi + 4 * q + (lane >> 4), c = bj + (lane & 15);
-        if (r < n && c < n) S[(size_t)r * n + c] = acc[q];
+        const int r = r0 + 4 * q + g;
+        double v = 0.0;
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) {
+            v = fma(acc[ct][q], yc[ct], v);
+            if (r < n) S[(size_t)r * n + k0 + 16 * ct + c] = acc[ct][q];
+        }
+        v = row16_sum(v);
+        if (c == 0 && r < n) b[r] -= v;
     }
 }
 
-// After the device-wide factor: forward / back substitution with it, or the
-// LU fallback on the saved copy in work, or singular without a fallback.
-// flags[0] = 1 when singular.
-__global__ __launch_bounds__(kSmallBlock) void k_dense_finish(DenseRows io, double* S, double* work, int n,
-                                                              int* flags, int allow_lu) {
+// Panel k0 of the back substitution: every work-group forms x_k from y_k for
+// itself (work-group 0 writes it) and takes the panel's part from y at its 64
+// earlier columns; four waves share the 64 rows.
+__global__ __launch_bounds__(256) void k_chol_back(DenseRows io, const double* S, int n, int k0, double* y,
+                                                   const double* rdiag, const int* flags) {
+    __shared__ double U[kPanel][kPanel + 1];  // L^-T above its diagonal
+    __shared__ double sy[kPanel], sx[kPanel], part[4][kPanel];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int w = min(kPanel, n - k0), j = (int)blockIdx.x * kPanel + lane;
+    const int r = tid >> 2, q0 = 16 * (tid & 3);  // row of L^-T, its 16 columns of this thread
+    // loads with no branch around them (clamped; what is past the end or not
+    // in the triangle is dropped after)
+    const int stop = __hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double yk = y[min(k0 + lane, n - 1)], rd = rdiag[min(k0 + r, n - 1)];
+    double u[16], l[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const double* row = S + (size_t)min(k0 + 16 * wave + q, n - 1) * n;
+        u[q] = row[min(k0 + lane, n - 1)];
+        l[q] = row[min(j, n - 1)];
+    }
+    if (stop) return;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) U[16 * wave + q][lane] = 16 * wave + q < lane && lane < w ? u[q] : 0.0;
+    if (tid < kPanel) sy[tid] = tid < w ? yk : 0.0;
+    __syncthreads();
+    double v = (tid & 3) == 0 && r < w ? rd * sy[r] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v = fma(U[r][q0 + q], sy[q0 + q], v);
+    v = v + dpp_partner<0xB1>(v);
+    v = v + dpp_partner<0x4E>(v);
+    if ((tid & 3) == 0) {
+        sx[r] = v;
+        if (blockIdx.x == 0 && r < w) io.put(k0 + r, v);
+    }
+    __syncthreads();
+    v = 0.0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v = fma(16 * wave + q < w ? l[q] : 0.0, sx[16 * wave + q], v);
+    part[wave][lane] = v;
+    __syncthreads();
+    if (wave == 0 && j < k0) y[j] -= ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+}
+
+// After the device-wide factor: nothing, or the LU fallback on the saved copy
+// in work, or singular without a fallback. flags[0] = 1 when singular.
+__global__ __launch_bounds__(kSmallBlock) void k_dense_finish(DenseRows io, double* work, double* y, int n, int* flags,
+                                                              int allow_lu) {
     __shared__ int fail;
     __shared__ double piv_val[kSmallBlock];
     __shared__ int piv_idx[kSmallBlock];
-    __shared__ double dblk[16 * 17];
-    double* y = work + (size_t)n * n;
-    for (int i = threadIdx.x; i < n; i += kSmallBlock) y[i] = io.rhs(i);
     if (threadIdx.x == 0) fail = __hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (!fail) chol_blocked_solve<kSmallBlock>(S, n, y, dblk);
-    else if (allow_lu) lu_fallback_body<kSmallBlock>(work, y, n, &fail, piv_val, piv_idx);
+    if (!fail) return;
+    for (int i = threadIdx.x; i < n; i += kSmallBlock) y[i] = io.rhs(i);
+    __syncthreads();
+    if (allow_lu) lu_fallback_body<kSmallBlock>(work, y, n, &fail, piv_val, piv_idx);
     else if (threadIdx.x == 0) fail = 2;
     __syncthreads();
     const int f = fail;
@@ -1217,7 +1440,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_dense_solve(DevProblem P, 
     dense_solve_small(pose_rows(P, D.var_slot, n), S, work, n, status, allow_lu, sh);
 }
 
-// S x = b for a caller's row-major S (overwritten); work holds n * n + n.
+// S x = b for a caller's row-major S (overwritten); work holds dense_work_size(n).
 __global__ __launch_bounds__(64 * kSmallWaves) void k_dense_solve_plain(double* S, double* work, const double* b,
                                                                         double* x, int n, int* status) {
     __shared__ SmallSolveLds sh;
@@ -1837,18 +2060,20 @@ hipError_t dense_solve_device_wide(const DenseRows& io, double* S, double* work,
         const hipError_t e = hipMemcpyAsync(work, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, s);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_dense_flags_clear, dim3(1), dim3(64), 0, s, status);
+    // work: the copy, then b, y and the reciprocal pivots (dense_work_size)
+    double* const b = work + (size_t)n * n;
+    double* const y = b + n;
+    double* const rdiag = y + n;
+    hipLaunchKernelGGL(k_dense_start, dim3(blocks_for(n, 256)), dim3(256), 0, s, io, b, n, status);
     for (int k0 = 0; k0 < n; k0 += kPanel) {
-        const int below = n - k0 - kPanel;
-        hipLaunchKernelGGL(k_chol_panel, dim3(below > 0 ? (below + 255) / 256 : 1), dim3(256), 0, s, S, n, k0,
-                           status);
-        if (below > 0) {
-            const long long m = (below + 15) / 16, tiles = m * (m + 1) / 2;
-            hipLaunchKernelGGL(k_chol_update, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, s, S, n, k0,
-                               (const int*)status);
-        }
+        const int below = n - k0 - kPanel, m = below > 0 ? blocks_for(below, kPanel) : 0, groups = std::max(m, 1);
+        hipLaunchKernelGGL(k_chol_step, dim3(groups + (k0 > 0 ? m * (m + 1) / 2 : 0)), dim3(256), 0, s, S, n, k0, groups,
+                           b, y, rdiag, status);
     }
-    hipLaunchKernelGGL(k_dense_finish, dim3(1), dim3(kSmallBlock), 0, s, io, S, work, n, status, (int)allow_lu);
+    for (int k0 = (n - 1) / kPanel * kPanel; k0 >= 0; k0 -= kPanel)
+        hipLaunchKernelGGL(k_chol_back, dim3(std::max(k0 / kPanel, 1)), dim3(256), 0, s, io, (const double*)S, n, k0,
+                           y, (const double*)rdiag, (const int*)status);
+    hipLaunchKernelGGL(k_dense_finish, dim3(1), dim3(kSmallBlock), 0, s, io, work, y, n, status, (int)allow_lu);
     return hipGetLastError();
 }
 }  // namespace

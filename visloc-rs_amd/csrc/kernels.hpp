@@ -273,7 +273,7 @@ void launch_dense_assemble(const DevProblem& P, const DensePairs& D, double* S, 
 // Solve S x = b (Cholesky, then an LU fallback with allow_lu, else singular)
 // for the variable poses; writes x and sets status[0] (0 ok, 1 singular);
 // status holds two words (the second records a failed pivot). S is
-// overwritten; `work` holds n * n + n. Systems of more than kDenseOneGroupMax
+// overwritten; `work` holds dense_work_size(n) doubles. Systems of more than kDenseOneGroupMax
 // unknowns are factored across the device (two launches per 64 columns, a
 // copy of S for the LU fallback in `work`), smaller ones by one work-group
 // that reads S and overwrites it only in the LU fallback.
@@ -281,6 +281,8 @@ void launch_dense_assemble(const DevProblem& P, const DensePairs& D, double* S, 
 // The same solve for a plain system: S row-major n x n (overwritten), b and x
 // n long, always with the LU fallback.
 constexpr int32_t kDenseOneGroupMax = 256;
+// Doubles of `work`: the copy, then three vectors.
+constexpr size_t dense_work_size(size_t n) { return n * n + 3 * n; }
 // The LU fallback runs in one work-group, reading and writing the trailing
 // matrix once per pivot (n^3 / 3 x 16 bytes through one CU); beyond this size
 // it would run for minutes, so a failed Cholesky is reported singular.

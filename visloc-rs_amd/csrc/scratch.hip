@@ -31,7 +31,7 @@ struct Regions {
 constexpr Regions regions(size_t n) {
     const size_t s = 0;
     const size_t work = round_up(s + n * n);
-    const size_t b = round_up(work + n * n + n);
+    const size_t b = round_up(work + dense_work_size(n));
     const size_t x = round_up(b + n);
     const size_t status = round_up(x + n);
     return Regions{s, work, b, x, status, status + 1};

@@ -487,7 +487,7 @@ int32_t dense_solve(Context& ctx, uint32_t n, const double* h, const double* b, 
         if (!ctx.host_status)
             hip_check(hipHostMalloc((void**)&ctx.host_status, sizeof(int32_t), hipHostMallocDefault), "hipHostMalloc");
         alloc(bS, nn * sizeof(double));
-        alloc(bwork, (nn + n) * sizeof(double));
+        alloc(bwork, dense_work_size(n) * sizeof(double));
         alloc(bb, n * sizeof(double));
         alloc(bx, n * sizeof(double));
         alloc(bst, 2 * sizeof(int32_t));
@@ -772,7 +772,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         }
         if (!matrix_free) {
             dS = (double*)ensure(pr, B_DENSE_S, (size_t)ndense * ndense * sizeof(double));
-            dwork = (double*)ensure(pr, B_DENSE_WORK, ((size_t)ndense * ndense + ndense) * sizeof(double));
+            dwork = (double*)ensure(pr, B_DENSE_WORK, dense_work_size(ndense) * sizeof(double));
             dstatus = (int32_t*)ensure(pr, B_DENSE_STATUS, 2 * sizeof(int32_t));
         }
         // Algorithmic bytes per launch of the profiled kernels: what the data
