@@ -294,13 +294,12 @@ __device__ __forceinline__ double schur_block_wave(const DevProblem& P, const De
                     acc[6 * i + j] += C[3 * i + j];
                     acc[6 * i + 3 + j] -= CK[3 * i + j];
                 }
-                // K C and -K (C K), row by row of K
-                acc[18 + j] = fma(x1, C[6 + j], fma(-x2, C[3 + j], acc[18 + j]));
-                acc[24 + j] = fma(x2, C[j], fma(-x0, C[6 + j], acc[24 + j]));
-                acc[30 + j] = fma(x0, C[3 + j], fma(-x1, C[j], acc[30 + j]));
-                acc[21 + j] = fma(-x1, CK[6 + j], fma(x2, CK[3 + j], acc[21 + j]));
-                acc[27 + j] = fma(-x2, CK[j], fma(x0, CK[6 + j], acc[27 + j]));
-                acc[33 + j] = fma(-x0, CK[3 + j], fma(x1, CK[j], acc[33 + j]));
+                acc[18 + j] += fma(x1, C[6 + j], -(x2 * C[3 + j]));
+                acc[24 + j] += fma(x2, C[j], -(x0 * C[6 + j]));
+                acc[30 + j] += fma(x0, C[3 + j], -(x1 * C[j]));
+                acc[21 + j] -= fma(x1, CK[6 + j], -(x2 * CK[3 + j]));
+                acc[27 + j] -= fma(x2, CK[j], -(x0 * CK[6 + j]));
+                acc[33 + j] -= fma(x0, CK[3 + j], -(x1 * CK[j]));
             }
             if (k >= end) break;
         }

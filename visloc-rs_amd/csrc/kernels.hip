@@ -822,11 +822,10 @@ __device__ void dense_solve_body(const DenseRows& io, double* S, double* work, i
 // a pivot that is not positive and finite (the same in every lane).
 //
 // The chain pivot -> reciprocal root -> column -> next pivot bounds it, so it
-// is kept short: v_rsq_f64 and one third-order step (y(1 + e/2 + 3e^2/8) with
-// e = 1 - d y^2 leaves 5e^3/16 of the 2^-20 or better that the instruction
-// gives), pivots and column entries by lane reads (no LDS, no barrier), and
-// one test of all pivots at the end (a bad one only makes values that the
-// caller drops).
+// is kept short: v_rsq_f64 and two Newton steps (each squares the relative
+// error, below 2^-52 after the second), pivots and column entries by lane
+// reads (no LDS, no barrier), and one test of all pivots at the end (a bad
+// one only makes values that the caller drops).
 __device__ __forceinline__ bool chol16_rows(double a[16], int lane, double* rinv) {
     double ri = 0.0;
     bool bad = false;
@@ -834,9 +833,9 @@ __device__ __forceinline__ bool chol16_rows(double a[16], int lane, double* rinv
     for (int j = 0; j < 16; ++j) {
         const double d = lane_value(a[j], j);
         bad = bad || !(d > 0.0 && d < __builtin_inf());
-        const double y0 = __builtin_amdgcn_rsq(d);
-        const double e = fma(-(d * y0), y0, 1.0);
-        const double y = fma(y0 * e, fma(0.375, e, 0.5), y0);
+        double y = __builtin_amdgcn_rsq(d);
+        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
         if (lane == j) ri = y;
         a[j] = a[j] * y;
 #pragma unroll
