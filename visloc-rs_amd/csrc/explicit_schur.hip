@@ -9,7 +9,8 @@
 //
 // Assembly: one wave per upper block sums the block's term list (one term per
 // landmark the two poses share, in landmark order) in a fixed order, then
-// writes S_pq and its transpose S_qp. Products: one wave per block row, 48 lanes as 6 rows x 8 column-block groups.
+// writes S_pq and its transpose S_qp. Products: four waves per block row, 48
+// lanes of each as 6 rows x 8 column-block groups.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -69,92 +70,168 @@ __global__ __launch_bounds__(kBlock) void k_explicit_precond(DevProblem P, Expli
     for (int i = 0; i < 36; ++i) out[i] = inv[i];
 }
 
-// (S v)_p for v = v1 + beta v2 (v2 may be null): lane 8i + g sums row i of
-// the row's blocks g, g + 8, ...; a butterfly over g leaves the row sum in
-// all 8 lanes of row i. Lanes 48..63 return 0.
-template <typename TS>
-__device__ __forceinline__ double row_product(const ExplicitDev& X, const TS* __restrict__ S, int p,
-                                              const double* __restrict__ v1, const double* __restrict__ v2,
-                                              double beta, int lane) {
-    const int i = lane >> 3, g = lane & 7;
-    double acc = 0.0;
-    if (lane < 48) {
-        // blocks g, g + 8, ... in that order, four at a time: their loads are
-        // issued together before the products
-        constexpr int KB = 4;
-        const int end = X.row_ptr[p + 1];
-        for (int t0 = X.row_ptr[p] + g; t0 < end; t0 += 8 * KB) {
-            int q[KB];
-#pragma unroll
-            for (int u = 0; u < KB; ++u) q[u] = t0 + 8 * u < end ? X.col[t0 + 8 * u] : 0;
-            TS s[KB][6];
-            double v[KB][6];
-#pragma unroll
-            for (int u = 0; u < KB; ++u) {
-                const int t = t0 + 8 * u < end ? t0 + 8 * u : t0;
-                load6(S + 36 * (size_t)t + 6 * i, s[u]);
-                load6(v1 + 6 * (size_t)q[u], v[u]);
-                if (v2) {
-                    double w[6];
-                    load6(v2 + 6 * (size_t)q[u], w);
-#pragma unroll
-                    for (int j = 0; j < 6; ++j) v[u][j] = v[u][j] + beta * w[j];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < KB; ++u)
-                if (t0 + 8 * u < end)
-#pragma unroll
-                    for (int j = 0; j < 6; ++j) acc += (double)s[u][j] * v[u][j];
-        }
-    }
-    acc += __shfl_xor(acc, 1, 64);
-    acc += __shfl_xor(acc, 2, 64);
-    acc += __shfl_xor(acc, 4, 64);
-    return acc;
+// A block row's product by kRowWaves waves, two rows a work-group. Lane 8i + g
+// of wave w takes row i of the blocks 8 w + g, 8 w + g + 32, ... of the row,
+// kRowBlocks of them at a time.
+//
+// The matrix is small (288 bytes a block; a loop's 60 blocks a row make 14 MB
+// for 800 poses) and stays in the L2s, so the product is bound by its chain of
+// dependent loads (row bounds, columns, vectors) and by the launch. A block a
+// lane and pass makes two passes of a row of 64 blocks, and the inputs of the
+// PCG scalars load with the first one. (Two blocks a lane: more registers and
+// the same time; eight waves a row: 8 to 20 % slower.) One wave a row, four
+// blocks at a time after the scalars, took 8.9 us at 210 poses (FP64 blocks)
+// and 11.1 us at 800 (FP32 blocks) by the trace; 5.6 and 8.7 us here.
+constexpr int kRowWaves = 4, kRowBlocks = 1;
+constexpr int kRowThreads = 64 * kRowWaves * kExplicitRows;
+
+// Work-groups' rows: neighbouring rows on one XCD, whose L2 then holds their
+// part of the matrix and of the vectors they share.
+__device__ __forceinline__ int row_groups(const DevProblem& P) {
+    return (P.num_pose_slots + kExplicitRows - 1) / kExplicitRows;
 }
 
-// d_new = z + beta d_old and q = S d_new for one pose per wave; d.q partials
-// per work-group. The work-groups first derive the iteration's scalars.
 template <typename TS>
-__global__ __launch_bounds__(kBlock) void k_pcg_explicit(DevProblem P, ExplicitDev X, const TS* __restrict__ S,
-                                                         const double* __restrict__ d_old, double* __restrict__ d_new,
-                                                         int k, int fresh) {
-    __shared__ double lds[(kBlock / 64) * 2];
-    double beta;
-    if (!pcg_prologue(P, k, fresh, &beta)) return;
-    const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    double v[2] = {0.0, 0.0};
-    if (p < P.num_pose_slots && P.pose_var[p] >= 0) {
-        const double y = row_product<TS>(X, S, p, P.z, fresh ? nullptr : d_old, beta, lane);
-        const int c = lane < 6 ? lane : 0;
-        const double qc = __shfl(y, 8 * c, 64);
-        const size_t kk = 6 * (size_t)p + c;
-        const double dc = fresh ? P.z[kk] : P.z[kk] + beta * d_old[kk];
-        if (lane < 6) {
-            d_new[kk] = dc;
-            P.q[kk] = qc;
-            v[0] = dc * qc;
-        }
-        v[0] = wave_sum(v[0]);
+struct RowLoads {
+    int q[kRowBlocks];
+    TS s[kRowBlocks][6];
+};
+// Blocks t, t + 32, ... of the row (clamped to its last block, whose product
+// the caller drops) and their columns.
+template <typename TS>
+__device__ __forceinline__ void load_row_blocks(const ExplicitDev& X, const TS* __restrict__ S, int t, int last, int i,
+                                                RowLoads<TS>* r) {
+#pragma unroll
+    for (int u = 0; u < kRowBlocks; ++u) {
+        const int tc = max(min(t + 8 * kRowWaves * u, last), 0);
+        r->q[u] = X.col[tc];
+        load6(S + 36 * (size_t)tc + 6 * i, r->s[u]);
     }
-    wave_values_to_partial(v, lds, P.bpart + 2 * (size_t)blockIdx.x);
+}
+
+// Sums over the 8 lanes of a group in every one of them.
+__device__ __forceinline__ double group8_sum(double v) {
+    v = v + dpp_partner<0xB1>(v);      // quad_perm [1,0,3,2]
+    v = v + dpp_partner<0x4E>(v);      // quad_perm [2,3,0,1]
+    return v + dpp_partner<0x141>(v);  // row_half_mirror
+}
+
+// (S v)_p for v = v1 + beta v2 (v2 may be null) over blocks t, t + 32, ...
+// from the loaded ones on; `beta` is called once the vectors' loads are out
+// and false ends the launch (the same in every wave). The row's sum of row
+// component c is valid in lanes c < 6 of the row's wave 0.
+template <typename TS, typename Beta>
+__device__ __forceinline__ bool row_product(const ExplicitDev& X, const TS* __restrict__ S, int begin, int end,
+                                            const double* __restrict__ v1, const double* __restrict__ v2, Beta beta,
+                                            int lane, int wave, double (*sum)[8], double* y) {
+    const int i = min(lane >> 3, 5), g = lane & 7, last = end - 1;
+    int base = begin + 8 * wave, t = base + g;
+    RowLoads<TS> r;
+    load_row_blocks(X, S, t, last, i, &r);
+    double acc = 0.0, bt = 0.0;
+    for (bool first = true;; first = false) {
+        double v[kRowBlocks][6], w[kRowBlocks][6];
+#pragma unroll
+        for (int u = 0; u < kRowBlocks; ++u) {
+            load6(v1 + 6 * (size_t)r.q[u], v[u]);
+            if (v2) load6(v2 + 6 * (size_t)r.q[u], w[u]);
+        }
+        if (first && !beta(&bt)) return false;
+#pragma unroll
+        for (int u = 0; u < kRowBlocks; ++u)
+            if (t + 8 * kRowWaves * u < end)
+#pragma unroll
+                for (int j = 0; j < 6; ++j)
+                    acc = fma((double)r.s[u][j], v2 ? fma(bt, w[u][j], v[u][j]) : v[u][j], acc);
+        base += 8 * kRowWaves * kRowBlocks;
+        t = base + g;
+        if (base >= end) break;  // no lane of the wave has a block left
+        load_row_blocks(X, S, t, last, i, &r);
+    }
+    acc = group8_sum(acc);
+    if (lane < 48 && g == 0) sum[wave][i] = acc;
+    __syncthreads();
+    *y = 0.0;
+    if (wave == 0 && lane < 6) *y = ((sum[0][lane] + sum[1][lane]) + sum[2][lane]) + sum[3][lane];
+    return true;
+}
+
+// Sums (over lanes 0..5 of each row's wave 0, then over the work-group's
+// rows) into the work-group's partial.
+__device__ __forceinline__ void rows_to_partial(double v0, double v1, bool head, int row, double (*lds)[2],
+                                                double* out) {
+    if (head) {
+        v0 = wave_sum(v0);
+        v1 = wave_sum(v1);
+        if ((threadIdx.x & 63) == 0) {
+            lds[row][0] = v0;
+            lds[row][1] = v1;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double a = lds[0][threadIdx.x];
+        for (int r = 1; r < kExplicitRows; ++r) a += lds[r][threadIdx.x];
+        out[threadIdx.x] = a;
+    }
+}
+
+// d_new = z + beta d_old and q = S d_new; d.q partials per work-group. The
+// work-groups first derive the iteration's scalars.
+template <typename TS>
+__global__ __launch_bounds__(kRowThreads) void k_pcg_explicit(DevProblem P, ExplicitDev X, const TS* __restrict__ S,
+                                                              const double* __restrict__ d_old,
+                                                              double* __restrict__ d_new, int k, int fresh) {
+    __shared__ double sum[kExplicitRows][kRowWaves][8], lds[kExplicitRows][2];
+    const PrologueIn pin = pcg_prologue_load(P, k);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int row = wv / kRowWaves, wave = wv % kRowWaves;
+    const int group = xcd_tile(blockIdx.x, row_groups(P)), p = group * kExplicitRows + row;
+    if (group >= row_groups(P)) return;
+    const int pc = min(p, P.num_pose_slots - 1);
+    const bool var = p < P.num_pose_slots && P.pose_var[pc] >= 0;
+    const size_t kk = 6 * (size_t)pc + (lane < 6 ? lane : 0);
+    const double zc = P.z[kk], dc0 = d_old[kk];
+    double beta = 0.0, y;
+    // (the first product of a solve or restart has d = z and d_old = 0, so
+    // the term that beta = 0 multiplies is finite)
+    if (!row_product<TS>(X, S, X.row_ptr[pc], X.row_ptr[pc + 1], P.z, d_old,
+                         [&](double* b) {
+                             const bool go = pcg_prologue_finish(P, k, fresh, pin, &beta);
+                             *b = beta;
+                             return go;
+                         },
+                         lane, wave, sum[row], &y))
+        return;
+    double dq = 0.0;
+    if (var && wave == 0 && lane < 6) {
+        const double dc = fma(beta, dc0, zc);
+        d_new[kk] = dc;
+        P.q[kk] = y;
+        dq = dc * y;
+    }
+    rows_to_partial(dq, 0.0, wave == 0, row, lds, P.bpart + 2 * (size_t)group);
 }
 
 // r_t = b - S64 x; with restart r = r_t, z = M^-1 r_t, d = 0. Partials
 // (r_t.r_t, r_t.z) per work-group, as the implicit operator's check.
-__global__ __launch_bounds__(kBlock) void k_explicit_true_pose(DevProblem P, ExplicitDev X, int restart) {
-    __shared__ double lds[(kBlock / 64) * 2];
-    const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+__global__ __launch_bounds__(kRowThreads) void k_explicit_true_pose(DevProblem P, ExplicitDev X, int restart) {
+    __shared__ double sum[kExplicitRows][kRowWaves][8], lds[kExplicitRows][2];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int row = wv / kRowWaves, wave = wv % kRowWaves;
+    const int group = xcd_tile(blockIdx.x, row_groups(P)), p = group * kExplicitRows + row;
+    if (group >= row_groups(P)) return;
+    const int pc = min(p, P.num_pose_slots - 1);
+    const bool var = p < P.num_pose_slots && P.pose_var[pc] >= 0;
+    const int c = lane < 6 ? lane : 0;
+    const size_t k = 6 * (size_t)pc + c;
+    const double bc = P.b[k];
+    double y;
+    (void)row_product<double>(X, X.S64, X.row_ptr[pc], X.row_ptr[pc + 1], P.x, nullptr, [](double*) { return true; },
+                              lane, wave, sum[row], &y);
     double v[2] = {0.0, 0.0};
-    if (p < P.num_pose_slots && P.pose_var[p] >= 0) {
-        const double y = row_product<double>(X, X.S64, p, P.x, nullptr, 0.0, lane);
-        const int c = lane < 6 ? lane : 0;
-        const double sx = __shfl(y, 8 * c, 64);
-        const size_t k = 6 * (size_t)p + c;
-        const double rt = P.b[k] - sx;
+    if (var && wave == 0) {
+        const double rt = bc - y;
         double zc = 0.0;
         if (restart) zc = pose_minv(P, p, c, 0, rt, lane < 6);
         if (lane < 6) {
@@ -166,10 +243,8 @@ __global__ __launch_bounds__(kBlock) void k_explicit_true_pose(DevProblem P, Exp
                 v[1] = rt * zc;
             }
         }
-        v[0] = wave_sum(v[0]);
-        v[1] = wave_sum(v[1]);
     }
-    wave_values_to_partial(v, lds, P.bpart + 2 * (size_t)blockIdx.x);
+    rows_to_partial(v[0], v[1], wave == 0, row, lds, P.bpart + 2 * (size_t)group);
 }
 
 }  // namespace
@@ -183,17 +258,17 @@ void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const Ex
 
 void launch_pcg_explicit(const DevProblem& P, const ExplicitDev& X, bool fp32, const double* d_old, double* d_new,
                          int32_t pcg_iter, int32_t fresh, hipStream_t s) {
-    const dim3 grid(blocks_for(P.num_pose_slots, kBlock / 64));
+    const dim3 grid(xcd_grid(blocks_for(P.num_pose_slots, kExplicitRows)));
     if (fp32)
-        hipLaunchKernelGGL(k_pcg_explicit<float>, grid, dim3(kBlock), 0, s, P, X, (const float*)X.S32, d_old, d_new,
+        hipLaunchKernelGGL(k_pcg_explicit<float>, grid, dim3(kRowThreads), 0, s, P, X, (const float*)X.S32, d_old, d_new,
                            (int)pcg_iter, (int)fresh);
     else
-        hipLaunchKernelGGL(k_pcg_explicit<double>, grid, dim3(kBlock), 0, s, P, X, (const double*)X.S64, d_old, d_new,
+        hipLaunchKernelGGL(k_pcg_explicit<double>, grid, dim3(kRowThreads), 0, s, P, X, (const double*)X.S64, d_old, d_new,
                            (int)pcg_iter, (int)fresh);
 }
 
 void launch_explicit_true_residual(const DevProblem& P, const ExplicitDev& X, int32_t restart, hipStream_t s) {
-    hipLaunchKernelGGL(k_explicit_true_pose, dim3(blocks_for(P.num_pose_slots, kBlock / 64)), dim3(kBlock), 0, s, P,
+    hipLaunchKernelGGL(k_explicit_true_pose, dim3(xcd_grid(blocks_for(P.num_pose_slots, kExplicitRows))), dim3(kRowThreads), 0, s, P,
                        X, (int)restart);
     launch_pcg_true_finish(P, restart, s);
 }

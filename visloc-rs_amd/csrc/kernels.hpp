@@ -244,6 +244,9 @@ struct ExplicitDev {
     double* S64;               // 36 per full position
     float* S32;                // FP32 copy for the mixed-precision matvec (null in FP64)
 };
+// Block rows a work-group of the explicit products takes: each leaves one
+// partial in bpart.
+constexpr int kExplicitRows = 2;
 // S64 (and S32) from the term lists, U and lambda, then the block-Jacobi
 // inverses of the diagonal blocks into Minv (implicit_schur.rs:241-287).
 void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, double lambda,

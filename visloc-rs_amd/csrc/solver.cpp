@@ -767,6 +767,8 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             X.diag_pos = buf<int32_t>(pr, B_X_DIAG_POS);
             X.S64 = (double*)ensure(pr, B_X_S64, 36 * (size_t)X.num_full * sizeof(double));
             X.S32 = mixed ? (float*)ensure(pr, B_X_S32, 36 * (size_t)X.num_full * sizeof(float)) : nullptr;
+            P.num_bpart = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);
+            P.bpart = (double*)ensure(pr, B_BPART, 2 * (size_t)std::max(P.num_bpart, 1) * sizeof(double));
             dbuf[1] = (double*)ensure(pr, B_VD2, 6 * NP * sizeof(double));
             hip_check(hipMemsetAsync(dbuf[1], 0, 6 * NP * sizeof(double), s), "memset");
         }
