@@ -515,8 +515,10 @@ int32_t vba_profile_query(vba_context* ctx, const char* kernel, uint64_t* launch
  * waiting and how many empty launches a solve costs:
  * - pcg_chunk: iterations enqueued per read of the device PCG state (>= 1;
  *   default 10);
- * - pcg_lookahead: chunks enqueued beyond the one whose state is awaited
- *   (0..2; default 0), so that the device does not idle while the host reads;
+ * - pcg_lookahead: chunks always enqueued beyond the one whose state is
+ *   awaited (0..2; default 0), so that the device does not idle while the
+ *   host reads; one more is enqueued where the residual's decrease so far
+ *   says that the solve goes on through it;
  * - pcg_predict: nonzero: a solve's first chunk runs to the iteration count
  *   of the previous PCG solve of the same prepared problem (default 0).
  * The schedule is per context and applies to the matrix-free and explicit

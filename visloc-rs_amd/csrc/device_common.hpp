@@ -96,6 +96,16 @@ __device__ __forceinline__ double block_max(double v, double* lds) {
     return v;
 }
 
+// One thread posts a value of its own: the number becomes visible to the host
+// after the value (a system-scope release).
+template <typename T>
+__device__ __forceinline__ void post_mail(const Post<T>& post, const T& value) {
+    if (!post.slot) return;
+    post.slot->value = value;
+    __threadfence_system();
+    __hip_atomic_store(&post.slot->seq, post.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Neumaier compensated pair (sum, compensation) and its exact-order merge.
 struct CSum {
     double s, c;

@@ -267,10 +267,11 @@ void launch_pcg_explicit(const DevProblem& P, const ExplicitDev& X, bool fp32, c
                            (int)pcg_iter, (int)fresh);
 }
 
-void launch_explicit_true_residual(const DevProblem& P, const ExplicitDev& X, int32_t restart, hipStream_t s) {
+void launch_explicit_true_residual(const DevProblem& P, const ExplicitDev& X, int32_t restart,
+                                   const Post<PcgState>& post, hipStream_t s) {
     hipLaunchKernelGGL(k_explicit_true_pose, dim3(xcd_grid(blocks_for(P.num_pose_slots, kExplicitRows))), dim3(kRowThreads), 0, s, P,
                        X, (int)restart);
-    launch_pcg_true_finish(P, restart, s);
+    launch_pcg_true_finish(P, restart, post, s);
 }
 
 }  // namespace vba

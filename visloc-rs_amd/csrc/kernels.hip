@@ -451,7 +451,8 @@ __global__ __launch_bounds__(kBlock) void k_cost(DevProblem P, int trial) {
     }
 }
 
-__global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, int num_pose_blocks) {
+__global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, int num_pose_blocks,
+                                                                 Post<StepScalars> post) {
     __shared__ double lds[(kSmallBlock / 64) * 4];
     // cost partials in tile order: thread t < parts merges a contiguous run
     // of per tiles, and thread 0 folds the parts in order. Up to
@@ -495,6 +496,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, 
         o->nonprojectable = (uint64_t)v[0];
         o->max_pose_step = m1;
         o->max_landmark_step = m2;
+        post_mail(post, StepScalars{a.s, a.c, m1, m2, (uint64_t)v[0], 0, 0});
     }
 }
 
@@ -2004,8 +2006,8 @@ void launch_cost(const DevProblem& P, bool trial, hipStream_t s) {
     else
         hipLaunchKernelGGL(k_cost<false>, dim3(xcd_grid(P.num_cam_tiles)), dim3(kBlock), 0, s, P, (int)trial);
 }
-void launch_scalars_finalize(const DevProblem& P, hipStream_t s) {
-    hipLaunchKernelGGL(k_scalars_finalize, dim3(1), dim3(kSmallBlock), 0, s, P, blocks_for(P.num_pose_slots, kBlock));
+void launch_scalars_finalize(const DevProblem& P, const Post<StepScalars>& post, hipStream_t s) {
+    hipLaunchKernelGGL(k_scalars_finalize, dim3(1), dim3(kSmallBlock), 0, s, P, blocks_for(P.num_pose_slots, kBlock), post);
 }
 template <int K>
 void joint_linearize_k(const DevProblem& P, hipStream_t s) {

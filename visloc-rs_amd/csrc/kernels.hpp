@@ -46,6 +46,21 @@ struct PcgState {
     double rho[2];
     int32_t iter, status, max_iter, stop;
 };
+
+// A result in pinned host memory: the kernel that has it writes the value,
+// then the number the host waits for, so a read costs no copy kernel, no
+// event and no wake-up of the waiting thread.
+template <typename T>
+struct alignas(64) Mail {
+    T value;
+    uint64_t seq;
+};
+// Where to post, and under which number; a null slot posts nothing.
+template <typename T>
+struct Post {
+    Mail<T>* slot = nullptr;
+    uint64_t seq = 0;
+};
 enum PcgStatus : int32_t {
     PCG_RUNNING = 0,
     PCG_CONVERGED = 1,   // recursive residual <= target
@@ -176,7 +191,7 @@ void launch_landmark_prepare(const DevProblem& P, double lambda, hipStream_t str
 void launch_pose_update(const DevProblem& P, hipStream_t stream);
 // Cost and non-projectable count of (poses, lms) or of the trial state.
 void launch_cost(const DevProblem& P, bool trial, hipStream_t stream);
-void launch_scalars_finalize(const DevProblem& P, hipStream_t stream);
+void launch_scalars_finalize(const DevProblem& P, const Post<StepScalars>& post, hipStream_t stream);
 
 // schur.hip: the Schur operator over landmark tiles and the PCG vector work.
 // Block-Jacobi inverse blocks of U + lambda I - W V^-1 W^T into Minv.
@@ -207,18 +222,19 @@ void launch_pcg_pose(const DevProblem& P, hipStream_t stream, const LaunchEvents
 // alpha, x += alpha d, r -= alpha q, z = M^-1 r and (r.z, r.r) partials.
 void launch_pcg_step(const DevProblem& P, int32_t pcg_iter, hipStream_t stream, const LaunchEvents& ev = {});
 // The scalars of iteration pcg_iter (status, residual norm) without its work.
-void launch_pcg_status(const DevProblem& P, int32_t pcg_iter, int32_t fresh, hipStream_t stream);
+void launch_pcg_status(const DevProblem& P, int32_t pcg_iter, int32_t fresh, const Post<PcgState>& post,
+                       hipStream_t stream);
 // True residual b - S x in FP64 (state: true_norm).
-void launch_pcg_true_residual(const DevProblem& P, hipStream_t stream);
+void launch_pcg_true_residual(const DevProblem& P, const Post<PcgState>& post, hipStream_t stream);
 // Continue the recursion from the residual of the last true-residual check:
 // r = b - S x, z = M^-1 r, d = 0 (FP64 refinement of the mixed solve).
-void launch_pcg_restart(const DevProblem& P, hipStream_t stream);
+void launch_pcg_restart(const DevProblem& P, const Post<PcgState>& post, hipStream_t stream);
 // delta_l = -V^-1 (g_l + sum_e W_e^T x_p), trial landmarks, step maxima.
 void launch_backsub(const DevProblem& P, hipStream_t stream);
 
 // r_t.r_t (and with restart r_t.z) from the pose kernels' partials into the
 // PCG state; with restart the recursion continues from r_t.
-void launch_pcg_true_finish(const DevProblem& P, int32_t restart, hipStream_t stream);
+void launch_pcg_true_finish(const DevProblem& P, int32_t restart, const Post<PcgState>& post, hipStream_t stream);
 
 // Dense reduced system (LinearSolver::Dense).
 struct DensePairs {
@@ -258,7 +274,8 @@ void launch_pcg_explicit(const DevProblem& P, const ExplicitDev& X, bool fp32, c
                          int32_t pcg_iter, int32_t fresh, hipStream_t stream);
 // True residual b - S64 x and its norm (launch_pcg_true_finish); with
 // restart also r = r_t, z = M^-1 r_t and d = 0 (d is P.d).
-void launch_explicit_true_residual(const DevProblem& P, const ExplicitDev& X, int32_t restart, hipStream_t stream);
+void launch_explicit_true_residual(const DevProblem& P, const ExplicitDev& X, int32_t restart,
+                                   const Post<PcgState>& post, hipStream_t stream);
 
 // Joint camera block (joint_k = 4, 6 or 8): the camera terms after
 // linearization; the border rows of S and the camera right-hand side once

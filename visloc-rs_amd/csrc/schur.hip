@@ -1027,6 +1027,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_pcg_init(DevProblem P, double r
         else s.status = PCG_RUNNING;
         s.stop = s.status != PCG_RUNNING;
         *P.pcg = s;
+        P.scalars->precond_failed = 0;  // for the next solve's block inverses
         P.cpart[0] = acc[0];
         P.cpart[1] = acc[1];
     }
@@ -1129,9 +1130,10 @@ __global__ __launch_bounds__(kBlock) void k_pcg_step(DevProblem P, int k) {
     wave_values_to_partial(v, lds, P.cpart + 2 * (size_t)blockIdx.x);
 }
 
-__global__ __launch_bounds__(64) void k_pcg_status(DevProblem P, int k, int fresh) {
+__global__ __launch_bounds__(64) void k_pcg_status(DevProblem P, int k, int fresh, Post<PcgState> post) {
     double beta;
     (void)pcg_prologue(P, k, fresh, &beta);
+    if (threadIdx.x == 0) post_mail(post, *P.pcg);
 }
 
 // True residual r_t = b - S x (part64 holds the tile pass run on x); with
@@ -1167,7 +1169,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_true_pose(DevProblem P, int rest
     wave_values_to_partial(v, lds, P.bpart + 2 * (size_t)blockIdx.x);
 }
 
-__global__ __launch_bounds__(kBlock) void k_pcg_true_finish(DevProblem P, int restart) {
+__global__ __launch_bounds__(kBlock) void k_pcg_true_finish(DevProblem P, int restart, Post<PcgState> post) {
     __shared__ double lds[(kBlock / 64) * 2];
     double v[2] = {0.0, 0.0};
     for (int i = threadIdx.x; i < P.num_bpart; i += kBlock) {
@@ -1192,6 +1194,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_true_finish(DevProblem P, int re
             st->status = status;
             st->stop = status != PCG_RUNNING;
         }
+        post_mail(post, *st);
     }
 }
 
@@ -1253,23 +1256,24 @@ void launch_pcg_step(const DevProblem& P, int32_t pcg_iter, hipStream_t s, const
                           dim3(kBlock), 0, s, ev.start, ev.stop, 0, P, pcg_iter);
 }
 
-void launch_pcg_status(const DevProblem& P, int32_t pcg_iter, int32_t fresh, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_status, dim3(1), dim3(64), 0, s, P, pcg_iter, fresh);
+void launch_pcg_status(const DevProblem& P, int32_t pcg_iter, int32_t fresh, const Post<PcgState>& post,
+                       hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_status, dim3(1), dim3(64), 0, s, P, pcg_iter, fresh, post);
 }
 
-void launch_pcg_true_residual(const DevProblem& P, hipStream_t s) {
+void launch_pcg_true_residual(const DevProblem& P, const Post<PcgState>& post, hipStream_t s) {
     launch_schur_apply(P, false, P.x, nullptr, -1, 0, s);
     hipLaunchKernelGGL(k_pcg_true_pose, dim3(gather_blocks(P)), dim3(kBlock), 0, s, P, 0);
-    hipLaunchKernelGGL(k_pcg_true_finish, dim3(1), dim3(kBlock), 0, s, P, 0);
+    launch_pcg_true_finish(P, 0, post, s);
 }
 
-void launch_pcg_true_finish(const DevProblem& P, int32_t restart, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_true_finish, dim3(1), dim3(kBlock), 0, s, P, (int)restart);
+void launch_pcg_true_finish(const DevProblem& P, int32_t restart, const Post<PcgState>& post, hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_true_finish, dim3(1), dim3(kBlock), 0, s, P, (int)restart, post);
 }
 
-void launch_pcg_restart(const DevProblem& P, hipStream_t s) {
+void launch_pcg_restart(const DevProblem& P, const Post<PcgState>& post, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_true_pose, dim3(gather_blocks(P)), dim3(kBlock), 0, s, P, 1);
-    hipLaunchKernelGGL(k_pcg_true_finish, dim3(1), dim3(kBlock), 0, s, P, 1);
+    launch_pcg_true_finish(P, 1, post, s);
 }
 
 void launch_backsub(const DevProblem& P, hipStream_t s) {

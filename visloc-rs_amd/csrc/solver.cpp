@@ -388,10 +388,6 @@ void release_context(Context& ctx) {
     if (ctx.host_status) (void)hipHostFree(ctx.host_status);
     if (ctx.host_pcg_ring) (void)hipHostFree(ctx.host_pcg_ring);
     ctx.host_pcg_ring = nullptr;
-    for (hipEvent_t& e : ctx.pcg_ev) {
-        if (e) (void)hipEventDestroy(e);
-        e = nullptr;
-    }
     ctx.host_scalars = nullptr;
     ctx.host_pcg = nullptr;
     ctx.host_status = nullptr;
@@ -405,22 +401,51 @@ void release_context(Context& ctx) {
     release_reduced(ctx);
 }
 
+namespace {
+
+// The context's pinned words, allocated once.
+void ensure_mail(Context& ctx) {
+    if (!ctx.host_status)
+        hip_check(hipHostMalloc((void**)&ctx.host_status, sizeof(int32_t), hipHostMallocDefault), "hipHostMalloc");
+    if (!ctx.host_scalars) {
+        hip_check(hipHostMalloc((void**)&ctx.host_scalars, sizeof(Mail<StepScalars>), hipHostMallocDefault),
+                  "hipHostMalloc");
+        ctx.host_scalars->seq = 0;
+    }
+    if (!ctx.host_pcg_ring) {
+        hip_check(hipHostMalloc((void**)&ctx.host_pcg_ring, Context::kPcgRing * sizeof(Mail<PcgState>),
+                                hipHostMallocDefault), "hipHostMalloc");
+        for (int i = 0; i < Context::kPcgRing; ++i) ctx.host_pcg_ring[i].seq = 0;
+    }
+}
+
+// Wait for a post. The word is looked at without a system call; the stream is
+// asked now and then, so that a failed launch or device ends the wait, and so
+// does a stream that has run out without posting.
+template <typename T>
+T await_mail(const Post<T>& post, hipStream_t s) {
+    for (uint32_t spins = 1;; ++spins) {
+        if (__atomic_load_n(&post.slot->seq, __ATOMIC_ACQUIRE) == post.seq) return post.slot->value;
+        if (spins % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(s);
+            if (e == hipErrorNotReady) continue;
+            hip_check(e, "hipStreamQuery");
+            if (__atomic_load_n(&post.slot->seq, __ATOMIC_ACQUIRE) == post.seq) return post.slot->value;
+            throw Fail{VBA_ERR_DEVICE, "the device finished without its result"};
+        }
+#if defined(__x86_64__)
+        __builtin_ia32_pause();
+#endif
+    }
+}
+
+}  // namespace
+
 int32_t prepare(Context& ctx, Prepared& pr, std::string* msg) {
     hipStream_t s = ctx.stream;
     const Model& m = pr.m;
     try {
-        if (!ctx.host_scalars) {
-            hip_check(hipHostMalloc((void**)&ctx.host_scalars, sizeof(StepScalars), hipHostMallocDefault), "hipHostMalloc");
-            hip_check(hipHostMalloc((void**)&ctx.host_pcg, sizeof(PcgState), hipHostMallocDefault), "hipHostMalloc");
-        }
-        if (!ctx.host_status)
-            hip_check(hipHostMalloc((void**)&ctx.host_status, sizeof(int32_t), hipHostMallocDefault), "hipHostMalloc");
-        if (!ctx.host_pcg_ring) {
-            hip_check(hipHostMalloc((void**)&ctx.host_pcg_ring, Context::kPcgRing * sizeof(PcgState),
-                                    hipHostMallocDefault), "hipHostMalloc");
-            for (hipEvent_t& e : ctx.pcg_ev)
-                hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-        }
+        ensure_mail(ctx);
         upload(pr, B_POSES0, m.poses, s);
         upload(pr, B_LMS0, m.lms, s);
         ensure(pr, B_POSES, m.poses.size() * sizeof(double));
@@ -810,19 +835,22 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
 
         hip_check(hipEventRecord(ctx.ev_start, s), "event");
 
-        auto read_scalars = [&]() {
-            launch_scalars_finalize(P, s);
+        // the device's results of a launch, as it posts them (while kernels
+        // are being timed, once the stream is idle and their events complete)
+        auto read = [&](const auto& post) {
             hip_check(hipGetLastError(), "kernel launch");
-            hip_check(hipMemcpyAsync(ctx.host_scalars, P.scalars, sizeof(StepScalars), hipMemcpyDeviceToHost, s), "D2H");
-            hip_check(hipStreamSynchronize(s), "sync");
-            harvest(ctx);
-            return *ctx.host_scalars;
+            if (ctx.profile_stride > 0) hip_check(hipStreamSynchronize(s), "sync");
+            return await_mail(post, s);
         };
-        auto read_pcg = [&]() {
-            hip_check(hipGetLastError(), "kernel launch");
-            hip_check(hipMemcpyAsync(ctx.host_pcg, P.pcg, sizeof(PcgState), hipMemcpyDeviceToHost, s), "D2H");
-            hip_check(hipStreamSynchronize(s), "sync");
-            return *ctx.host_pcg;
+        auto read_scalars = [&]() {
+            const Post<StepScalars> post{ctx.host_scalars, ++ctx.mail_seq};
+            launch_scalars_finalize(P, post, s);
+            const StepScalars sc = read(post);
+            if (ctx.profile_stride > 0) harvest(ctx);
+            return sc;
+        };
+        auto pcg_post = [&]() {
+            return Post<PcgState>{ctx.host_pcg_ring + ctx.pcg_ring_next++ % Context::kPcgRing, ++ctx.mail_seq};
         };
 
         // ---- initial cost (lm.rs:323-327) ----
@@ -859,7 +887,6 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                 need_lin = false;
                 ++linearizations;
             }
-            hip_check(hipMemsetAsync(P.scalars, 0, sizeof(StepScalars), s), "memset");
             launch_landmark_prepare(P, lambda, s);
             launch_rhs(P, s);
 
@@ -927,46 +954,55 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                 };
                 while (true) {
                     // Iterations k .. in chunks (the context's schedule): each
-                    // chunk ends with a status kernel and a copy of the PCG
-                    // state into a pinned ring slot; the host waits for one
-                    // chunk's slot while `lookahead` later chunks are already
-                    // queued. The device stops itself, so launches past the
-                    // stop do nothing and no schedule changes a result.
+                    // chunk ends with a status kernel that posts the PCG
+                    // state; the host waits for one chunk's post while
+                    // `lookahead` later chunks are already queued, and one
+                    // more where the solve is expected to go on through it
+                    // (without it the device idles 25-30 us a chunk while the
+                    // host reads and launches: 4 of 17 ms for 1,350 iterations
+                    // on 210 poses, 9 of 144 ms for 2,850 on 1,200). Expected:
+                    // by the residual's average decrease per iteration so far,
+                    // before the first read by the last solve's count. The
+                    // device stops itself, so launches past the stop do
+                    // nothing and no schedule changes a result.
                     {
                         struct Ticket {
                             int32_t end;
-                            int slot;
+                            Post<PcgState> post;
                             size_t pending_end;
                         };
                         Ticket inflight[Context::kPcgRing];
                         int n_inflight = 0;
                         const vba_tuning& T = ctx.tuning;
-                        const int32_t k0 = k, fresh0 = fresh;
+                        const int32_t k0 = k, fresh0 = fresh, chunk = (int32_t)T.pcg_chunk;
                         int32_t next = k0;
+                        double expected_end = k0 == 0 ? pr.last_pcg : 0;
                         auto enqueue = [&](int32_t end) {
                             for (int32_t kk = next; kk < end; ++kk) launch_iteration(kk, fresh0 && kk == k0);
-                            launch_pcg_status(P, end, fresh0 && end == k0, s);
-                            const int slot = (int)(ctx.pcg_ring_next++ % Context::kPcgRing);
-                            hip_check(hipMemcpyAsync(ctx.host_pcg_ring + slot, P.pcg, sizeof(PcgState),
-                                                     hipMemcpyDeviceToHost, s), "D2H");
-                            hip_check(hipEventRecord(ctx.pcg_ev[slot], s), "hipEventRecord");
-                            inflight[n_inflight++] = Ticket{end, slot, ctx.pending.size()};
+                            const Post<PcgState> post = pcg_post();
+                            launch_pcg_status(P, end, fresh0 && end == k0, post, s);
+                            inflight[n_inflight++] = Ticket{end, post, ctx.pending.size()};
                             next = end;
                         };
-                        int32_t first = k0 + (int32_t)T.pcg_chunk;
+                        // chunks queued beyond the first one in flight: T.pcg_lookahead,
+                        // and one the solve should run well beyond
+                        auto fill = [&]() {
+                            while (next < max_pcg && n_inflight < Context::kPcgRing &&
+                                   (n_inflight <= (int)T.pcg_lookahead ||
+                                    (n_inflight == (int)T.pcg_lookahead + 1 && expected_end >= next + 2.0 * chunk)))
+                                enqueue(std::min(next + chunk, max_pcg));
+                        };
+                        int32_t first = k0 + chunk;
                         if (T.pcg_predict && k0 == 0 && pr.last_pcg > first) first = pr.last_pcg;
                         enqueue(std::min(first, max_pcg));
-                        for (uint32_t a = 0; a < T.pcg_lookahead && next < max_pcg; ++a)
-                            enqueue(std::min(next + (int32_t)T.pcg_chunk, max_pcg));
+                        fill();
                         int32_t seen = k0;
                         while (true) {
                             if (n_inflight == 0) throw Fail{VBA_ERR_DEVICE, "PCG did not stop at its cap"};
                             const Ticket t = inflight[0];
                             for (int i = 1; i < n_inflight; ++i) inflight[i - 1] = inflight[i];
                             --n_inflight;
-                            hip_check(hipGetLastError(), "kernel launch");
-                            hip_check(hipEventSynchronize(ctx.pcg_ev[t.slot]), "hipEventSynchronize");
-                            ps = ctx.host_pcg_ring[t.slot];
+                            ps = read(t.post);
                             if (ps.stop) {
                                 // every later launch found the stop flag; their
                                 // profile records are dropped (the records still
@@ -979,7 +1015,9 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                             for (int i = 0; i < n_inflight; ++i) inflight[i].pending_end -= done;
                             if (ps.iter <= seen) throw Fail{VBA_ERR_DEVICE, "PCG made no progress"};
                             seen = ps.iter;
-                            if (next < max_pcg) enqueue(std::min(next + (int32_t)T.pcg_chunk, max_pcg));
+                            const double fall = std::log(ps.rhs_norm / ps.rnorm), left = std::log(ps.rnorm / ps.target);
+                            expected_end = fall > 0.0 ? ps.iter + left * ps.iter / fall : (double)max_pcg;
+                            fill();
                         }
                         k = ps.iter;
                         fresh = 0;
@@ -989,9 +1027,10 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                         break;
                     }
                     // true residual re-check (implicit_schur.rs:613-690, 750-761)
-                    if (xplicit) launch_explicit_true_residual(P, X, 0, s);
-                    else launch_pcg_true_residual(P, s);
-                    ps = read_pcg();
+                    const Post<PcgState> checked = pcg_post();
+                    if (xplicit) launch_explicit_true_residual(P, X, 0, checked, s);
+                    else launch_pcg_true_residual(P, checked, s);
+                    ps = read(checked);
                     if (std::isfinite(ps.true_norm) && ps.true_norm <= ps.target) break;
                     if (!std::isfinite(ps.true_norm)) {
                         solved = false;
@@ -999,15 +1038,16 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     }
                     if (mixed && ps.iter < ps.max_iter) {
                         // FP64 refinement: continue from the true residual
+                        const Post<PcgState> restarted = pcg_post();
                         if (xplicit) {
                             // the next iteration (ps.iter) starts fresh from d = 0
                             DevProblem Pr = P;
                             Pr.d = dbuf[ps.iter & 1];
-                            launch_explicit_true_residual(Pr, X, 1, s);
+                            launch_explicit_true_residual(Pr, X, 1, restarted, s);
                         } else {
-                            launch_pcg_restart(P, s);
+                            launch_pcg_restart(P, restarted, s);
                         }
-                        ps = read_pcg();
+                        ps = read(restarted);
                         if (ps.stop) {
                             solved = ps.status == PCG_MAXIT && accept_iterate;
                             break;
@@ -1362,12 +1402,6 @@ int32_t run_batch(Context& ctx, PreparedBatch& pb, const vba_options& o, vba_ite
     const int32_t W = (int32_t)pb.index.size();
     if (W == 0) return VBA_OK;
     try {
-        if (!ctx.host_scalars) {
-            hip_check(hipHostMalloc((void**)&ctx.host_scalars, sizeof(StepScalars), hipHostMallocDefault), "hipHostMalloc");
-            hip_check(hipHostMalloc((void**)&ctx.host_pcg, sizeof(PcgState), hipHostMallocDefault), "hipHostMalloc");
-        }
-        if (!ctx.host_status)
-            hip_check(hipHostMalloc((void**)&ctx.host_status, sizeof(int32_t), hipHostMallocDefault), "hipHostMalloc");
         DevProblem P = bind(ctx, pb, o, false, false, s);
         P.any_rig = 1;
         P.obs_sensor = buf<uint16_t>(pb, B_OBS_SENSOR);

@@ -39,8 +39,8 @@ struct Context {
     std::mutex mu;
     std::string last_error;
     // pinned staging for the per-iteration scalars
-    StepScalars* host_scalars = nullptr;
-    PcgState* host_pcg = nullptr;
+    Mail<StepScalars>* host_scalars = nullptr;  // posted by k_scalars_finalize
+    PcgState* host_pcg = nullptr;               // pinned staging of the reduced-camera solve
     int32_t* host_status = nullptr;
     // profiling: events around every `profile_stride`-th launch of each
     // kernel family (0: off)
@@ -57,13 +57,13 @@ struct Context {
     std::vector<hipEvent_t> event_pool;
     // device buffers of the reduced-camera solve (reduced.hip), kept between calls
     ReducedState* reduced = nullptr;
-    // PCG launch schedule (vba_tuning) and the pinned ring its chunk reads
-    // land in, one event per slot
+    // PCG launch schedule (vba_tuning) and the pinned ring the device posts
+    // its PCG state to; mail_seq numbers every post of the context
     vba_tuning tuning{10, 0, 0, 0};
     static constexpr int kPcgRing = 4;
-    PcgState* host_pcg_ring = nullptr;
-    hipEvent_t pcg_ev[kPcgRing] = {};
+    Mail<PcgState>* host_pcg_ring = nullptr;
     uint32_t pcg_ring_next = 0;
+    uint64_t mail_seq = 0;
 };
 
 // One problem laid out on the device: structure, initial state and working
