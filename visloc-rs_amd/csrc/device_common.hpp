@@ -251,9 +251,10 @@ __device__ __forceinline__ int wave_entry36(int lane) {
 // lie near one another in storage, so the lanes of a gather share lines.
 // Eight lanes per block, each walking an eighth of the list, took 594 us for
 // the 50-camera circle's 6.4M terms against 103 us here, 821 us for 64 stereo
-// windows (longest list about 1,200 terms) against 158 us, and 635 us for a
-// 2.3M-observation loop's 17M terms against 576 us: that one reads 2.9 GB of
-// blocks through L1 and is bound there.
+// windows (longest list about 1,200 terms) against 158 us, and 840 us for
+// the 3.5M-observation loop's 27.5M terms, lists in first-met order, against
+// 492 us with the lists row by row: that one reads 4.6 GB of blocks through
+// L1 and is bound there.
 __device__ __forceinline__ double schur_block_wave(const DevProblem& P, const DensePairs& D, int b, int lane) {
     double acc[36];
 #pragma unroll

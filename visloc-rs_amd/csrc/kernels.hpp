@@ -263,6 +263,37 @@ struct ExplicitDev {
 // Block rows a work-group of the explicit products takes: each leaves one
 // partial in bpart.
 constexpr int kExplicitRows = 2;
+// Building the explicit matrix's structure on the device from the problem's
+// edges: lpose is the pose of each l-order edge, bits the row bitmaps (nw
+// words a row) of the variable poses a pose shares a landmark with, itself
+// among them.
+struct ExplicitBuild {
+    int32_t nw;
+    int32_t* lpose;
+    uint32_t* bits;
+    int32_t* row_count;  // per pose: full columns, upper columns (from the diagonal on), terms
+    int32_t* up_count;
+    int32_t* row_terms;
+    int32_t* row_ptr;    // exclusive sums of the above, num_pose_slots + 1 each
+    int32_t* up_ptr;
+    int32_t* term_row;
+    int32_t* col;        // outputs: ExplicitDev's and DensePairs' arrays
+    int32_t* diag_pos;
+    int32_t* block_pos;
+    int32_t* block_pq;
+    int32_t* block_ptr;
+    int32_t* terms;
+};
+// Columns a row of the device-built structure may have from its diagonal on
+// (a counter each in LDS) and poses it may have (a bitmap row each).
+constexpr int32_t kExplicitMaxUpper = 4096;
+constexpr int32_t kExplicitMaxPoses = 16384;
+// Rows: lpose, bits, row_count, up_count, then row_ptr and up_ptr. The host
+// reads their last entries to size the outputs, and up_count's maximum.
+void launch_explicit_rows(const DevProblem& P, const ExplicitBuild& B, hipStream_t stream);
+// Columns, block positions and the term lists, given row_ptr and up_ptr;
+// max_upper is the largest up_count.
+void launch_explicit_lists(const DevProblem& P, const ExplicitBuild& B, int32_t max_upper, hipStream_t stream);
 // S64 (and S32) from the term lists, U and lambda, then the block-Jacobi
 // inverses of the diagonal blocks into Minv (implicit_schur.rs:241-287).
 void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, double lambda,

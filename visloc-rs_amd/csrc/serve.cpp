@@ -132,6 +132,9 @@ uint64_t estimate_bytes(const vba_problem& p, bool window) {
     const uint64_t n = vba::observation_count(p);
     const uint64_t L = p.num_landmarks, P = p.num_poses;
     uint64_t b = n * 40 + n * 196 + L * 260 + P * 1400 + (64u << 10);
+    // the explicit reduced matrix a matrix-free solve may form: its lists and
+    // blocks within 144 bytes an edge, row bitmaps and row arrays
+    if (!window) b += n * 144 + P * (P / 8 + 64);
     if (window) {
         uint64_t var = 0;
         for (uint64_t i = 0; i < P; ++i) var += p.pose_fixed ? (p.pose_fixed[i] == 0) : 1;

@@ -32,7 +32,8 @@ enum BufId {
     B_SCALARS, B_DENSE_BLOCK_PQ, B_DENSE_BLOCK_PTR, B_DENSE_TERMS, B_DENSE_VAR_SLOT, B_DENSE_S,
     B_DENSE_WORK, B_DENSE_STATUS, B_X_BLOCK_POS, B_X_ROW_PTR, B_X_COL, B_X_DIAG_POS, B_X_S64, B_X_S32, B_VD2,
     B_G32_POS, B_OBS_W, B_OBS_S, B_OBS_KIND, B_OBS_EXTRA, B_SENSORS_T, B_J_E, B_J_TILE, B_J_HPK, B_J_KK, B_J_WK,
-    B_J_PART, B_J_RHS, B_J_DELTA, B_J_GL, B_T_LM, B_T_HEAD, B_T_RPOSE, B_T_RSLOT, B_COUNT
+    B_J_PART, B_J_RHS, B_J_DELTA, B_J_GL, B_T_LM, B_T_HEAD, B_T_RPOSE, B_T_RSLOT, B_X_PQ, B_X_PTR, B_X_TERMS,
+    B_X_SCRATCH, B_X_BITS, B_COUNT
 };
 
 // Profiled kernel families.
@@ -154,41 +155,122 @@ void build_dense(Prepared& pr) {
     pr.dense_built = true;
 }
 
-// Full block rows of the explicit reduced camera matrix over the term lists'
-// upper blocks: row p holds S_pq for every block (p, q) and S_qp^T for every
-// block (q, p), columns ascending.
-void build_explicit(Prepared& pr) {
+// Terms of the reduced camera matrix's blocks: every pair of a variable
+// landmark's edges once (fixed poses' pairs too, an upper bound).
+int64_t count_terms(Prepared& pr) {
+    if (pr.x_terms < 0) {
+        int64_t t = 0;
+        for (uint32_t l = 0; l < pr.m.num_lm_slots; ++l) {
+            const int64_t n = pr.m.lm_edge_ptr[l + 1] - pr.m.lm_edge_ptr[l];
+            if (pr.m.lm_var[l] >= 0) t += n * (n + 1) / 2;
+        }
+        pr.x_terms = t;
+    }
+    return pr.x_terms;
+}
+
+// The explicit matrix's structure from host lists, for problems the device
+// build does not take: full block rows over the term lists' upper blocks, row
+// p holding S_pq for every block (p, q) and S_qp^T for every block (q, p),
+// columns ascending.
+void build_explicit_host(Prepared& pr, hipStream_t s) {
     const Model& m = pr.m;
-    const size_t nb = pr.dense_block_pq.size() / 2, NP = m.num_pose_slots;
+    DenseLists d;
+    build_dense_lists(m, &d);
+    const size_t nb = d.block_pq.size() / 2, NP = m.num_pose_slots;
     std::vector<int32_t> count(NP + 1, 0);
     for (size_t b = 0; b < nb; ++b) {
-        const int32_t p = pr.dense_block_pq[2 * b], q = pr.dense_block_pq[2 * b + 1];
+        const int32_t p = d.block_pq[2 * b], q = d.block_pq[2 * b + 1];
         ++count[p + 1];
         if (p != q) ++count[q + 1];
     }
     for (size_t p = 0; p < NP; ++p) count[p + 1] += count[p];
-    pr.x_row_ptr = count;
     const size_t nfull = (size_t)count[NP];
     // (column, block * 2 + transposed) per full position, then each row by column
     std::vector<std::pair<int32_t, int32_t>> ent(nfull);
     std::vector<int32_t> cursor(count.begin(), count.end() - 1);
     for (size_t b = 0; b < nb; ++b) {
-        const int32_t p = pr.dense_block_pq[2 * b], q = pr.dense_block_pq[2 * b + 1];
+        const int32_t p = d.block_pq[2 * b], q = d.block_pq[2 * b + 1];
         ent[cursor[p]++] = {q, (int32_t)(2 * b)};
         if (p != q) ent[cursor[q]++] = {p, (int32_t)(2 * b + 1)};
     }
-    pr.x_col.assign(nfull, 0);
-    pr.x_block_pos.assign(2 * nb, -1);
-    pr.x_diag_pos.assign(NP, -1);
+    std::vector<int32_t> col(nfull, 0), block_pos(2 * nb, -1), diag_pos(NP, -1);
     for (size_t p = 0; p < NP; ++p) {
         std::sort(ent.begin() + count[p], ent.begin() + count[p + 1]);
         for (int32_t t = count[p]; t < count[p + 1]; ++t) {
-            pr.x_col[t] = ent[t].first;
-            pr.x_block_pos[ent[t].second] = t;
-            if (ent[t].first == (int32_t)p) pr.x_diag_pos[p] = t;
+            col[t] = ent[t].first;
+            block_pos[ent[t].second] = t;
+            if (ent[t].first == (int32_t)p) diag_pos[p] = t;
         }
     }
+    upload(pr, B_X_PQ, d.block_pq, s);
+    upload(pr, B_X_PTR, d.block_ptr, s);
+    upload(pr, B_X_TERMS, d.terms, s);
+    upload(pr, B_X_ROW_PTR, count, s);
+    upload(pr, B_X_COL, col, s);
+    upload(pr, B_X_BLOCK_POS, block_pos, s);
+    upload(pr, B_X_DIAG_POS, diag_pos, s);
+    hip_check(hipStreamSynchronize(s), "sync");  // the host vectors go out of scope
+    pr.x_num_blocks = (int32_t)nb;
+    pr.x_num_full = (int32_t)nfull;
+}
+
+// The explicit matrix's structure, on the device where its limits allow.
+// With max_full >= 0 (the matrix-free solver asking) a structure of more full
+// blocks, or one the device does not build, is not built: false.
+bool build_explicit(Prepared& pr, const DevProblem& P, int64_t max_full, hipStream_t s) {
+    if (pr.explicit_built) return max_full < 0 || pr.x_num_full <= max_full;
+    const size_t NP = (size_t)P.num_pose_slots, NE = (size_t)P.num_edges;
+    const int64_t terms = count_terms(pr);
+    if (terms > (int64_t)INT32_MAX / 3) {
+        if (max_full >= 0) return false;
+        throw Fail{VBA_ERR_INVALID_ARGUMENT, "Schur term lists too large"};
+    }
+    if (NP > (size_t)kExplicitMaxPoses || NE == 0) {
+        if (max_full >= 0) return false;
+        build_explicit_host(pr, s);
+        pr.explicit_built = true;
+        return true;
+    }
+    ExplicitBuild B{};
+    B.nw = (int32_t)((NP + 31) / 32);
+    B.bits = (uint32_t*)ensure(pr, B_X_BITS, (size_t)B.nw * NP * sizeof(uint32_t));
+    int32_t* w = (int32_t*)ensure(pr, B_X_SCRATCH, (NE + 5 * NP + 2) * sizeof(int32_t));
+    B.lpose = w;
+    B.row_count = w + NE;
+    B.up_count = B.row_count + NP;
+    B.row_terms = B.up_count + NP;
+    B.up_ptr = B.row_terms + NP;
+    B.term_row = B.up_ptr + NP + 1;
+    B.row_ptr = (int32_t*)ensure(pr, B_X_ROW_PTR, (NP + 1) * sizeof(int32_t));
+    launch_explicit_rows(P, B, s);
+    hip_check(hipGetLastError(), "kernel launch");
+    std::vector<int32_t> up(NP);
+    int32_t full = 0, blocks = 0;
+    hip_check(hipMemcpyAsync(up.data(), B.up_count, NP * sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
+    hip_check(hipMemcpyAsync(&full, B.row_ptr + NP, sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
+    hip_check(hipMemcpyAsync(&blocks, B.up_ptr + NP, sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
+    hip_check(hipStreamSynchronize(s), "sync");
+    const int32_t max_upper = *std::max_element(up.begin(), up.end());
+    if (max_full >= 0 && full > max_full) return false;
+    if (max_upper > kExplicitMaxUpper) {
+        if (max_full >= 0) return false;
+        build_explicit_host(pr, s);
+        pr.explicit_built = true;
+        return true;
+    }
+    B.col = (int32_t*)ensure(pr, B_X_COL, (size_t)full * sizeof(int32_t));
+    B.diag_pos = (int32_t*)ensure(pr, B_X_DIAG_POS, NP * sizeof(int32_t));
+    B.block_pos = (int32_t*)ensure(pr, B_X_BLOCK_POS, 2 * (size_t)blocks * sizeof(int32_t));
+    B.block_pq = (int32_t*)ensure(pr, B_X_PQ, 2 * (size_t)blocks * sizeof(int32_t));
+    B.block_ptr = (int32_t*)ensure(pr, B_X_PTR, ((size_t)blocks + 1) * sizeof(int32_t));
+    B.terms = (int32_t*)ensure(pr, B_X_TERMS, 3 * (size_t)terms * sizeof(int32_t));
+    launch_explicit_lists(P, B, max_upper, s);
+    hip_check(hipGetLastError(), "kernel launch");
+    pr.x_num_blocks = blocks;
+    pr.x_num_full = full;
     pr.explicit_built = true;
+    return true;
 }
 
 // ---- profiling with HIP events on the context stream ----
@@ -706,7 +788,9 @@ DevProblem bind(const Context& ctx, Prepared& pr, const vba_options& o, bool mix
         P.q = (double*)ensure(pr, B_VQ, 6 * NP * sizeof(double));
         P.num_bpart = (int32_t)((NP + (kBlock / 64) - 1) / (kBlock / 64));
         P.num_cpart = (int32_t)((NP + (kBlock / 64) * kPosesPerWave - 1) / ((kBlock / 64) * kPosesPerWave));
-        P.bpart = (double*)ensure(pr, B_BPART, 2 * (size_t)std::max(P.num_bpart, 1) * sizeof(double));
+        // (sized for the explicit product's work-groups too, which are more)
+        const size_t bparts = std::max<size_t>(P.num_bpart, (NP + kExplicitRows - 1) / kExplicitRows);
+        P.bpart = (double*)ensure(pr, B_BPART, 2 * std::max<size_t>(bparts, 1) * sizeof(double));
         P.cpart = (double*)ensure(pr, B_CPART, 2 * (size_t)std::max(P.num_cpart, 1) * sizeof(double));
         P.pcg = (PcgState*)ensure(pr, B_PCG, sizeof(PcgState));
     }
@@ -718,6 +802,40 @@ DevProblem bind(const Context& ctx, Prepared& pr, const vba_options& o, bool mix
     hip_check(hipMemsetAsync(P.delta_l, 0, 3 * NL * sizeof(double), s), "memset");
     hip_check(hipMemsetAsync(P.tile_scalar, 0, nscalar * sizeof(double), s), "memset");
     return P;
+}
+
+}  // namespace
+
+namespace {
+
+// Device memory the matrix-free solver may add for the explicit matrix, bytes
+// per edge: its term lists and its blocks (what the request loop's estimate
+// counts beside the layout).
+constexpr int64_t kExplicitTermBytes = 112, kExplicitBlockBytes = 32;
+
+// Whether the explicit reduced matrix is the faster operator for the rest of
+// a matrix-free solve, from the last PCG solve's iterations and the problem's
+// sizes alone (so that every solve of the problem decides alike).
+//
+// Measured on this card: a PCG iteration over the edges takes 13.6 us + 8.1 ps
+// an edge with FP32 G (16.4 us at 0.33M edges, 42 us at 3.5M), 15.6 us + 10.7
+// ps with FP64 G (25 us at 0.87M); one over the matrix, FP64 blocks in either
+// precision, 8.2 us + 0.06 ns a stored block (8.4 us at 163 poses and 9k
+// blocks, 9.8 us at 300 and 29k, 17.3 us at 1,200 and 140k). Against that
+// stand the assembly, 20 us + 17.5 ps a term for every LM iteration (55 us at
+// 2.3M terms, 492 us at 27.5M; the edges' block-Jacobi passes, which it
+// replaces, take 20 us + 30 ps an edge), and the structure, once: 1 ms + 75 ps
+// a term (3.1 ms at 27.5M). The lists' and blocks' memory has to stay within
+// the bounds above, which long tracks (more than some 9 terms an edge) and
+// scenes whose poses share landmarks with most others exceed.
+bool explicit_pays(Prepared& pr, bool mixed, int32_t its, uint32_t remaining, const int32_t* num_full) {
+    const double edges = (double)pr.m.num_edges, terms = (double)count_terms(pr);
+    if (12.0 * terms + 4.0 * edges > (double)kExplicitTermBytes * edges) return false;
+    const double over_edges = mixed ? 13.6e-6 + 8.1e-12 * edges : 15.6e-6 + 10.7e-12 * edges;
+    const double over_matrix = 8.2e-6 + (num_full ? 0.06e-9 * *num_full : 0.0);
+    const double assembly = (20e-6 + 17.5e-12 * terms) - (20e-6 + 30e-12 * edges);
+    const double build = 1e-3 + 75e-12 * terms;
+    return (its * (over_edges - over_matrix) - assembly) * remaining > build;
 }
 
 }  // namespace
@@ -760,7 +878,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             P.joint_gl = (double*)ensure(pr, B_J_GL, 3 * std::max<size_t>(NL, 1) * sizeof(double));
         }
         const int32_t ndense = (int32_t)(6 * m.P) + JK;
-        if (!matrix_free || xplicit) {
+        if (!matrix_free) {
             if (!pr.dense_built) {
                 build_dense(pr);
                 upload(pr, B_DENSE_BLOCK_PQ, pr.dense_block_pq, s);
@@ -774,29 +892,32 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             D.terms = buf<int32_t>(pr, B_DENSE_TERMS);
             D.var_slot = buf<int32_t>(pr, B_DENSE_VAR_SLOT);
         }
+        // The explicit matrix, when this solve uses it (xp): from the start
+        // for the explicit solver, later for the matrix-free one (below).
         ExplicitDev X{};
-        double* dbuf[2] = {P.d, nullptr};  // PCG direction by iteration parity (explicit)
-        if (xplicit) {
-            if (!pr.explicit_built) {
-                build_explicit(pr);
-                upload(pr, B_X_BLOCK_POS, pr.x_block_pos, s);
-                upload(pr, B_X_ROW_PTR, pr.x_row_ptr, s);
-                upload(pr, B_X_COL, pr.x_col, s);
-                upload(pr, B_X_DIAG_POS, pr.x_diag_pos, s);
-            }
-            X.num_blocks = D.num_blocks;
-            X.num_full = (int32_t)pr.x_col.size();
+        bool xp = false;
+        const bool x32 = xplicit && mixed;           // FP32 copy for its products
+        double* dbuf[2] = {P.d, nullptr};            // PCG direction by iteration parity
+        auto use_explicit = [&](int64_t max_full) {
+            if (!build_explicit(pr, P, max_full, s)) return false;
+            D.num_blocks = pr.x_num_blocks;
+            D.block_pq = buf<int32_t>(pr, B_X_PQ);
+            D.block_ptr = buf<int32_t>(pr, B_X_PTR);
+            D.terms = buf<int32_t>(pr, B_X_TERMS);
+            X.num_blocks = pr.x_num_blocks;
+            X.num_full = pr.x_num_full;
             X.block_pos = buf<int32_t>(pr, B_X_BLOCK_POS);
             X.row_ptr = buf<int32_t>(pr, B_X_ROW_PTR);
             X.col = buf<int32_t>(pr, B_X_COL);
             X.diag_pos = buf<int32_t>(pr, B_X_DIAG_POS);
             X.S64 = (double*)ensure(pr, B_X_S64, 36 * (size_t)X.num_full * sizeof(double));
-            X.S32 = mixed ? (float*)ensure(pr, B_X_S32, 36 * (size_t)X.num_full * sizeof(float)) : nullptr;
-            P.num_bpart = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);
-            P.bpart = (double*)ensure(pr, B_BPART, 2 * (size_t)std::max(P.num_bpart, 1) * sizeof(double));
+            X.S32 = x32 ? (float*)ensure(pr, B_X_S32, 36 * (size_t)X.num_full * sizeof(float)) : nullptr;
             dbuf[1] = (double*)ensure(pr, B_VD2, 6 * NP * sizeof(double));
             hip_check(hipMemsetAsync(dbuf[1], 0, 6 * NP * sizeof(double), s), "memset");
-        }
+            P.num_bpart = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);
+            return xp = true;
+        };
+        if (xplicit) use_explicit(-1);
         if (!matrix_free) {
             dS = (double*)ensure(pr, B_DENSE_S, (size_t)ndense * ndense * sizeof(double));
             dwork = (double*)ensure(pr, B_DENSE_WORK, dense_work_size(ndense) * sizeof(double));
@@ -821,10 +942,13 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         // landmark X and V^-1 once; per stored block 36 values (FP64, and the
         // FP32 copy); per pose U, the diagonal read and Minv. Product: per
         // stored block 36 reals and its column; per pose z, d_old, d_new, q.
-        const double nterms = xplicit ? (double)pr.dense_terms.size() / 3.0 : 0.0;
-        const double bytes_xassemble = nterms * 12.0 + NE * 48.0 + NL * 72.0 +
-                                       X.num_full * 36.0 * (8.0 + (mixed ? 4.0 : 0.0)) + NP * (168.0 + 288.0 + 288.0);
-        const double bytes_xapply = X.num_full * (36.0 * real + 4.0) + NP * (4.0 + 4.0 * 48.0);
+        auto bytes_xassemble = [&]() {
+            return (double)count_terms(pr) * 12.0 + NE * 48.0 + NL * 72.0 +
+                   X.num_full * 36.0 * (8.0 + (x32 ? 4.0 : 0.0)) + NP * (168.0 + 288.0 + 288.0);
+        };
+        auto bytes_xapply = [&]() {
+            return X.num_full * (36.0 * (x32 ? 4.0 : 8.0) + 4.0) + NP * (4.0 + 4.0 * 48.0);
+        };
         // dense assembly: per term its indices (12); per edge G, per landmark X
         // and V^-1, per pose U once; per block its pair and term pointer (12);
         // the whole n x n S written. Dense factor: n^3 / 3 FLOPs.
@@ -869,6 +993,8 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         double lambda = o.has_initial_lambda ? o.initial_lambda : 0.0;
         bool converged = false, need_lin = true;
         uint32_t written = 0, total_pcg = 0, linearizations = 0;
+        int32_t last_its = -1;  // PCG iterations of the last solve of this call
+        bool ask = matrix_free && !xplicit && !pr.x_refused;  // whether to use the explicit matrix
         const int32_t max_pcg = (int32_t)o.max_pcg_iterations;
         auto push = [&](const vba_iteration_stats& st) {
             if (stats && written < cap) stats[written] = st;
@@ -879,13 +1005,36 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             if (need_lin) {
                 {
                     ProfScope ps(ctx, K_LINEARIZE, bytes_linearize);
-                    launch_linearize(P, mixed, s);
+                    launch_linearize(P, P.Gl32 != nullptr, s);
                 }
                 launch_camera_finalize(P, s);
                 launch_landmark_reduce(P, s);
                 if (JK) launch_joint_linearize(P, s);
                 need_lin = false;
                 ++linearizations;
+            }
+            // The matrix-free solver forms the explicit matrix once the last
+            // PCG solve has shown that it pays (explicit_pays), and keeps it:
+            // its FP32 copies of G are then not needed any more.
+            if (ask && !xp && last_its > 0 &&
+                explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, nullptr)) {
+                bool done = false;
+                try {
+                    done = use_explicit((int64_t)(kExplicitBlockBytes * NE / 304)) &&
+                           explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, &pr.x_num_full);
+                } catch (const Fail& f) {
+                    if (f.code != VBA_ERR_OUT_OF_MEMORY) throw;
+                    (void)hipGetLastError();  // no memory for it: stay with the edges
+                }
+                xp = done;
+                if (done) {
+                    P.Gl32 = nullptr;
+                    P.Vm = P.VinvM = nullptr;
+                } else {
+                    P.num_bpart = (int32_t)((NP + (kBlock / 64) - 1) / (kBlock / 64));
+                    ask = false;
+                    pr.x_refused = true;
+                }
             }
             launch_landmark_prepare(P, lambda, s);
             launch_rhs(P, s);
@@ -912,8 +1061,8 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                 hip_check(hipStreamSynchronize(s), "sync");
                 solved = *ctx.host_status == 0;
             } else {
-                if (xplicit) {
-                    ProfScope a(ctx, K_EXPLICIT_ASSEMBLE, bytes_xassemble);
+                if (xp) {
+                    ProfScope a(ctx, K_EXPLICIT_ASSEMBLE, bytes_xassemble());
                     launch_explicit_assemble(P, D, X, lambda, s);
                 } else {
                     launch_precondition(P, lambda, s);
@@ -925,12 +1074,12 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                 // one PCG iteration's launches; fresh_kk: the first of a
                 // solve or restart (d starts from z)
                 auto launch_iteration = [&](int32_t kk, int32_t fresh_kk) {
-                    if (xplicit) {
+                    if (xp) {
                         // iteration kk reads d from dbuf[kk & 1] and writes the next
                         double* d_new = dbuf[(kk + 1) & 1];
                         {
-                            ProfScope a(ctx, K_EXPLICIT_APPLY, bytes_xapply, kk);
-                            launch_pcg_explicit(P, X, mixed, dbuf[kk & 1], d_new, kk, fresh_kk, s);
+                            ProfScope a(ctx, K_EXPLICIT_APPLY, bytes_xapply(), kk);
+                            launch_pcg_explicit(P, X, x32, dbuf[kk & 1], d_new, kk, fresh_kk, s);
                         }
                         DevProblem Ps = P;
                         Ps.d = d_new;
@@ -1028,7 +1177,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     }
                     // true residual re-check (implicit_schur.rs:613-690, 750-761)
                     const Post<PcgState> checked = pcg_post();
-                    if (xplicit) launch_explicit_true_residual(P, X, 0, checked, s);
+                    if (xp) launch_explicit_true_residual(P, X, 0, checked, s);
                     else launch_pcg_true_residual(P, checked, s);
                     ps = read(checked);
                     if (std::isfinite(ps.true_norm) && ps.true_norm <= ps.target) break;
@@ -1039,7 +1188,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     if (mixed && ps.iter < ps.max_iter) {
                         // FP64 refinement: continue from the true residual
                         const Post<PcgState> restarted = pcg_post();
-                        if (xplicit) {
+                        if (xp) {
                             // the next iteration (ps.iter) starts fresh from d = 0
                             DevProblem Pr = P;
                             Pr.d = dbuf[ps.iter & 1];
@@ -1064,6 +1213,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                 st.pcg_target = ps.target;
                 total_pcg += (uint32_t)ps.iter;
                 pr.last_pcg = ps.iter;
+                last_its = ps.iter;
             }
             const double cost_before = current_cost;
             if (!solved) {  // lm.rs:610-662: a failed solve is a rejected step
