@@ -360,6 +360,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_update(RsDev D, int k, int nu
 struct ElDev {
     int32_t num_edges, num_slots, num_extra, num_run_edges;
     int32_t coarse_group, coarse_nodes, coarse_m, pad;
+    int32_t row_major;  // the caller's blocks (H, V^-1, couplings, run blocks, sums) are row-major
     const int64_t* term_ptr;     // per edge: its terms
     const uint32_t* terms;       // 3 per term: slot index of k, slot index of j, point
     const uint8_t* shard;        // per point
@@ -379,68 +380,121 @@ struct ElDev {
     double* coarse_out;
 };
 
-__global__ __launch_bounds__(kRsThreads) void k_el_scaled(ElDev D) {
+// x = H V^-1, column-major, from blocks whose rows and columns are HR, HK
+// (H, 6 x 3) and VK, VC (V^-1) values apart.
+template <int HR, int HK, int VK, int VC>
+__device__ __forceinline__ void el_scale(const double h[18], const double v[9], double x[18]) {
     // every product and sum rounded on its own, as the CPU's (no fusion)
 #pragma clang fp contract(off)
-    const int q = blockIdx.x * kRsThreads + threadIdx.x;
-    if (q >= D.num_slots) return;
-    const uint32_t p = D.point_of[q];
-    if (!D.has[p]) return;
-    const double* h = D.hcp + 18 * (size_t)q;
-    const double* v = D.vinv + 9 * (size_t)p;
-    double* o = D.scaled + 18 * (size_t)q;
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int r = 0; r < 6; ++r) {
-            double x = h[r] * v[3 * c];
-            x = x + h[6 + r] * v[3 * c + 1];
-            x = x + h[12 + r] * v[3 * c + 2];
-            o[6 * c + r] = x;
+            double t = h[HR * r] * v[VC * c];
+            t = t + h[HR * r + HK] * v[VC * c + VK];
+            t = t + h[HR * r + 2 * HK] * v[VC * c + 2 * VK];
+            x[6 * c + r] = t;
         }
+}
+
+__global__ __launch_bounds__(kRsThreads) void k_el_scaled(ElDev D) {
+    const int q = blockIdx.x * kRsThreads + threadIdx.x;
+    if (q >= D.num_slots) return;
+    const uint32_t p = D.point_of[q];
+    if (!D.has[p]) return;
+    const double2* hv = (const double2*)(D.hcp + 18 * (size_t)q);
+    const double* v = D.vinv + 9 * (size_t)p;
+    double2* o = (double2*)(D.scaled + 18 * (size_t)q);
+    double h[18], vi[9], x[18];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const double2 t = hv[i];
+        h[2 * i] = t.x;
+        h[2 * i + 1] = t.y;
+        vi[i] = v[i];
+    }
+    if (D.row_major) el_scale<3, 1, 3, 1>(h, vi, x);
+    else el_scale<1, 6, 1, 3>(h, vi, x);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) o[i] = make_double2(x[2 * i], x[2 * i + 1]);
 }
 
 // One wave per edge block; lane q < 36 forms entry q (column q / 6, row
 // q % 6) over the edge's terms in point order.
+//
+// An entry is one chain of fused multiply-adds (the CPU's), so its terms
+// cannot be split over lanes; what a term waits for is three dependent loads
+// (its indices, the point's flags, the blocks). Four terms' indices, then
+// their flags and blocks, are loaded before the chain takes them in order
+// (one at a time: 373 us for 41.5k edges and 1.2M terms, 304 here).
 __global__ __launch_bounds__(kRsThreads) void k_el_blocks(ElDev D) {
     const int lane = threadIdx.x & 63;
     const int wg = xcd_tile(blockIdx.x, (D.num_edges + kRsThreads / 64 - 1) / (kRsThreads / 64));
-    const int e = wg * (kRsThreads / 64) + (threadIdx.x >> 6);
+    const int e = __builtin_amdgcn_readfirstlane(wg * (kRsThreads / 64) + (int)(threadIdx.x >> 6));
     if (e >= D.num_edges || lane >= 36) return;
     const int c = lane / 6, r = lane % 6;
+    // row r of an edge's H: its three values a0, a0 + as, a0 + 2 as
+    const int a0 = D.row_major ? 3 * r : r, as = D.row_major ? 1 : 6;
     double total = 0.0, acc = 0.0;
     int cur = -1;
     const int64_t t1 = D.term_ptr[e + 1];
-    for (int64_t t = D.term_ptr[e]; t < t1; ++t) {
-        const uint32_t sk = D.terms[3 * t], sj = D.terms[3 * t + 1], p = D.terms[3 * t + 2];
-        if (!D.has[p]) continue;
-        const int sh = D.shard[p];
-        if (sh != cur) {
-            if (cur >= 0) {
-                total = total + acc;
-                acc = 0.0;
-            }
-            cur = sh;
+    constexpr int KB = 4;
+    for (int64_t t0 = D.term_ptr[e]; t0 < t1; t0 += KB) {
+        uint32_t sk[KB], sj[KB], p[KB];
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            const int64_t t = min(t0 + u, t1 - 1);
+            sk[u] = D.terms[3 * t];
+            sj[u] = D.terms[3 * t + 1];
+            p[u] = D.terms[3 * t + 2];
         }
-        const double* b = D.scaled + 18 * (size_t)sk;
-        const double* a = D.hcp + 18 * (size_t)sj;
-        acc = fma(a[12 + r], -b[12 + c], fma(a[6 + r], -b[6 + c], fma(a[r], -b[c], acc)));
+        int has[KB], sh[KB];
+        double a[KB][3], b[KB][3];
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            has[u] = D.has[p[u]];
+            sh[u] = D.shard[p[u]];
+            const double* bs = D.scaled + 18 * (size_t)sk[u];
+            const double* ah = D.hcp + 18 * (size_t)sj[u];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                b[u][k] = bs[6 * k + c];
+                a[u][k] = ah[a0 + k * as];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            if (t0 + u >= t1 || !has[u]) continue;
+            if (sh[u] != cur) {
+                if (cur >= 0) {
+                    total = total + acc;
+                    acc = 0.0;
+                }
+                cur = sh[u];
+            }
+            acc = fma(a[u][2], -b[u][2], fma(a[u][1], -b[u][1], fma(a[u][0], -b[u][0], acc)));
+        }
     }
     if (cur >= 0) total = total + acc;
     D.b64[36 * (size_t)e + lane] = total;
 }
+
+// The place in the caller's 6 x 6 block of an entry of a column-major one, and
+// the other way round.
+__device__ __forceinline__ int caller_entry(const ElDev& D, int q) { return D.row_major ? q % 6 * 6 + q / 6 : q; }
 
 // Direct couplings (one per edge at most), then the FP32 blocks of the solve.
 __global__ __launch_bounds__(kRsThreads) void k_el_extra(ElDev D) {
     const size_t i = (size_t)blockIdx.x * kRsThreads + threadIdx.x;
     if (i >= 36 * (size_t)D.num_extra) return;
     const size_t k = 36 * (size_t)D.extra_edge[i / 36] + i % 36;
-    D.b64[k] = D.b64[k] + D.extra_blocks[i];
+    D.b64[k] = D.b64[k] + D.extra_blocks[i / 36 * 36 + caller_entry(D, (int)(i % 36))];
 }
 __global__ __launch_bounds__(kRsThreads) void k_el_store(ElDev D) {
     const size_t i = (size_t)blockIdx.x * kRsThreads + threadIdx.x;
     if (i < 36 * (size_t)D.num_edges) D.off[i] = __double2float_rn(D.b64[i]);
-    if (i < 36 * (size_t)D.num_run_edges) D.run_out[i] = D.b64[36 * (size_t)D.run_edges[i / 36] + i % 36];
+    if (i < 36 * (size_t)D.num_run_edges)
+        D.run_out[i] = D.b64[36 * (size_t)D.run_edges[i / 36] + caller_entry(D, (int)(i % 36))];
 }
 
 // Aggregate pair (g, h), g <= h: the sum of the blocks of edges (a, b), a in
@@ -470,7 +524,7 @@ __global__ __launch_bounds__(kRsThreads) void k_el_coarse(ElDev D) {
         }
     }
 #pragma unroll
-    for (int q = 0; q < 36; ++q) o[q] = sum[q];
+    for (int q = 0; q < 36; ++q) o[caller_entry(D, q)] = sum[q];
 }
 
 }  // namespace
@@ -769,6 +823,7 @@ int32_t reduced_eliminate(Context& ctx, const vba_point_elimination& el, double*
         D.coarse_group = (int32_t)el.coarse_group;
         D.coarse_nodes = (int32_t)el.coarse_nodes;
         D.coarse_m = m;
+        D.row_major = (int32_t)(el.reserved & VBA_ELIMINATION_ROW_MAJOR);
         if (el.structure_id != R.elim_structure || R.structure_id != el.structure_id || R.n != (int32_t)n ||
             R.num_edges != (int32_t)E) {
             // validate the structure and build the pair index

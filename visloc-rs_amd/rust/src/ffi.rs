@@ -71,6 +71,7 @@ pub const VBA_GNC_GEMAN_MCCLURE: u32 = 0;
 pub const VBA_GNC_TRUNCATED_LEAST_SQUARES: u32 = 1;
 
 pub const VBA_DENSE_NOALLOC_MAX_N: u32 = 1024;
+pub const VBA_ELIMINATION_ROW_MAJOR: u32 = 1;
 
 #[repr(C)]
 #[derive(Clone, Copy, Debug)]

@@ -240,6 +240,8 @@ class ServerConfig(C.Structure):
     ]
 
 
+ELIMINATION_ROW_MAJOR = 1  # vba_point_elimination.reserved
+
 GNC_GEMAN_MCCLURE = 0
 GNC_TRUNCATED_LEAST_SQUARES = 1
 

@@ -330,9 +330,14 @@ class PointEliminationInput:
         group, nodes = self.coarse
         return -(-nodes // group)
 
-    def view(self):
-        """(abi.PointElimination, arrays to keep alive while it is used)."""
-        col = lambda m: np.ascontiguousarray(np.swapaxes(np.asarray(m, np.float64), -1, -2))
+    def view(self, row_major: bool = False):
+        """(abi.PointElimination, arrays to keep alive while it is used):
+        column-major copies of the blocks, or with row_major the blocks as
+        they are (abi.ELIMINATION_ROW_MAJOR)."""
+        def blocks(m, r, c):
+            m = np.asarray(m, np.float64).reshape(-1, r, c)
+            return np.ascontiguousarray(m if row_major else np.swapaxes(m, -1, -2))
+
         arrs = dict(
             edges=np.ascontiguousarray(np.asarray(self.edges, np.uint32).reshape(-1, 2)),
             row_off=np.ascontiguousarray(self.row_off, np.uint64),
@@ -340,12 +345,12 @@ class PointEliminationInput:
             slots=np.ascontiguousarray(np.asarray(self.slots, np.uint32).reshape(-1, 2)),
             point_off=np.ascontiguousarray(self.point_off, np.uint64),
             point_nodes=np.ascontiguousarray(self.point_nodes, np.uint32),
-            hcp=col(np.asarray(self.hcp).reshape(-1, 6, 3)),
-            point_inverse=col(np.asarray(self.point_inverse).reshape(-1, 3, 3)),
+            hcp=blocks(self.hcp, 6, 3),
+            point_inverse=blocks(self.point_inverse, 3, 3),
             has_inverse=np.ascontiguousarray(self.has_inverse, np.uint8),
             scale=np.ascontiguousarray(np.asarray(self.scale, np.float64).reshape(-1, 6)),
             extra_edge=np.ascontiguousarray(self.extra_edge, np.uint32),
-            extra_blocks=col(np.asarray(self.extra_blocks).reshape(-1, 6, 6)),
+            extra_blocks=blocks(self.extra_blocks, 6, 6),
             run_edges=np.ascontiguousarray(self.run_edges, np.uint32),
         )
         v = abi.PointElimination()
@@ -356,6 +361,7 @@ class PointEliminationInput:
         v.num_points = len(arrs["point_off"]) - 1
         v.num_extra = len(arrs["extra_edge"])
         v.num_run_edges = len(arrs["run_edges"])
+        v.reserved = abi.ELIMINATION_ROW_MAJOR if row_major else 0
         if self.coarse is not None:
             v.coarse_group, v.coarse_nodes = int(self.coarse[0]), int(self.coarse[1])
         ptr = {np.dtype(np.uint32): abi.PU32, np.dtype(np.uint64): abi.PU64, np.dtype(np.uint8): abi.PU8,
@@ -562,10 +568,10 @@ class Device:
         6x6 here, or None where the trait returns None. The blocks stay on
         the device for the next reduced_solve(offdiag=None) of the
         structure."""
-        view, keep = elim.view()
-        runs = np.zeros((max(1, len(elim.run_edges)), 36))
+        view, keep = elim.view(row_major=True)
+        runs = np.empty((max(1, len(elim.run_edges)), 36))
         m = elim.coarse_aggregates()
-        coarse = np.zeros((max(1, m * m), 36))
+        coarse = np.empty((max(1, m * m), 36))
         st = self.lib.vba_reduced_eliminate(self.ctx, C.byref(view), runs.ctypes.data_as(abi.P64),
                                             coarse.ctypes.data_as(abi.P64))
         del keep
@@ -573,8 +579,8 @@ class Device:
             return None
         if st != abi.OK:
             raise RuntimeError(f"vba_reduced_eliminate: {st} {self.last_error()}")
-        rb = np.swapaxes(runs[:len(elim.run_edges)].reshape(-1, 6, 6), -1, -2).copy()
-        cs = np.swapaxes(coarse[:m * m].reshape(m, m, 6, 6), -1, -2).copy() if m else None
+        rb = runs[:len(elim.run_edges)].reshape(-1, 6, 6)
+        cs = coarse[:m * m].reshape(m, m, 6, 6) if m else None
         return rb, cs
 
     def optimize_batch(self, problems: List[BundleProblem], options: abi.Options,
