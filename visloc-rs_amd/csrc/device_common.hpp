@@ -32,6 +32,40 @@ __device__ __forceinline__ size_t g32_off2(int pp) {
 }
 inline int blocks_for(int n, int per) { return (n + per - 1) / per; }
 
+__device__ __forceinline__ double from_halves(unsigned lo, unsigned hi) {
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The value of the partner lane under DPP control CTRL (within a row).
+template <int CTRL>
+__device__ __forceinline__ double dpp_partner(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xf, 0xf, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+    return from_halves(lo, hi);
+}
+
+// One halving step of wave_sum36: the lane and its partner sum a where the
+// lane's `upper` is false and b where it is true.
+template <int CTRL>
+__device__ __forceinline__ double halve_dpp(double a, double b, bool upper) {
+    return (upper ? b : a) + dpp_partner<CTRL>(upper ? a : b);
+}
+__device__ __forceinline__ double halve_rows(double a, double b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a),
+                             y = (unsigned long long)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return from_halves(lo[0], hi[0]) + from_halves(lo[1], hi[1]);
+}
+__device__ __forceinline__ double halve_wave(double a, double b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a),
+                             y = (unsigned long long)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return from_halves(lo[0], hi[0]) + from_halves(lo[1], hi[1]);
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
@@ -67,6 +101,41 @@ __device__ __forceinline__ void block_sum(T (&v)[N], T* lds) {
         }
     }
     __syncthreads();
+}
+// Sums of N values over an NT-thread work-group, value i to out[i], with
+// block_sum's additions in block_sum's order (so the same bits) but lane moves
+// in the VALU and half as many values after each of the first two steps:
+// lanes pair i with i + 32 and i + 16 by permlane swaps, one lane of a pair
+// keeping one half of the values, then i + 8, 4, 2, 1 by row rotations. With
+// 27 values, 147 VALU instructions a wave where shuffles take 324 LDS ones.
+// lds must hold (NT / 64) * 4 * ceil(N / 4) values.
+template <int NT, int N>
+__device__ __forceinline__ void block_sum_out(const double (&v)[N], double* lds, double* out) {
+    constexpr int NW = NT / 64, H = (N + 1) / 2, Q = (H + 1) / 2;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double a[H], b[Q];
+#pragma unroll
+    for (int i = 0; i < H; ++i) a[i] = halve_wave(v[i], i + H < N ? v[i + H] : 0.0);
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        b[i] = halve_rows(a[i], i + Q < H ? a[i + Q] : 0.0);
+        b[i] = b[i] + dpp_partner<0x128>(b[i]);  // row_ror:8
+        b[i] = b[i] + dpp_partner<0x124>(b[i]);  // row_ror:4
+        b[i] = b[i] + dpp_partner<0x122>(b[i]);  // row_ror:2
+        b[i] = b[i] + dpp_partner<0x121>(b[i]);  // row_ror:1
+    }
+    // row r of the wave holds values H (r >> 1) + Q (r & 1) + i
+    if ((lane & 15) == 0)
+#pragma unroll
+        for (int i = 0; i < Q; ++i) lds[(4 * wave + (lane >> 4)) * Q + i] = b[i];
+    __syncthreads();
+    if ((int)threadIdx.x < N) {
+        const int i = threadIdx.x, h = i >= H, r = i - h * H, q = r >= Q;
+        const double* p = lds + (2 * h + q) * Q + (r - q * Q);
+        double s = p[0];
+        for (int w = 1; w < NW; ++w) s += p[4 * w * Q];
+        out[i] = s;
+    }
 }
 // Sum broadcast to every thread.
 template <int NT, typename T, int N>
@@ -125,6 +194,37 @@ __device__ __forceinline__ CSum csum_merge(CSum a, CSum b) {
     return r;
 }
 
+// Compensated sum over an NT-thread work-group as a pairwise tree over the
+// thread index (valid in thread 0): the order does not depend on NT for
+// leaves that are zero from some thread on, so a window's cost is the same
+// summed by 256 threads in a batch and by 1,024 alone. (A fold over the
+// threads in one thread is up to 1,024 dependent merges, 26 to 40 us.)
+template <int NT>
+__device__ __forceinline__ CSum block_csum(CSum a, double (*lds)[2]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const CSum o{__shfl_down(a.s, off, 64), __shfl_down(a.c, off, 64)};
+        if ((lane & (2 * off - 1)) == 0) a = csum_merge(a, o);
+    }
+    if (lane == 0) {
+        lds[wave][0] = a.s;
+        lds[wave][1] = a.c;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        constexpr int NW = NT / 64;
+        a = lane < NW ? CSum{lds[lane][0], lds[lane][1]} : CSum{0.0, 0.0};
+#pragma unroll
+        for (int off = 1; off < NW; off <<= 1) {
+            const CSum o{__shfl_down(a.s, off, 64), __shfl_down(a.c, off, 64)};
+            if ((lane & (2 * off - 1)) == 0) a = csum_merge(a, o);
+        }
+    }
+    __syncthreads();
+    return a;
+}
+
 // Packed upper-triangle index of a symmetric 6x6.
 __host__ __device__ constexpr int up6(int i, int j) { return i * 6 - i * (i - 1) / 2 + (j - i); }
 
@@ -175,40 +275,6 @@ __device__ __forceinline__ void sym6_mul(const double* U, const double* x, doubl
         for (int j = 0; j < 6; ++j) s += U[i <= j ? up6(i, j) : up6(j, i)] * x[j];
         y[i] = s;
     }
-}
-
-__device__ __forceinline__ double from_halves(unsigned lo, unsigned hi) {
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// The value of the partner lane under DPP control CTRL (within a row).
-template <int CTRL>
-__device__ __forceinline__ double dpp_partner(double v) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xf, 0xf, false);
-    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
-    return from_halves(lo, hi);
-}
-
-// One halving step of wave_sum36: the lane and its partner sum a where the
-// lane's `upper` is false and b where it is true.
-template <int CTRL>
-__device__ __forceinline__ double halve_dpp(double a, double b, bool upper) {
-    return (upper ? b : a) + dpp_partner<CTRL>(upper ? a : b);
-}
-__device__ __forceinline__ double halve_rows(double a, double b) {
-    const unsigned long long x = (unsigned long long)__double_as_longlong(a),
-                             y = (unsigned long long)__double_as_longlong(b);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-    return from_halves(lo[0], hi[0]) + from_halves(lo[1], hi[1]);
-}
-__device__ __forceinline__ double halve_wave(double a, double b) {
-    const unsigned long long x = (unsigned long long)__double_as_longlong(a),
-                             y = (unsigned long long)__double_as_longlong(b);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-    return from_halves(lo[0], hi[0]) + from_halves(lo[1], hi[1]);
 }
 
 // Sums of 36 values over a wave, one sum per lane: a lane of each pair keeps

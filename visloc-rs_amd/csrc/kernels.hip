@@ -91,7 +91,7 @@ __device__ __forceinline__ bool stereo_rows(const DevProblem& P, int o, const De
 // ---------------------------------------------------------------------------
 template <bool RIG>
 __global__ __launch_bounds__(kBlock) void k_linearize(DevProblem P, int store32) {
-    __shared__ double lds[(kBlock / 64) * 27];
+    __shared__ double lds[(kBlock / 64) * 28];
     const int tile = xcd_tile(blockIdx.x, P.num_cam_tiles);
     if (tile >= P.num_cam_tiles) return;
     if (P.wstate && !P.wstate[P.cam_tile_win[tile]].relin) return;
@@ -193,28 +193,29 @@ __global__ __launch_bounds__(kBlock) void k_linearize(DevProblem P, int store32)
         acc[25] += X[2] * h[0] - X[0] * h[2];
         acc[26] += X[0] * h[1] - X[1] * h[0];
     }
-    block_sum<kBlock, double, 27>(acc, lds);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int i = 0; i < 27; ++i) P.tile27[27 * (size_t)tile + i] = acc[i];
-    }
+    block_sum_out<kBlock, 27>(acc, lds, P.tile27 + 27 * (size_t)tile);
 }
 
-// U_p, g_p: in-order sum of the pose's tile partials.
-__global__ void k_camera_finalize(DevProblem P) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= P.num_pose_slots) return;
+// U_p, g_p: in-order sum of the pose's tile partials, a lane per value and
+// half a wave per pose. The tiles are one chain of additions a value, so their
+// loads go out eight at a time. (A thread per pose with all 27 values: 40 to
+// 70 us where a pose has tens of tiles, 2 to 5 us here.)
+__global__ __launch_bounds__(kBlock) void k_camera_finalize(DevProblem P) {
+    const int p = blockIdx.x * (kBlock / 32) + (int)(threadIdx.x >> 5), i = threadIdx.x & 31;
+    if (p >= P.num_pose_slots || i >= 27) return;
     if (P.wstate && !P.wstate[P.pose_win[p]].relin) return;
-    double acc[27];
+    const int t1 = P.cam_tile_ptr[p + 1];
+    double acc = 0.0;
+    for (int t = P.cam_tile_ptr[p]; t < t1; t += 8) {
+        double v[8];
 #pragma unroll
-    for (int i = 0; i < 27; ++i) acc[i] = 0.0;
-    for (int t = P.cam_tile_ptr[p]; t < P.cam_tile_ptr[p + 1]; ++t)
+        for (int u = 0; u < 8; ++u) v[u] = P.tile27[27 * (size_t)min(t + u, t1 - 1) + i];
 #pragma unroll
-        for (int i = 0; i < 27; ++i) acc[i] += P.tile27[27 * (size_t)t + i];
-#pragma unroll
-    for (int i = 0; i < 21; ++i) P.U[21 * (size_t)p + i] = acc[i];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) P.g[6 * (size_t)p + i] = acc[21 + i];
+        for (int u = 0; u < 8; ++u)
+            if (t + u < t1) acc += v[u];
+    }
+    if (i < 21) P.U[21 * (size_t)p + i] = acc;
+    else P.g[6 * (size_t)p + i - 21] = acc;
 }
 
 // V_l, g_l: in-order sum over the landmark's l-order edges.
@@ -453,15 +454,11 @@ __global__ __launch_bounds__(kBlock) void k_cost(DevProblem P, int trial) {
 
 __global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, int num_pose_blocks,
                                                                  Post<StepScalars> post) {
-    __shared__ double lds[(kSmallBlock / 64) * 4];
-    // cost partials in tile order: thread t < parts merges a contiguous run
-    // of per tiles, and thread 0 folds the parts in order. Up to
-    // kSmallBlock tiles a part is one tile (the fold is then the tile-order
-    // fold that k_batch_scalars does for a window); beyond, 128 parts keep
-    // the serial fold short.
+    __shared__ double lds[(kSmallBlock / 64) * 4], cl[kSmallBlock / 64][2];
+    // cost partials: thread t merges a contiguous run of tiles, then a tree
+    // over the threads
     const int n = P.num_cam_tiles;
-    const int parts = n <= kSmallBlock ? n : 128;
-    const int per = parts > 0 ? (n + parts - 1) / parts : 0;
+    const int per = (n + kSmallBlock - 1) / kSmallBlock;
     CSum cs{0.0, 0.0};
     double bad = 0.0, mp = 0.0, ml = 0.0;
     // (unrolled so that each thread's loads are in flight together; the
@@ -478,18 +475,12 @@ __global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, 
 #pragma unroll 8
     for (int i = threadIdx.x; i < num_pose_blocks; i += kSmallBlock)
         mp = fmax(mp, P.tile_scalar[4 * (size_t)(n + P.num_lm_tiles + i) + 3]);
-    // ordered merge across threads through LDS (thread order = tile order)
-    __shared__ double ss[kSmallBlock], sc[kSmallBlock];
-    ss[threadIdx.x] = cs.s;
-    sc[threadIdx.x] = cs.c;
+    const CSum a = block_csum<kSmallBlock>(cs, cl);
     double v[1] = {bad};
     block_sum<kSmallBlock, double, 1>(v, lds);
     const double m1 = block_max<kSmallBlock>(mp, lds + 16);
     const double m2 = block_max<kSmallBlock>(ml, lds + 32);
-    __syncthreads();
     if (threadIdx.x == 0) {
-        CSum a{ss[0], sc[0]};
-        for (int i = 1; i < parts; ++i) a = csum_merge(a, CSum{ss[i], sc[i]});
         StepScalars* o = P.scalars;
         o->cost_sum = a.s;
         o->cost_comp = a.c;
@@ -1503,8 +1494,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_batch_dense_solve(DevProbl
 // Per window: compensated cost and non-projectable count over its camera
 // tiles (tile order), and the largest pose / landmark step.
 __global__ __launch_bounds__(kBlock) void k_batch_scalars(DevProblem P, BatchDev B) {
-    __shared__ double ss[kBlock], sc[kBlock];
-    __shared__ double lds[(kBlock / 64) * 3];
+    __shared__ double lds[(kBlock / 64) * 3], cl[kBlock / 64][2];
     const int w = blockIdx.x;
     WindowState& st = B.state[w];
     if (!st.active) return;
@@ -1529,16 +1519,12 @@ __global__ __launch_bounds__(kBlock) void k_batch_scalars(DevProblem P, BatchDev
         const double* d = P.delta_l + 3 * (size_t)l;
         v[2] = fmax(v[2], sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]));
     }
-    ss[threadIdx.x] = cs.s;
-    sc[threadIdx.x] = cs.c;
+    const CSum a = block_csum<kBlock>(cs, cl);
     double cnt[1] = {v[0]};
     block_sum<kBlock, double, 1>(cnt, lds);
     const double mp = block_max<kBlock>(v[1], lds);
     const double ml = block_max<kBlock>(v[2], lds);
-    __syncthreads();
     if (threadIdx.x == 0) {
-        CSum a{ss[0], sc[0]};
-        for (int i = 1; i < kBlock; ++i) a = csum_merge(a, CSum{ss[i], sc[i]});
         st.cost_after = a.s + a.c;
         st.nonproj_after = (uint64_t)cnt[0];
         st.max_pose_step = mp;
@@ -1988,7 +1974,7 @@ void launch_linearize(const DevProblem& P, bool store32, hipStream_t s) {
         hipLaunchKernelGGL(k_linearize<false>, dim3(xcd_grid(P.num_cam_tiles)), dim3(kBlock), 0, s, P, (int)store32);
 }
 void launch_camera_finalize(const DevProblem& P, hipStream_t s) {
-    hipLaunchKernelGGL(k_camera_finalize, dim3(blocks_for(P.num_pose_slots, 256)), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(k_camera_finalize, dim3(blocks_for(P.num_pose_slots, kBlock / 32)), dim3(kBlock), 0, s, P);
 }
 void launch_landmark_reduce(const DevProblem& P, hipStream_t s) {
     hipLaunchKernelGGL(k_landmark_reduce, dim3(blocks_for(P.num_lm_slots, 256)), dim3(256), 0, s, P);
