@@ -94,8 +94,10 @@ enum vba_robust_kernel {
  * (implicit_schur.rs:133-824); PCG_EXPLICIT is the same PCG on an explicitly
  * assembled block-sparse Schur matrix. A MATRIX_FREE problem forms that matrix
  * too, after a PCG solve, where the iterations left are faster on it and it
- * takes at most 144 bytes an edge (FP64 blocks, in mixed precision too); it
- * stays with the edges otherwise, also when the memory is not to be had. */
+ * takes at most 144 bytes an edge; it stays with the edges otherwise, also when
+ * the memory is not to be had. The matrix holds the operator that the product
+ * over the edges applies (that of the FP32-stored blocks in mixed precision),
+ * in FP64, and replaces that product alone. */
 enum vba_linear_solver {
     VBA_SOLVER_DENSE = 0,
     /* LinearSolver::Sparse (normal_equations.rs:1483-1535): the reduced

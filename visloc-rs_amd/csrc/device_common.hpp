@@ -321,7 +321,13 @@ __device__ __forceinline__ int wave_entry36(int lane) {
 // the 3.5M-observation loop's 27.5M terms, lists in first-met order, against
 // 492 us with the lists row by row: that one reads 4.6 GB of blocks through
 // L1 and is bound there.
+//
+// With F32 the sum is of the mixed operator's blocks, its FP32-stored G and the
+// V^-1 that it pairs with them: G rounded as it loads gives the same values.
+template <bool F32>
 __device__ __forceinline__ double schur_block_wave(const DevProblem& P, const DensePairs& D, int b, int lane) {
+    const double* const Vinv = F32 ? P.VinvM : P.Vinv64;
+    auto stored = [](double2 v) { return F32 ? make_double2((float)v.x, (float)v.y) : v; };
     double acc[36];
 #pragma unroll
     for (int i = 0; i < 36; ++i) acc[i] = 0.0;
@@ -331,13 +337,13 @@ __device__ __forceinline__ double schur_block_wave(const DevProblem& P, const De
         const int32_t* t = D.terms + 3 * (size_t)k;
         int l = t[0], ep = t[1], eq = t[2];
         while (true) {
-            const double2* v2 = (const double2*)(P.Vinv64 + 6 * (size_t)l);
+            const double2* v2 = (const double2*)(Vinv + 6 * (size_t)l);
             const double2* a2 = (const double2*)(P.Gl64 + 6 * (size_t)ep);
             const double2* b2 = (const double2*)(P.Gl64 + 6 * (size_t)eq);
             const double* X = P.lms + 3 * (size_t)l;
             const double2 v01 = v2[0], v23 = v2[1], v45 = v2[2];
-            const double2 p01 = a2[0], p23 = a2[1], p45 = a2[2];
-            const double2 q01 = b2[0], q23 = b2[1], q45 = b2[2];
+            const double2 p01 = stored(a2[0]), p23 = stored(a2[1]), p45 = stored(a2[2]);
+            const double2 q01 = stored(b2[0]), q23 = stored(b2[1]), q45 = stored(b2[2]);
             const double x0 = X[0], x1 = X[1], x2 = X[2];
             k += 64;
             const int32_t* tn = D.terms + 3 * (size_t)min(k, end - 1);

@@ -260,12 +260,13 @@ __global__ __launch_bounds__(64) void k_explicit_fill(DevProblem P, ExplicitBuil
 // terms, stored row-major at block_pos[2b] and transposed at
 // block_pos[2b + 1]. The diagonal block keeps its upper triangle and mirrors
 // it, so that it is exactly symmetric.
+template <bool F32>
 __global__ __launch_bounds__(kBlock, 4) void k_explicit_assemble(DevProblem P, DensePairs D, ExplicitDev X,
-                                                               double lambda) {
+                                                                 double lambda) {
     const int b = block_of_wave(D.num_blocks);
     if (b >= D.num_blocks) return;
     const int lane = threadIdx.x & 63;
-    double v = -schur_block_wave(P, D, b, lane);
+    double v = -schur_block_wave<F32>(P, D, b, lane);
     const int sp = D.block_pq[2 * b], sq = D.block_pq[2 * b + 1];
     const int pos = X.block_pos[2 * b], idx = wave_entry36(lane);
     if (idx < 0) return;
@@ -500,10 +501,14 @@ void launch_explicit_lists(const DevProblem& P, const ExplicitBuild& B, int32_t 
     hipLaunchKernelGGL(k_explicit_fill, dim3(n), dim3(64), lds, s, P, B);
 }
 
-void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, double lambda,
+void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, bool f32, double lambda,
                               hipStream_t s) {
-    if (D.num_blocks)
-        hipLaunchKernelGGL(k_explicit_assemble, dim3(block_grid(D.num_blocks)), dim3(kBlock), 0, s, P, D, X, lambda);
+    if (!D.num_blocks) return;
+    const auto kernel = f32 ? k_explicit_assemble<true> : k_explicit_assemble<false>;
+    hipLaunchKernelGGL(kernel, dim3(block_grid(D.num_blocks)), dim3(kBlock), 0, s, P, D, X, lambda);
+}
+
+void launch_explicit_precond(const DevProblem& P, const ExplicitDev& X, hipStream_t s) {
     hipLaunchKernelGGL(k_explicit_precond, dim3(blocks_for(P.num_pose_slots, kBlock)), dim3(kBlock), 0, s, P, X);
 }
 

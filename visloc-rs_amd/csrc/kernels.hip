@@ -511,7 +511,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_scalars_finalize(DevProblem P, 
 __device__ __forceinline__ void dense_assemble_wave(const DevProblem& P, const DensePairs& D, int b, double* S, int n,
                                                     int var_begin, double lambda, int lane) {
     const int sp = D.block_pq[2 * b], sq = D.block_pq[2 * b + 1];
-    const double v = schur_block_wave(P, D, b, lane);
+    const double v = schur_block_wave<false>(P, D, b, lane);
     const int idx = wave_entry36(lane);
     if (idx < 0) return;
     const int vp = P.pose_var[sp] - var_begin, vq = P.pose_var[sq] - var_begin;

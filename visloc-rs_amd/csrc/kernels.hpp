@@ -294,10 +294,13 @@ void launch_explicit_rows(const DevProblem& P, const ExplicitBuild& B, hipStream
 // Columns, block positions and the term lists, given row_ptr and up_ptr;
 // max_upper is the largest up_count.
 void launch_explicit_lists(const DevProblem& P, const ExplicitBuild& B, int32_t max_upper, hipStream_t stream);
-// S64 (and S32) from the term lists, U and lambda, then the block-Jacobi
-// inverses of the diagonal blocks into Minv (implicit_schur.rs:241-287).
-void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, double lambda,
+// S64 (and S32) from the term lists, U and lambda; with f32 the Schur terms
+// are those of the mixed operator (FP32-stored G, VinvM).
+void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, bool f32, double lambda,
                               hipStream_t stream);
+// The block-Jacobi inverses of the diagonal blocks into Minv
+// (implicit_schur.rs:241-287).
+void launch_explicit_precond(const DevProblem& P, const ExplicitDev& X, hipStream_t stream);
 // PCG iteration pcg_iter on the explicit matrix: d_new = z + beta d_old,
 // q = S d_new and d.q partials; the scalars come from the step kernel's
 // partials as for the implicit operator. fp32 reads S32.

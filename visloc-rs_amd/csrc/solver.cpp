@@ -823,9 +823,8 @@ constexpr int64_t kExplicitTermBytes = 112, kExplicitBlockBytes = 32;
 // precision, 8.2 us + 0.06 ns a stored block (8.4 us at 163 poses and 9k
 // blocks, 9.8 us at 300 and 29k, 17.3 us at 1,200 and 140k). Against that
 // stand the assembly, 20 us + 17.5 ps a term for every LM iteration (55 us at
-// 2.3M terms, 492 us at 27.5M; the edges' block-Jacobi passes, which it
-// replaces, take 20 us + 30 ps an edge), and the structure, once: 1 ms + 75 ps
-// a term (3.1 ms at 27.5M). The lists' and blocks' memory has to stay within
+// 2.3M terms, 492 us at 27.5M), and the structure, once: 1 ms + 75 ps a term
+// (3.1 ms at 27.5M). The lists' and blocks' memory has to stay within
 // the bounds above, which long tracks (more than some 9 terms an edge) and
 // scenes whose poses share landmarks with most others exceed.
 bool explicit_pays(Prepared& pr, bool mixed, int32_t its, uint32_t remaining, const int32_t* num_full) {
@@ -833,7 +832,7 @@ bool explicit_pays(Prepared& pr, bool mixed, int32_t its, uint32_t remaining, co
     if (12.0 * terms + 4.0 * edges > (double)kExplicitTermBytes * edges) return false;
     const double over_edges = mixed ? 13.6e-6 + 8.1e-12 * edges : 15.6e-6 + 10.7e-12 * edges;
     const double over_matrix = 8.2e-6 + (num_full ? 0.06e-9 * *num_full : 0.0);
-    const double assembly = (20e-6 + 17.5e-12 * terms) - (20e-6 + 30e-12 * edges);
+    const double assembly = 20e-6 + 17.5e-12 * terms;
     const double build = 1e-3 + 75e-12 * terms;
     return (its * (over_edges - over_matrix) - assembly) * remaining > build;
 }
@@ -914,10 +913,13 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             X.S32 = x32 ? (float*)ensure(pr, B_X_S32, 36 * (size_t)X.num_full * sizeof(float)) : nullptr;
             dbuf[1] = (double*)ensure(pr, B_VD2, 6 * NP * sizeof(double));
             hip_check(hipMemsetAsync(dbuf[1], 0, 6 * NP * sizeof(double), s), "memset");
-            P.num_bpart = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);
             return xp = true;
         };
-        if (xplicit) use_explicit(-1);
+        const int32_t row_bparts = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);  // d.q partials of its product
+        if (xplicit) {
+            use_explicit(-1);
+            P.num_bpart = row_bparts;
+        }
         if (!matrix_free) {
             dS = (double*)ensure(pr, B_DENSE_S, (size_t)ndense * ndense * sizeof(double));
             dwork = (double*)ensure(pr, B_DENSE_WORK, dense_work_size(ndense) * sizeof(double));
@@ -940,11 +942,12 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         const double bytes_cost = m.num_obs * 16.0 + NE * 8.0 + NL * 24.0 + NT * (16.0 + 24.0) + NP * 56.0;
         // explicit matrix: per term its indices (12); per edge G and per
         // landmark X and V^-1 once; per stored block 36 values (FP64, and the
-        // FP32 copy); per pose U, the diagonal read and Minv. Product: per
-        // stored block 36 reals and its column; per pose z, d_old, d_new, q.
+        // FP32 copy); per pose U, and for the explicit solver the diagonal
+        // read and Minv. Product: per stored block 36 reals and its column; per
+        // pose z, d_old, d_new, q.
         auto bytes_xassemble = [&]() {
             return (double)count_terms(pr) * 12.0 + NE * 48.0 + NL * 72.0 +
-                   X.num_full * 36.0 * (8.0 + (x32 ? 4.0 : 0.0)) + NP * (168.0 + 288.0 + 288.0);
+                   X.num_full * 36.0 * (8.0 + (x32 ? 4.0 : 0.0)) + NP * (168.0 + (xplicit ? 288.0 + 288.0 : 0.0));
         };
         auto bytes_xapply = [&]() {
             return X.num_full * (36.0 * (x32 ? 4.0 : 8.0) + 4.0) + NP * (4.0 + 4.0 * 48.0);
@@ -1005,7 +1008,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             if (need_lin) {
                 {
                     ProfScope ps(ctx, K_LINEARIZE, bytes_linearize);
-                    launch_linearize(P, P.Gl32 != nullptr, s);
+                    launch_linearize(P, mixed, s);
                 }
                 launch_camera_finalize(P, s);
                 launch_landmark_reduce(P, s);
@@ -1014,8 +1017,14 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                 ++linearizations;
             }
             // The matrix-free solver forms the explicit matrix once the last
-            // PCG solve has shown that it pays (explicit_pays), and keeps it:
-            // its FP32 copies of G are then not needed any more.
+            // PCG solve has shown that it pays (explicit_pays), and keeps it.
+            // The matrix then takes the place of the edges in the PCG product
+            // and nowhere else: in mixed precision it is formed from the
+            // FP32-stored G and the V^-1 that the product over the edges
+            // reads, and the block-Jacobi inverses and the FP64 residual check
+            // stay with the edges. (From FP64 blocks instead, 75 mixed loops
+            // ended up to 8e-5 of the landmarks from those over the edges;
+            // with the same operator 2.6e-8, the median 1.3e-13.)
             if (ask && !xp && last_its > 0 &&
                 explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, nullptr)) {
                 bool done = false;
@@ -1027,11 +1036,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     (void)hipGetLastError();  // no memory for it: stay with the edges
                 }
                 xp = done;
-                if (done) {
-                    P.Gl32 = nullptr;
-                    P.Vm = P.VinvM = nullptr;
-                } else {
-                    P.num_bpart = (int32_t)((NP + (kBlock / 64) - 1) / (kBlock / 64));
+                if (!done) {
                     ask = false;
                     pr.x_refused = true;
                 }
@@ -1063,10 +1068,10 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             } else {
                 if (xp) {
                     ProfScope a(ctx, K_EXPLICIT_ASSEMBLE, bytes_xassemble());
-                    launch_explicit_assemble(P, D, X, lambda, s);
-                } else {
-                    launch_precondition(P, lambda, s);
+                    launch_explicit_assemble(P, D, X, mixed && !xplicit, lambda, s);
+                    if (xplicit) launch_explicit_precond(P, X, s);
                 }
+                if (!xplicit) launch_precondition(P, lambda, s);
                 launch_pcg_init(P, o.pcg_relative_tolerance, o.pcg_absolute_tolerance, max_pcg, lambda, s);
                 int32_t k = 0;
                 int32_t fresh = 1;
@@ -1083,6 +1088,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                         }
                         DevProblem Ps = P;
                         Ps.d = d_new;
+                        Ps.num_bpart = row_bparts;
                         ProfScope c(ctx, K_PCG_STEP, bytes_pcg_step, kk);
                         launch_pcg_step(Ps, kk, s);
                         return;
@@ -1177,7 +1183,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     }
                     // true residual re-check (implicit_schur.rs:613-690, 750-761)
                     const Post<PcgState> checked = pcg_post();
-                    if (xp) launch_explicit_true_residual(P, X, 0, checked, s);
+                    if (xplicit) launch_explicit_true_residual(P, X, 0, checked, s);
                     else launch_pcg_true_residual(P, checked, s);
                     ps = read(checked);
                     if (std::isfinite(ps.true_norm) && ps.true_norm <= ps.target) break;
@@ -1188,14 +1194,11 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     if (mixed && ps.iter < ps.max_iter) {
                         // FP64 refinement: continue from the true residual
                         const Post<PcgState> restarted = pcg_post();
-                        if (xp) {
-                            // the next iteration (ps.iter) starts fresh from d = 0
-                            DevProblem Pr = P;
-                            Pr.d = dbuf[ps.iter & 1];
-                            launch_explicit_true_residual(Pr, X, 1, restarted, s);
-                        } else {
-                            launch_pcg_restart(P, restarted, s);
-                        }
+                        // the next iteration (ps.iter) starts fresh from d = 0
+                        DevProblem Pr = P;
+                        if (xp) Pr.d = dbuf[ps.iter & 1];
+                        if (xplicit) launch_explicit_true_residual(Pr, X, 1, restarted, s);
+                        else launch_pcg_restart(Pr, restarted, s);
                         ps = read(restarted);
                         if (ps.stop) {
                             solved = ps.status == PCG_MAXIT && accept_iterate;
