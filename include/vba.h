@@ -93,9 +93,9 @@ enum vba_robust_kernel {
  * the implicit-Schur block-Jacobi PCG of `optimize_matrix_free`
  * (implicit_schur.rs:133-824); PCG_EXPLICIT is the same PCG on an explicitly
  * assembled block-sparse Schur matrix. A MATRIX_FREE problem forms that matrix
- * too, after a PCG solve, where the iterations left are faster on it and it
- * takes at most 144 bytes an edge; it stays with the edges otherwise, also when
- * the memory is not to be had. The matrix holds the operator that the product
+ * too, after a PCG solve, where pcg_maxit_policy is REJECT, the iterations left
+ * are faster on it and it takes at most 144 bytes an edge; it stays with the
+ * edges otherwise, also when the memory is not to be had. The matrix holds the operator that the product
  * over the edges applies (that of the FP32-stored blocks in mixed precision),
  * in FP64, and replaces that product alone. */
 enum vba_linear_solver {

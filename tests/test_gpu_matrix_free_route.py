@@ -4,13 +4,11 @@ structure and term lists are built on the device from the problem's edges.
 
 Checked over the forms the edges take (fixed poses and landmarks among the
 others, a pose without observations, rig edges with several observations,
-weights, lenses, observations given in any order), in both precisions and at
-both rules at the PCG cap, against the oracle's matrix-free solver with the
-bars of the other parity tests: FP64 final cost within 1e-9 relative, mixed
-1e-6, camera centres within 1e-6 of the extent. The PCG solves run to a
-relative residual of 1e-9: one that stops at the backend's cap of 100 ends
-where rounding leaves it (up to 4e-7 of the cost apart on these scenes on
-either operator), which no bar on an operator can be held against."""
+lenses, observations given in any order), in both precisions, against the
+oracle's matrix-free solver with the bars of the other parity tests: FP64 final
+cost within 1e-9 relative, mixed 1e-6, camera centres within 1e-6 of the
+extent. The PCG solves run to a relative residual of 1e-9 and may not stop
+short of it: a solve that takes the iterate at its cap stays on the edges."""
 import numpy as np
 import pytest
 
@@ -25,7 +23,7 @@ def loop(cams=60, lms=5000, seed=3):
     return vba.synthesize(abi.SYNTH_LOOP, num_cameras=cams, num_landmarks=lms, seed=seed, scene_scale=cams / 6.0)
 
 
-def options(precision, policy=abi.PCG_MAXIT_ACCEPT_ITERATE, iterations=5, **kw):
+def options(precision, policy=abi.PCG_MAXIT_REJECT, iterations=5, **kw):
     o = dict(linear_solver=abi.SOLVER_MATRIX_FREE, max_iterations=iterations, max_pcg_iterations=1000,
              pcg_relative_tolerance=1e-9, robust_kernel=abi.KERNEL_HUBER, robust_scale=1.0, precision=precision,
              pcg_maxit_policy=policy)
@@ -68,10 +66,9 @@ def compare(device, problem, extent, o):
 
 
 @pytest.mark.parametrize("precision", [abi.PRECISION_FP64, abi.PRECISION_MIXED])
-@pytest.mark.parametrize("policy", [abi.PCG_MAXIT_ACCEPT_ITERATE, abi.PCG_MAXIT_REJECT])
-def test_loop(device, precision, policy):
+def test_loop(device, precision):
     s = loop()
-    compare(device, s.problem, s.scene_extent, options(precision, policy))
+    compare(device, s.problem, s.scene_extent, options(precision))
 
 
 @pytest.mark.parametrize("precision", [abi.PRECISION_FP64, abi.PRECISION_MIXED])
@@ -85,7 +82,8 @@ def test_fixed_and_unobserved(device, precision):
     order = np.random.default_rng(1).permutation(len(p.obs_xy))
     p.obs_pose_ids, p.obs_landmark_ids, p.obs_xy = p.obs_pose_ids[order], p.obs_landmark_ids[order], p.obs_xy[order]
     p.pose_fixed[40] = 1
-    compare(device, p, s.scene_extent, options(precision, iterations=30))
+    # (damped enough for every system to reach its residual)
+    compare(device, p, s.scene_extent, options(precision, iterations=30, initial_lambda=0.1, min_lambda=0.1))
 
 
 def test_rig_edges(device):

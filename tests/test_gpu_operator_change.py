@@ -7,7 +7,9 @@ starts from its state and damping. The matrix replaces the product alone and
 holds the same operator, so both solves are the same up to FP64 rounding: with
 every step a converged one (REJECT at the cap of 100, relative residual 1e-4,
 the workloads' setting) 110 scenes ended within 2.6e-8 of each other; the bar
-is 1e-6."""
+is 1e-6. Where the iterate at the cap is taken as it is (ACCEPT_ITERATE), the
+answer hangs on the operator's rounding, and the whole solve stays on the edges:
+bit for bit the same."""
 import numpy as np
 import pytest
 
@@ -67,3 +69,16 @@ def test_the_matrix_is_the_edges_operator(device, precision, cameras, landmarks,
     assert out.accepted == accepted and any(accepted)
     assert relative(out.poses, poses) <= 1e-6
     assert relative(out.landmarks, lms) <= 1e-6
+
+
+@pytest.mark.parametrize("precision", [abi.PRECISION_FP64, abi.PRECISION_MIXED])
+@pytest.mark.parametrize("cameras,landmarks,seed,iterations", [(163, 40009, 7003, 15), (114, 11423, 1527, 15)])
+def test_capped_iterates_keep_their_operator(device, precision, cameras, landmarks, seed, iterations):
+    problem = scene(cameras, landmarks, seed)
+    o = workloads.loop_options(precision, abi.PCG_MAXIT_ACCEPT_ITERATE, max_iterations=iterations)
+    out, over_edges, over_matrix = launches(device, problem, o)
+    assert any(it["pcg_iterations"] == o.max_pcg_iterations for it in out.iterations)
+    assert over_edges > 0 and over_matrix == 0
+    poses, lms, accepted = one_iteration_at_a_time(device, problem, o)
+    assert out.accepted == accepted
+    assert np.array_equal(out.poses, poses) and np.array_equal(out.landmarks, lms)
