@@ -95,9 +95,9 @@ enum vba_robust_kernel {
  * assembled block-sparse Schur matrix. A MATRIX_FREE problem forms that matrix
  * too, after a PCG solve, where pcg_maxit_policy is REJECT, the iterations left
  * are faster on it and it takes at most 144 bytes an edge; it stays with the
- * edges otherwise, also when the memory is not to be had. The matrix holds the operator that the product
- * over the edges applies (that of the FP32-stored blocks in mixed precision),
- * in FP64, and replaces that product alone. */
+ * edges otherwise, also when the memory is not to be had. The matrix holds, in FP64, the operator that the
+ * product over the edges applies: that of the FP32-stored blocks in mixed
+ * precision. */
 enum vba_linear_solver {
     VBA_SOLVER_DENSE = 0,
     /* LinearSolver::Sparse (normal_equations.rs:1483-1535): the reduced

@@ -823,7 +823,8 @@ constexpr int64_t kExplicitTermBytes = 112, kExplicitBlockBytes = 32;
 // precision, 8.2 us + 0.06 ns a stored block (8.4 us at 163 poses and 9k
 // blocks, 9.8 us at 300 and 29k, 17.3 us at 1,200 and 140k). Against that
 // stand the assembly, 20 us + 17.5 ps a term for every LM iteration (55 us at
-// 2.3M terms, 492 us at 27.5M), and the structure, once: 1 ms + 75 ps a term
+// 2.3M terms, 492 us at 27.5M; in FP64 it replaces the edges' block-Jacobi
+// passes, 20 us + 30 ps an edge), and the structure, once: 1 ms + 75 ps a term
 // (3.1 ms at 27.5M). The lists' and blocks' memory has to stay within
 // the bounds above, which long tracks (more than some 9 terms an edge) and
 // scenes whose poses share landmarks with most others exceed.
@@ -832,7 +833,7 @@ bool explicit_pays(Prepared& pr, bool mixed, int32_t its, uint32_t remaining, co
     if (12.0 * terms + 4.0 * edges > (double)kExplicitTermBytes * edges) return false;
     const double over_edges = mixed ? 13.6e-6 + 8.1e-12 * edges : 15.6e-6 + 10.7e-12 * edges;
     const double over_matrix = 8.2e-6 + (num_full ? 0.06e-9 * *num_full : 0.0);
-    const double assembly = 20e-6 + 17.5e-12 * terms;
+    const double assembly = 20e-6 + 17.5e-12 * terms - (mixed ? 0.0 : 20e-6 + 30e-12 * edges);
     const double build = 1e-3 + 75e-12 * terms;
     return (its * (over_edges - over_matrix) - assembly) * remaining > build;
 }
@@ -896,6 +897,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         ExplicitDev X{};
         bool xp = false;
         const bool x32 = xplicit && mixed;           // FP32 copy for its products
+        const bool x64 = xplicit || !mixed;          // it holds the FP64 operator
         double* dbuf[2] = {P.d, nullptr};            // PCG direction by iteration parity
         auto use_explicit = [&](int64_t max_full) {
             if (!build_explicit(pr, P, max_full, s)) return false;
@@ -915,11 +917,14 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             hip_check(hipMemsetAsync(dbuf[1], 0, 6 * NP * sizeof(double), s), "memset");
             return xp = true;
         };
-        const int32_t row_bparts = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);  // d.q partials of its product
-        if (xplicit) {
-            use_explicit(-1);
-            P.num_bpart = row_bparts;
-        }
+        if (xplicit) use_explicit(-1);
+        // P as the matrix's kernels take it: their partials, and the direction `d`
+        auto over_matrix = [&](double* d) {
+            DevProblem Px = P;
+            Px.num_bpart = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);
+            Px.d = d;
+            return Px;
+        };
         if (!matrix_free) {
             dS = (double*)ensure(pr, B_DENSE_S, (size_t)ndense * ndense * sizeof(double));
             dwork = (double*)ensure(pr, B_DENSE_WORK, dense_work_size(ndense) * sizeof(double));
@@ -942,12 +947,12 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         const double bytes_cost = m.num_obs * 16.0 + NE * 8.0 + NL * 24.0 + NT * (16.0 + 24.0) + NP * 56.0;
         // explicit matrix: per term its indices (12); per edge G and per
         // landmark X and V^-1 once; per stored block 36 values (FP64, and the
-        // FP32 copy); per pose U, and for the explicit solver the diagonal
-        // read and Minv. Product: per stored block 36 reals and its column; per
+        // FP32 copy); per pose U, and where it is the FP64 operator the
+        // diagonal read and Minv. Product: per stored block 36 reals and its column; per
         // pose z, d_old, d_new, q.
         auto bytes_xassemble = [&]() {
             return (double)count_terms(pr) * 12.0 + NE * 48.0 + NL * 72.0 +
-                   X.num_full * 36.0 * (8.0 + (x32 ? 4.0 : 0.0)) + NP * (168.0 + (xplicit ? 288.0 + 288.0 : 0.0));
+                   X.num_full * 36.0 * (8.0 + (x32 ? 4.0 : 0.0)) + NP * (168.0 + (x64 ? 288.0 + 288.0 : 0.0));
         };
         auto bytes_xapply = [&]() {
             return X.num_full * (36.0 * (x32 ? 4.0 : 8.0) + 4.0) + NP * (4.0 + 4.0 * 48.0);
@@ -1025,13 +1030,13 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             }
             // The matrix-free solver forms the explicit matrix once the last
             // PCG solve has shown that it pays (explicit_pays), and keeps it.
-            // The matrix then takes the place of the edges in the PCG product
-            // and nowhere else: in mixed precision it is formed from the
-            // FP32-stored G and the V^-1 that the product over the edges
-            // reads, and the block-Jacobi inverses and the FP64 residual check
-            // stay with the edges. (From FP64 blocks instead, 75 mixed loops
-            // ended up to 8e-5 of the landmarks from those over the edges;
-            // with the same operator 2.6e-8, the median 1.3e-13.)
+            // The matrix holds the operator that it replaces: in mixed
+            // precision it is formed from the FP32-stored G and the V^-1 that
+            // the product over the edges reads, and takes the place of that
+            // product alone (the block-Jacobi inverses and the residual check
+            // are of the FP64 operator). (From FP64 blocks instead, 75 mixed
+            // loops ended up to 8e-5 of the landmarks from those over the
+            // edges; with the same operator 2.6e-8, the median 1.3e-13.)
             if (ask && !xp && last_its > 0 &&
                 explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, nullptr)) {
                 bool done = false;
@@ -1075,10 +1080,10 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             } else {
                 if (xp) {
                     ProfScope a(ctx, K_EXPLICIT_ASSEMBLE, bytes_xassemble());
-                    launch_explicit_assemble(P, D, X, mixed && !xplicit, lambda, s);
-                    if (xplicit) launch_explicit_precond(P, X, s);
+                    launch_explicit_assemble(P, D, X, !x64, lambda, s);
+                    if (x64) launch_explicit_precond(P, X, s);
                 }
-                if (!xplicit) launch_precondition(P, lambda, s);
+                if (!(xp && x64)) launch_precondition(P, lambda, s);
                 launch_pcg_init(P, o.pcg_relative_tolerance, o.pcg_absolute_tolerance, max_pcg, lambda, s);
                 int32_t k = 0;
                 int32_t fresh = 1;
@@ -1093,11 +1098,8 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                             ProfScope a(ctx, K_EXPLICIT_APPLY, bytes_xapply(), kk);
                             launch_pcg_explicit(P, X, x32, dbuf[kk & 1], d_new, kk, fresh_kk, s);
                         }
-                        DevProblem Ps = P;
-                        Ps.d = d_new;
-                        Ps.num_bpart = row_bparts;
                         ProfScope c(ctx, K_PCG_STEP, bytes_pcg_step, kk);
-                        launch_pcg_step(Ps, kk, s);
+                        launch_pcg_step(over_matrix(d_new), kk, s);
                         return;
                     }
                     {
@@ -1190,7 +1192,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                     }
                     // true residual re-check (implicit_schur.rs:613-690, 750-761)
                     const Post<PcgState> checked = pcg_post();
-                    if (xplicit) launch_explicit_true_residual(P, X, 0, checked, s);
+                    if (xp && x64) launch_explicit_true_residual(over_matrix(P.d), X, 0, checked, s);
                     else launch_pcg_true_residual(P, checked, s);
                     ps = read(checked);
                     if (std::isfinite(ps.true_norm) && ps.true_norm <= ps.target) break;
@@ -1204,7 +1206,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                         // the next iteration (ps.iter) starts fresh from d = 0
                         DevProblem Pr = P;
                         if (xp) Pr.d = dbuf[ps.iter & 1];
-                        if (xplicit) launch_explicit_true_residual(Pr, X, 1, restarted, s);
+                        if (xp && x64) launch_explicit_true_residual(over_matrix(Pr.d), X, 1, restarted, s);
                         else launch_pcg_restart(Pr, restarted, s);
                         ps = read(restarted);
                         if (ps.stop) {
