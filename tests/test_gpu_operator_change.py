@@ -82,3 +82,27 @@ def test_capped_iterates_keep_their_operator(device, precision, cameras, landmar
     poses, lms, accepted = one_iteration_at_a_time(device, problem, o)
     assert out.accepted == accepted
     assert np.array_equal(out.poses, poses) and np.array_equal(out.landmarks, lms)
+
+
+def test_a_solve_does_not_depend_on_those_before_it(device):
+    """Short solves, whose few iterations left do not pay for the matrix, then
+    a long one on the same handle: as on a handle of its own. One of the short
+    ones passes the cost of the lists and fails that of the blocks."""
+    problem = scene(300, 60000, 41)
+    o = workloads.loop_options(abi.PRECISION_MIXED, abi.PCG_MAXIT_REJECT, max_iterations=15)
+    handle = device.prepare(problem, o)
+    want = handle.solve(o)
+    state = handle.state()
+    handle.free()
+    for iterations in range(2, 9):
+        handle = device.prepare(problem, o)
+        short = abi.Options.from_buffer_copy(o)
+        short.max_iterations = iterations
+        assert handle.solve(short).status == abi.OK
+        device.profile(True)
+        got = handle.solve(o)
+        device.profile(False, reset=False)
+        assert device.profile_query("explicit_apply")["launches"] > 0
+        assert got.iterations == want.iterations
+        assert all(np.array_equal(a, b) for a, b in zip(handle.state(), state))
+        handle.free()

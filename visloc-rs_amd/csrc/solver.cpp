@@ -215,62 +215,59 @@ void build_explicit_host(Prepared& pr, hipStream_t s) {
     pr.x_num_full = (int32_t)nfull;
 }
 
-// The explicit matrix's structure, on the device where its limits allow.
-// With max_full >= 0 (the matrix-free solver asking) a structure of more full
-// blocks, or one the device does not build, is not built: false.
-bool build_explicit(Prepared& pr, const DevProblem& P, int64_t max_full, hipStream_t s) {
-    if (pr.explicit_built) return max_full < 0 || pr.x_num_full <= max_full;
+// The row kernels: the matrix's sizes into pr (they follow from the problem
+// alone and are kept), its row arrays into `B`, for the lists.
+void explicit_rows(Prepared& pr, const DevProblem& P, ExplicitBuild* B, hipStream_t s) {
     const size_t NP = (size_t)P.num_pose_slots, NE = (size_t)P.num_edges;
-    const int64_t terms = count_terms(pr);
-    if (terms > (int64_t)INT32_MAX / 3) {
-        if (max_full >= 0) return false;
-        throw Fail{VBA_ERR_INVALID_ARGUMENT, "Schur term lists too large"};
-    }
-    if (NP > (size_t)kExplicitMaxPoses || NE == 0) {
-        if (max_full >= 0) return false;
-        build_explicit_host(pr, s);
-        pr.explicit_built = true;
-        return true;
-    }
-    ExplicitBuild B{};
-    B.nw = (int32_t)((NP + 31) / 32);
-    B.bits = (uint32_t*)ensure(pr, B_X_BITS, (size_t)B.nw * NP * sizeof(uint32_t));
+    B->nw = (int32_t)((NP + 31) / 32);
+    B->bits = (uint32_t*)ensure(pr, B_X_BITS, (size_t)B->nw * NP * sizeof(uint32_t));
     int32_t* w = (int32_t*)ensure(pr, B_X_SCRATCH, (NE + 5 * NP + 2) * sizeof(int32_t));
-    B.lpose = w;
-    B.row_count = w + NE;
-    B.up_count = B.row_count + NP;
-    B.row_terms = B.up_count + NP;
-    B.up_ptr = B.row_terms + NP;
-    B.term_row = B.up_ptr + NP + 1;
-    B.row_ptr = (int32_t*)ensure(pr, B_X_ROW_PTR, (NP + 1) * sizeof(int32_t));
-    launch_explicit_rows(P, B, s);
+    B->lpose = w;
+    B->row_count = w + NE;
+    B->up_count = B->row_count + NP;
+    B->row_terms = B->up_count + NP;
+    B->up_ptr = B->row_terms + NP;
+    B->term_row = B->up_ptr + NP + 1;
+    B->row_ptr = (int32_t*)ensure(pr, B_X_ROW_PTR, (NP + 1) * sizeof(int32_t));
+    launch_explicit_rows(P, *B, s);
     hip_check(hipGetLastError(), "kernel launch");
     std::vector<int32_t> up(NP);
     int32_t full = 0, blocks = 0;
-    hip_check(hipMemcpyAsync(up.data(), B.up_count, NP * sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
-    hip_check(hipMemcpyAsync(&full, B.row_ptr + NP, sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
-    hip_check(hipMemcpyAsync(&blocks, B.up_ptr + NP, sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
+    hip_check(hipMemcpyAsync(up.data(), B->up_count, NP * sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
+    hip_check(hipMemcpyAsync(&full, B->row_ptr + NP, sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
+    hip_check(hipMemcpyAsync(&blocks, B->up_ptr + NP, sizeof(int32_t), hipMemcpyDeviceToHost, s), "D2H");
     hip_check(hipStreamSynchronize(s), "sync");
-    const int32_t max_upper = *std::max_element(up.begin(), up.end());
-    if (max_full >= 0 && full > max_full) return false;
-    if (max_upper > kExplicitMaxUpper) {
-        if (max_full >= 0) return false;
-        build_explicit_host(pr, s);
-        pr.explicit_built = true;
-        return true;
-    }
-    B.col = (int32_t*)ensure(pr, B_X_COL, (size_t)full * sizeof(int32_t));
-    B.diag_pos = (int32_t*)ensure(pr, B_X_DIAG_POS, NP * sizeof(int32_t));
-    B.block_pos = (int32_t*)ensure(pr, B_X_BLOCK_POS, 2 * (size_t)blocks * sizeof(int32_t));
-    B.block_pq = (int32_t*)ensure(pr, B_X_PQ, 2 * (size_t)blocks * sizeof(int32_t));
-    B.block_ptr = (int32_t*)ensure(pr, B_X_PTR, ((size_t)blocks + 1) * sizeof(int32_t));
-    B.terms = (int32_t*)ensure(pr, B_X_TERMS, 3 * (size_t)terms * sizeof(int32_t));
-    launch_explicit_lists(P, B, max_upper, s);
-    hip_check(hipGetLastError(), "kernel launch");
-    pr.x_num_blocks = blocks;
     pr.x_num_full = full;
+    pr.x_num_blocks = blocks;
+    pr.x_max_upper = *std::max_element(up.begin(), up.end());
+}
+
+// Whether the row kernels take the problem (a bitmap per pose).
+bool explicit_rows_on_device(const Model& m) { return m.num_pose_slots <= kExplicitMaxPoses && m.num_edges > 0; }
+
+// The explicit matrix's structure, on the device where its limits allow, from
+// B's row arrays if it has them.
+void build_explicit(Prepared& pr, const DevProblem& P, ExplicitBuild& B, hipStream_t s) {
+    if (pr.explicit_built) return;
+    const size_t NP = (size_t)P.num_pose_slots;
+    const int64_t terms = count_terms(pr);
+    if (terms > (int64_t)INT32_MAX / 3) throw Fail{VBA_ERR_INVALID_ARGUMENT, "Schur term lists too large"};
+    const bool rows = explicit_rows_on_device(pr.m);
+    if (rows && !B.bits) explicit_rows(pr, P, &B, s);
+    if (!rows || pr.x_max_upper > kExplicitMaxUpper) {
+        build_explicit_host(pr, s);
+    } else {
+        const size_t full = (size_t)pr.x_num_full, blocks = (size_t)pr.x_num_blocks;
+        B.col = (int32_t*)ensure(pr, B_X_COL, full * sizeof(int32_t));
+        B.diag_pos = (int32_t*)ensure(pr, B_X_DIAG_POS, NP * sizeof(int32_t));
+        B.block_pos = (int32_t*)ensure(pr, B_X_BLOCK_POS, 2 * blocks * sizeof(int32_t));
+        B.block_pq = (int32_t*)ensure(pr, B_X_PQ, 2 * blocks * sizeof(int32_t));
+        B.block_ptr = (int32_t*)ensure(pr, B_X_PTR, (blocks + 1) * sizeof(int32_t));
+        B.terms = (int32_t*)ensure(pr, B_X_TERMS, 3 * (size_t)terms * sizeof(int32_t));
+        launch_explicit_lists(P, B, pr.x_max_upper, s);
+        hip_check(hipGetLastError(), "kernel launch");
+    }
     pr.explicit_built = true;
-    return true;
 }
 
 // ---- profiling with HIP events on the context stream ----
@@ -813,9 +810,23 @@ namespace {
 // counts beside the layout).
 constexpr int64_t kExplicitTermBytes = 112, kExplicitBlockBytes = 32;
 
+// Whether the matrix-free solver may form the explicit matrix: by sizes alone.
+// Its lists and blocks have to stay within the bounds above, which long tracks
+// (more than some 9 terms an edge), scenes whose poses share landmarks with
+// most others, and many poses with few edges exceed; a structure that only the
+// host builds would take longer than it saves.
+bool explicit_fits(Prepared& pr, const DevProblem& P, ExplicitBuild* B, hipStream_t s) {
+    const int64_t edges = (int64_t)pr.m.num_edges, poses = (int64_t)pr.m.num_pose_slots, terms = count_terms(pr);
+    if (!explicit_rows_on_device(pr.m) || terms > (int64_t)INT32_MAX / 3 ||
+        12 * terms + 4 * edges + poses * (poses / 8 + 4) > kExplicitTermBytes * edges)
+        return false;
+    if (pr.x_num_full < 0) explicit_rows(pr, P, B, s);
+    return pr.x_max_upper <= kExplicitMaxUpper && 304 * (int64_t)pr.x_num_full <= kExplicitBlockBytes * edges;
+}
+
 // Whether the explicit reduced matrix is the faster operator for the rest of
-// a matrix-free solve, from the last PCG solve's iterations and the problem's
-// sizes alone (so that every solve of the problem decides alike).
+// a matrix-free solve, from its last PCG solve's iterations and the problem's
+// sizes alone, so that a solve does not depend on those before it.
 //
 // Measured on this card: a PCG iteration over the edges takes 13.6 us + 8.1 ps
 // an edge with FP32 G (16.4 us at 0.33M edges, 42 us at 3.5M), 15.6 us + 10.7
@@ -825,12 +836,9 @@ constexpr int64_t kExplicitTermBytes = 112, kExplicitBlockBytes = 32;
 // stand the assembly, 20 us + 17.5 ps a term for every LM iteration (55 us at
 // 2.3M terms, 492 us at 27.5M; in FP64 it replaces the edges' block-Jacobi
 // passes, 20 us + 30 ps an edge), and the structure, once: 1 ms + 75 ps a term
-// (3.1 ms at 27.5M). The lists' and blocks' memory has to stay within
-// the bounds above, which long tracks (more than some 9 terms an edge) and
-// scenes whose poses share landmarks with most others exceed.
+// (3.1 ms at 27.5M).
 bool explicit_pays(Prepared& pr, bool mixed, int32_t its, uint32_t remaining, const int32_t* num_full) {
     const double edges = (double)pr.m.num_edges, terms = (double)count_terms(pr);
-    if (12.0 * terms + 4.0 * edges > (double)kExplicitTermBytes * edges) return false;
     const double over_edges = mixed ? 13.6e-6 + 8.1e-12 * edges : 15.6e-6 + 10.7e-12 * edges;
     const double over_matrix = 8.2e-6 + (num_full ? 0.06e-9 * *num_full : 0.0);
     const double assembly = 20e-6 + 17.5e-12 * terms - (mixed ? 0.0 : 20e-6 + 30e-12 * edges);
@@ -895,12 +903,13 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         // The explicit matrix, when this solve uses it (xp): from the start
         // for the explicit solver, later for the matrix-free one (below).
         ExplicitDev X{};
+        ExplicitBuild xrows{};
         bool xp = false;
         const bool x32 = xplicit && mixed;           // FP32 copy for its products
         const bool x64 = xplicit || !mixed;          // it holds the FP64 operator
         double* dbuf[2] = {P.d, nullptr};            // PCG direction by iteration parity
-        auto use_explicit = [&](int64_t max_full) {
-            if (!build_explicit(pr, P, max_full, s)) return false;
+        auto use_explicit = [&]() {
+            build_explicit(pr, P, xrows, s);
             D.num_blocks = pr.x_num_blocks;
             D.block_pq = buf<int32_t>(pr, B_X_PQ);
             D.block_ptr = buf<int32_t>(pr, B_X_PTR);
@@ -915,9 +924,9 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             X.S32 = x32 ? (float*)ensure(pr, B_X_S32, 36 * (size_t)X.num_full * sizeof(float)) : nullptr;
             dbuf[1] = (double*)ensure(pr, B_VD2, 6 * NP * sizeof(double));
             hip_check(hipMemsetAsync(dbuf[1], 0, 6 * NP * sizeof(double), s), "memset");
-            return xp = true;
+            xp = true;
         };
-        if (xplicit) use_explicit(-1);
+        if (xplicit) use_explicit();
         // P as the matrix's kernels take it: their partials, and the direction `d`
         auto over_matrix = [&](double* d) {
             DevProblem Px = P;
@@ -1009,7 +1018,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         // ended up to 10 % of the landmarks away (1 of 48; most within 1e-6)
         // where one weak landmark decided whether a step was accepted. With
         // REJECT, 110 loops ended within 2.6e-8.
-        bool ask = matrix_free && !xplicit && !accept_iterate && !pr.x_refused;
+        bool ask = matrix_free && !xplicit && !accept_iterate;
         const int32_t max_pcg = (int32_t)o.max_pcg_iterations;
         auto push = [&](const vba_iteration_stats& st) {
             if (stats && written < cap) stats[written] = st;
@@ -1039,18 +1048,14 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             // edges; with the same operator 2.6e-8, the median 1.3e-13.)
             if (ask && !xp && last_its > 0 &&
                 explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, nullptr)) {
-                bool done = false;
                 try {
-                    done = use_explicit((int64_t)(kExplicitBlockBytes * NE / 304)) &&
-                           explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, &pr.x_num_full);
+                    if (!explicit_fits(pr, P, &xrows, s)) ask = false;
+                    else if (explicit_pays(pr, mixed, last_its, o.max_iterations - iteration, &pr.x_num_full))
+                        use_explicit();
                 } catch (const Fail& f) {
                     if (f.code != VBA_ERR_OUT_OF_MEMORY) throw;
-                    (void)hipGetLastError();  // no memory for it: stay with the edges
-                }
-                xp = done;
-                if (!done) {
+                    (void)hipGetLastError();  // no memory for it: this solve stays with the edges
                     ask = false;
-                    pr.x_refused = true;
                 }
             }
             launch_landmark_prepare(P, lambda, s);

@@ -78,8 +78,7 @@ struct Prepared {
     // explicit reduced camera matrix (over the dense term lists): full block
     // rows, the full positions of each upper block and of each diagonal
     bool explicit_built = false;
-    bool x_refused = false;  // the matrix-free solver does not take it for this problem
-    int32_t x_num_blocks = 0, x_num_full = 0;
+    int32_t x_num_blocks = 0, x_num_full = -1, x_max_upper = 0;  // (-1: not known yet)
     int64_t x_terms = -1;  // terms of its lists, fixed poses' included (-1: not counted)
     int final_slot = -1;  // buffer holding the final poses (-1: none yet)
     int final_lm_slot = -1;
