@@ -1,0 +1,88 @@
+"""The explicit reduced matrix's structure beyond the device build's limits, and
+the memory it keeps."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import vba
+from vba import abi
+
+pytestmark = pytest.mark.gpu
+
+
+def scene(cameras, landmarks, seed=4):
+    return vba.synthesize(abi.SYNTH_LOOP, num_cameras=cameras, num_landmarks=landmarks, seed=seed,
+                          scene_scale=200.0 * cameras / 1200.0).problem
+
+
+def options(solver, **kw):
+    o = dict(linear_solver=solver, max_iterations=8, max_pcg_iterations=500, pcg_relative_tolerance=1e-8,
+             initial_lambda=1.0, robust_kernel=abi.KERNEL_HUBER, robust_scale=1.0)
+    o.update(kw)
+    return vba.default_options(**o)
+
+
+def free_bytes(device):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert device.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def matrix_sizes(problem):
+    """(terms, stored blocks) of the reduced matrix, all poses but the fixed ones."""
+    slot = {int(i): k for k, i in enumerate(problem.pose_ids)}
+    pose = np.array([slot[int(i)] for i in problem.obs_pose_ids])
+    keep = problem.pose_fixed[pose] == 0
+    order = np.lexsort((pose[keep], problem.obs_landmark_ids[keep]))
+    pose, lm = pose[keep][order], problem.obs_landmark_ids[keep][order]
+    n = len(problem.pose_ids)
+    pairs, terms, d = [], 0, 0
+    while True:  # pairs of a landmark's observations d places apart
+        same = lm[d:] == lm[:len(lm) - d]
+        if not same.any():
+            break
+        terms += int(same.sum())
+        pairs.append(np.unique(pose[:len(pose) - d][same] * n + pose[d:][same]))
+        d += 1
+    upper = np.unique(np.concatenate(pairs))
+    return terms, 2 * len(upper) - int((upper // n == upper % n).sum())
+
+
+def test_the_lists_scratch_is_given_back(device):
+    """What the explicit solver adds to a handle is its lists and blocks, not
+    the row bitmaps (32 MB at 16,000 poses) that the lists were built from."""
+    problem = scene(16000, 24000)
+    handle = device.prepare(problem, options(abi.SOLVER_MATRIX_FREE))
+    assert handle.solve(options(abi.SOLVER_MATRIX_FREE, max_iterations=1)).status == abi.OK
+    before = free_bytes(device)
+    assert handle.solve(options(abi.SOLVER_PCG_EXPLICIT, max_iterations=1)).status == abi.OK
+    used = before - free_bytes(device)
+    handle.free()
+    terms, blocks = matrix_sizes(problem)
+    lists = 12 * terms + blocks * (4 + 288) + (blocks + 16000) / 2 * 20 + 16000 * 60
+    assert used <= 1.02 * lists + (12 << 20)  # (allocations' granularity)
+
+
+def test_structure_built_on_the_host(device):
+    """More poses than the device build takes: the explicit solver's lists come
+    from the host, and its steps are those of the product over the edges. A
+    matrix-free solve does not take such a structure over."""
+    problem = scene(16400, 12000)
+    free, explicit = options(abi.SOLVER_MATRIX_FREE), options(abi.SOLVER_PCG_EXPLICIT)
+    handle = device.prepare(problem, free)
+    a = handle.solve(free)
+    poses, landmarks = handle.state()
+    b = handle.solve(explicit)
+    p, l = handle.state()
+    assert a.status == b.status == abi.OK and a.accepted == b.accepted and any(a.accepted)
+    # both solve each system to 1e-8 at a damping of 1 and more
+    assert np.linalg.norm(p - poses) <= 1e-7 * np.linalg.norm(poses)
+    assert np.linalg.norm(l - landmarks) <= 1e-7 * np.linalg.norm(landmarks)
+    assert b.result.total_pcg_iterations > 0
+    device.profile(True)
+    again = handle.solve(free)
+    device.profile(False, reset=False)
+    assert device.profile_query("explicit_apply")["launches"] == 0
+    assert again.iterations == a.iterations
+    handle.free()

@@ -215,6 +215,21 @@ void build_explicit_host(Prepared& pr, hipStream_t s) {
     pr.x_num_full = (int32_t)nfull;
 }
 
+// The explicit matrix's buffers; the first two only serve to build its lists.
+constexpr BufId kExplicitBufs[] = {B_X_BITS, B_X_SCRATCH, B_X_ROW_PTR, B_X_COL, B_X_DIAG_POS, B_X_BLOCK_POS, B_X_PQ,
+                                   B_X_PTR, B_X_TERMS, B_X_S64, B_X_S32, B_VD2};
+
+// Gives back the first `count` of them. The stream has to be idle.
+void drop_explicit(Prepared& pr, size_t count) {
+    for (size_t i = 0; i < count && !pr.bufs.empty(); ++i) {
+        DevBuffer& b = pr.bufs[kExplicitBufs[i]];
+        if (!b.ptr) continue;
+        (void)hipFree(b.ptr);
+        b = DevBuffer{};
+        ++pr.alloc_gen;
+    }
+}
+
 // The row kernels: the matrix's sizes into pr (they follow from the problem
 // alone and are kept), its row arrays into `B`, for the lists.
 void explicit_rows(Prepared& pr, const DevProblem& P, ExplicitBuild* B, hipStream_t s) {
@@ -1054,7 +1069,12 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
                         use_explicit();
                 } catch (const Fail& f) {
                     if (f.code != VBA_ERR_OUT_OF_MEMORY) throw;
-                    (void)hipGetLastError();  // no memory for it: this solve stays with the edges
+                    // no memory for it: this solve stays with the edges, and
+                    // what it got is given back
+                    (void)hipGetLastError();
+                    hip_check(hipStreamSynchronize(s), "sync");
+                    drop_explicit(pr, std::size(kExplicitBufs));
+                    pr.explicit_built = false;
                     ask = false;
                 }
             }
@@ -1308,6 +1328,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         }
         hip_check(hipEventRecord(ctx.ev_stop, s), "event");
         hip_check(hipStreamSynchronize(s), "sync");
+        drop_explicit(pr, 2);
         harvest(ctx);
         float ms = 0.f;
         hip_check(hipEventElapsedTime(&ms, ctx.ev_start, ctx.ev_stop), "event");
@@ -1330,6 +1351,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
     } catch (const Fail& f) {
         ctx.last_error = f.msg;
         (void)hipStreamSynchronize(s);
+        drop_explicit(pr, 2);
         for (const Context::Pending& p : ctx.pending) {
             ctx.event_pool.push_back(p.a);
             ctx.event_pool.push_back(p.b);
