@@ -86,3 +86,30 @@ def test_structure_built_on_the_host(device):
     assert device.profile_query("explicit_apply")["launches"] == 0
     assert again.iterations == a.iterations
     handle.free()
+
+
+def test_fixed_poses_do_not_count_against_the_lists(device):
+    """Six landmarks seen by 16,000 fixed poses and 4 variable ones: 768M pairs
+    of observations, more than the lists can hold, but 60 terms, as fixed poses
+    have no part in the matrix."""
+    rng = np.random.default_rng(7)
+    n = 16004
+    centres = np.stack([rng.uniform(-1, 1, n), rng.uniform(-1, 1, n), np.zeros(n)], 1)
+    points = np.stack([rng.uniform(-1, 1, 6), rng.uniform(-1, 1, 6), rng.uniform(5, 7, 6)], 1)
+    rel = points[None] - centres[:, None]
+    xy = 500.0 * rel[..., :2] / rel[..., 2:] + np.array([320.0, 240.0]) + rng.normal(0, 0.3, (n, 6, 2))
+    poses = np.concatenate([np.tile([1.0, 0, 0, 0], (n, 1)), -centres], 1)
+    poses[-4:, 4:] += 0.05
+    fixed = np.ones(n, np.uint8)
+    fixed[-4:] = 0
+    problem = vba.BundleProblem(
+        camera=vba.camera(abi.CAMERA_PINHOLE, [500.0, 500.0, 320.0, 240.0], 640, 480),
+        pose_ids=np.arange(n), poses=poses, pose_fixed=fixed, landmark_ids=np.arange(6), landmarks=points + 0.02,
+        landmark_fixed=np.zeros(6, np.uint8), obs_pose_ids=np.repeat(np.arange(n), 6),
+        obs_landmark_ids=np.tile(np.arange(6), n), obs_xy=xy.reshape(-1, 2))
+    a = device.optimize(problem, options(abi.SOLVER_PCG_EXPLICIT, initial_lambda=1e-3, max_iterations=3))
+    assert a.status == abi.OK, a.message
+    b = device.optimize(problem, options(abi.SOLVER_DENSE, initial_lambda=1e-3, max_iterations=3))
+    assert a.accepted == b.accepted and any(a.accepted)
+    assert abs(a.result.final_cost - b.result.final_cost) <= 1e-9 * b.result.final_cost
+    assert np.abs(a.poses - b.poses).max() <= 1e-7

@@ -155,16 +155,22 @@ void build_dense(Prepared& pr) {
     pr.dense_built = true;
 }
 
+constexpr int64_t kMaxTerms = INT32_MAX / 3;
+
 // Terms of the reduced camera matrix's blocks: every pair of a variable
-// landmark's edges once (fixed poses' pairs too, an upper bound).
+// landmark's edges once. Fixed poses' pairs count too, so that the edges need
+// not be walked, unless the limit is passed only with them.
 int64_t count_terms(Prepared& pr) {
-    if (pr.x_terms < 0) {
+    const Model& m = pr.m;
+    for (int exact = 0; pr.x_terms < 0; ++exact) {
         int64_t t = 0;
-        for (uint32_t l = 0; l < pr.m.num_lm_slots; ++l) {
-            const int64_t n = pr.m.lm_edge_ptr[l + 1] - pr.m.lm_edge_ptr[l];
-            if (pr.m.lm_var[l] >= 0) t += n * (n + 1) / 2;
+        for (uint32_t l = 0; l < m.num_lm_slots; ++l) {
+            int64_t n = m.lm_var[l] >= 0 ? m.lm_edge_ptr[l + 1] - m.lm_edge_ptr[l] : 0;
+            for (int32_t e = m.lm_edge_ptr[l]; exact && n > 0 && e < m.lm_edge_ptr[l + 1]; ++e)
+                n -= m.pose_var[m.l_pose[e]] < 0;
+            t += n * (n + 1) / 2;
         }
-        pr.x_terms = t;
+        if (exact || t <= kMaxTerms) pr.x_terms = t;
     }
     return pr.x_terms;
 }
@@ -266,7 +272,7 @@ void build_explicit(Prepared& pr, const DevProblem& P, ExplicitBuild& B, hipStre
     if (pr.explicit_built) return;
     const size_t NP = (size_t)P.num_pose_slots;
     const int64_t terms = count_terms(pr);
-    if (terms > (int64_t)INT32_MAX / 3) throw Fail{VBA_ERR_INVALID_ARGUMENT, "Schur term lists too large"};
+    if (terms > kMaxTerms) throw Fail{VBA_ERR_INVALID_ARGUMENT, "Schur term lists too large"};
     const bool rows = explicit_rows_on_device(pr.m);
     if (rows && !B.bits) explicit_rows(pr, P, &B, s);
     if (!rows || pr.x_max_upper > kExplicitMaxUpper) {
@@ -832,7 +838,7 @@ constexpr int64_t kExplicitTermBytes = 112, kExplicitBlockBytes = 32;
 // host builds would take longer than it saves.
 bool explicit_fits(Prepared& pr, const DevProblem& P, ExplicitBuild* B, hipStream_t s) {
     const int64_t edges = (int64_t)pr.m.num_edges, poses = (int64_t)pr.m.num_pose_slots, terms = count_terms(pr);
-    if (!explicit_rows_on_device(pr.m) || terms > (int64_t)INT32_MAX / 3 ||
+    if (!explicit_rows_on_device(pr.m) || terms > kMaxTerms ||
         12 * terms + 4 * edges + poses * (poses / 8 + 4) > kExplicitTermBytes * edges)
         return false;
     if (pr.x_num_full < 0) explicit_rows(pr, P, B, s);

@@ -79,7 +79,7 @@ struct Prepared {
     // rows, the full positions of each upper block and of each diagonal
     bool explicit_built = false;
     int32_t x_num_blocks = 0, x_num_full = -1, x_max_upper = 0;  // (-1: not known yet)
-    int64_t x_terms = -1;  // terms of its lists, fixed poses' included (-1: not counted)
+    int64_t x_terms = -1;  // terms of its lists, or a bound on them (-1: not counted)
     int final_slot = -1;  // buffer holding the final poses (-1: none yet)
     int final_lm_slot = -1;
     int32_t last_pcg = 0;  // iterations of the last PCG solve (the schedule's prediction)
