@@ -148,3 +148,29 @@ def test_admission_keeps_batches_within_the_hbm_budget(device):
             assert got.status == abi.OK
             assert got.result.final_cost == alone.result.final_cost
             assert np.array_equal(got.poses, alone.poses)
+
+
+def test_request_bytes_charge_the_reduced_matrix_where_it_may_be_formed(device):
+    """144 bytes an observation (an edge each here) more for a matrix-free
+    solve that refuses the iterate at its cap, of at most 16,384 poses; nothing
+    for any other request, however many poses it has."""
+    s = vba.synthesize(abi.SYNTH_LOOP, num_cameras=300, num_landmarks=4000, seed=3, scene_scale=50.0).problem
+    many = s.copy()
+    n = 200000
+    many.pose_ids = np.arange(n, dtype=np.uint64) + 1000000
+    many.poses = np.tile([1.0, 0, 0, 0, 0, 0, 0], (n, 1))
+    many.pose_fixed = np.zeros(n, np.uint8)
+
+    def layout(p):  # structure and working buffers
+        return 236 * p.num_observations + 260 * len(p.landmark_ids) + 1400 * len(p.pose_ids) + 65536
+
+    with vba.Server(window_streams=1, submap_streams=1) as srv:
+        for p in (s, many):
+            for solver in (abi.SOLVER_MATRIX_FREE, abi.SOLVER_PCG_EXPLICIT, abi.SOLVER_SPARSE, abi.SOLVER_DENSE):
+                for policy in (abi.PCG_MAXIT_ACCEPT_ITERATE, abi.PCG_MAXIT_REJECT):
+                    o = vba.default_options(linear_solver=solver, pcg_maxit_policy=policy)
+                    more = srv.request_bytes(p, o) - layout(p)
+                    if p is s and solver == abi.SOLVER_MATRIX_FREE and policy == abi.PCG_MAXIT_REJECT:
+                        assert 144 * p.num_observations <= more <= 144 * p.num_observations + 64 * len(p.pose_ids)
+                    else:
+                        assert more == 0, (len(p.pose_ids), solver, policy, more)

@@ -32,6 +32,7 @@
 #include "../../include/vba.h"
 #include "capi_types.hpp"
 #include "host_common.hpp"
+#include "kernels.hpp"
 #include "problem.hpp"
 #include "solver.hpp"
 
@@ -128,13 +129,15 @@ struct Request {
 
 // Device bytes a request holds while it runs (structure, working buffers
 // and, for a window, its dense system), an upper estimate.
-uint64_t estimate_bytes(const vba_problem& p, bool window) {
+uint64_t estimate_bytes(const vba_problem& p, const vba_options& o, bool window) {
     const uint64_t n = vba::observation_count(p);
     const uint64_t L = p.num_landmarks, P = p.num_poses;
     uint64_t b = n * 40 + n * 196 + L * 260 + P * 1400 + (64u << 10);
-    // the explicit reduced matrix a matrix-free solve may form: its lists and
-    // blocks within 144 bytes an edge, row bitmaps and row arrays
-    if (!window) b += n * 144 + P * (P / 8 + 64);
+    // the explicit reduced matrix, where a solve may change to it: within 144
+    // bytes an edge, and row arrays
+    if (o.linear_solver == VBA_SOLVER_MATRIX_FREE && o.pcg_maxit_policy == VBA_PCG_MAXIT_REJECT &&
+        P <= (uint64_t)vba::kExplicitMaxPoses)
+        b += n * 144 + P * 64;
     if (window) {
         uint64_t var = 0;
         for (uint64_t i = 0; i < P; ++i) var += p.pose_fixed ? (p.pose_fixed[i] == 0) : 1;
@@ -382,7 +385,7 @@ uint64_t submit(vba_server* s, const vba_problem* problem, const vba_options* op
         vba::set_thread_error("vba_server_submit: no lane serves this request");
         return 0;
     }
-    r->est_bytes = estimate_bytes(*problem, r->window_lane);
+    r->est_bytes = estimate_bytes(*problem, *options, r->window_lane);
     {
         std::lock_guard<std::mutex> lock(s->mu);
         if (s->stopping) {
@@ -436,7 +439,7 @@ int32_t vba_server_wait(vba_server* s, uint64_t ticket, double timeout_seconds, 
 
 uint64_t vba_server_request_bytes(const vba_server* s, const vba_problem* problem, const vba_options* options) {
     if (!s || !problem || !options) return 0;
-    return estimate_bytes(*problem, window_lane(*s, *problem, *options));
+    return estimate_bytes(*problem, *options, window_lane(*s, *problem, *options));
 }
 
 void vba_server_counters(vba_server* s, uint64_t* completed, uint64_t* batches, uint64_t* batched_windows,
