@@ -946,7 +946,12 @@ __device__ void dense_solve_small(const DenseRows& io, double* S, double* work, 
 #pragma unroll
             for (int j = 0; j < 16; ++j) a[j] = lane == 63 ? sh.b[16 * k + j] : below || lane < 16 ? panel[row * 17 + j] : 0.0;
             double ri;
-            if (!chol16_rows(a, lane, &ri)) {
+            const bool ok = chol16_rows(a, lane, &ri);
+            // lane 63's results, read while it is active
+            double yk[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) yk[j] = lane_value(a[j], 63);
+            if (!ok) {
                 if (lane == 0) sh.fail = 1;
             } else {
                 if (mine) {
@@ -954,7 +959,7 @@ __device__ void dense_solve_small(const DenseRows& io, double* S, double* work, 
 #pragma unroll
                     for (int j = 0; j < 16; ++j) panel[row * 17 + j] = a[j];
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) bb = fma(-a[j], lane_value(a[j], 63), bb);
+                    for (int j = 0; j < 16; ++j) bb = fma(-a[j], yk[j], bb);
                     sh.b[row] = bb;
                 }
                 if (wave == 0) {
