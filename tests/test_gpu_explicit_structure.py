@@ -113,3 +113,18 @@ def test_fixed_poses_do_not_count_against_the_lists(device):
     assert a.accepted == b.accepted and any(a.accepted)
     assert abs(a.result.final_cost - b.result.final_cost) <= 1e-9 * b.result.final_cost
     assert np.abs(a.poses - b.poses).max() <= 1e-7
+
+
+@pytest.mark.parametrize("cameras,landmarks", [(40, 12000), (300, 40000)])
+def test_two_builds_give_the_same_bits(device, cameras, landmarks):
+    """The term lists' order, and so every sum's, is that of the edges: a
+    structure built again, on a new handle, gives the same solve (a block's
+    terms are some 200 neighbouring edges of its row here, so most of a wave's
+    lanes add to the same lists)."""
+    problem = scene(cameras, landmarks)
+    o = options(abi.SOLVER_PCG_EXPLICIT, initial_lambda=1e-3, max_iterations=4)
+    outs = [device.optimize(problem, o) for _ in range(4)]
+    assert outs[0].status == abi.OK and any(outs[0].accepted)
+    for out in outs[1:]:
+        assert out.iterations == outs[0].iterations
+        assert np.array_equal(out.poses, outs[0].poses) and np.array_equal(out.landmarks, outs[0].landmarks)

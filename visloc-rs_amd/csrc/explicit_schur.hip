@@ -27,9 +27,8 @@ namespace {
 // the number of set bits before it, and the upper blocks are numbered row by
 // row. The term lists come from each row's wave walking the row's edges 64 at
 // a time (a lane per edge, its landmark's later poses one by one) and taking
-// the next place of the block's list from a counter in LDS: the counters of
-// one wave's instruction are served in lane order, so the lists have a fixed
-// order. Once per prepared problem; the 26M terms of the 1,200-camera loop
+// the next places of the blocks' lists from counters in LDS, the lanes of one
+// list in lane order, so the lists have a fixed order. Once per prepared problem; the 26M terms of the 1,200-camera loop
 // take 1.7 ms here (first solve 38 ms), against lists built on the host and
 // sent (first solve 251 ms).
 // ---------------------------------------------------------------------------
@@ -245,10 +244,21 @@ __global__ __launch_bounds__(64) void k_explicit_fill(DevProblem P, ExplicitBuil
         int i = on ? P.lm_edge_ptr[l] : 0;
         while (i < le && B.lpose[i] < p) ++i;  // this edge's own place in its landmark
         for (; __any(i < le); ++i) {
-            if (i >= le) continue;
-            const int q = B.lpose[i];
-            if (P.pose_var[q] < 0) continue;
-            const int t = atomicAdd(&r.count[r.upper_of(q)], 1);
+            const int q = i < le ? B.lpose[i] : p;
+            const bool term = i < le && P.pose_var[q] >= 0;
+            const int j = term ? r.upper_of(q) : 0;
+            // the lanes whose terms go to this lane's list, by the bits of j
+            uint64_t same = __ballot(term);
+            for (int bit = 1; bit < upper; bit <<= 1) {
+                const uint64_t set = __ballot((j & bit) != 0);
+                same &= j & bit ? set : ~set;
+            }
+            const int rank = __popcll(same & ((1ull << lane) - 1)), first = r.count[j];
+            __builtin_amdgcn_wave_barrier();
+            if (term && rank == 0) r.count[j] = first + __popcll(same);
+            __builtin_amdgcn_wave_barrier();
+            if (!term) continue;
+            const int t = first + rank;
             B.terms[3 * (size_t)t] = l;
             B.terms[3 * (size_t)t + 1] = ep;
             B.terms[3 * (size_t)t + 2] = P.lm_store[i];
