@@ -664,10 +664,6 @@ int32_t vba_reduced_solve(vba_context* ctx, const vba_reduced_system* system, do
  * vba_reduced_solve of the same structure with offdiag == NULL.
  * VBA_OK, or VBA_DECLINED (`None`: the caller eliminates on the CPU) for
  * inconsistent input; vba_last_error(ctx) says why. */
-/* Bit of vba_point_elimination.reserved: hcp, point_inverse, extra_blocks and
- * the outputs run_blocks and coarse_sums are row-major (column-major, as
- * nalgebra stores them, without it). */
-#define VBA_ELIMINATION_ROW_MAJOR 1u
 typedef struct vba_point_elimination {
     uint64_t structure_id;
     uint64_t linearization_id;
@@ -691,11 +687,15 @@ typedef struct vba_point_elimination {
     uint32_t coarse_group;
     const uint32_t* run_edges;
     uint32_t coarse_nodes;
-    uint32_t reserved; /* 0, or VBA_ELIMINATION_ROW_MAJOR */
+    uint32_t reserved;
 } vba_point_elimination;
 
 int32_t vba_reduced_eliminate(vba_context* ctx, const vba_point_elimination* elimination, double* run_blocks,
                               double* coarse_sums);
+/* The same with hcp, point_inverse, extra_blocks and the outputs run_blocks and
+ * coarse_sums row-major, for callers that hold their blocks so. */
+int32_t vba_reduced_eliminate_row_major(vba_context* ctx, const vba_point_elimination* elimination,
+                                        double* run_blocks, double* coarse_sums);
 
 #ifdef __cplusplus
 } /* extern "C" */

@@ -787,8 +787,8 @@ int32_t reduced_solve(Context& ctx, const vba_reduced_system& sys, double* step,
     }
 }
 
-int32_t reduced_eliminate(Context& ctx, const vba_point_elimination& el, double* run_blocks, double* coarse_sums,
-                          std::string* msg) {
+int32_t reduced_eliminate(Context& ctx, const vba_point_elimination& el, bool row_major, double* run_blocks,
+                          double* coarse_sums, std::string* msg) {
     const uint32_t n = el.num_nodes, E = el.num_edges, NP = el.num_points;
     if (n == 0 || n > (1u << 24) || E >= (1u << 31) || el.structure_id == 0)
         return decline(msg, "point elimination: no nodes, too large, or structure_id 0");
@@ -823,7 +823,7 @@ int32_t reduced_eliminate(Context& ctx, const vba_point_elimination& el, double*
         D.coarse_group = (int32_t)el.coarse_group;
         D.coarse_nodes = (int32_t)el.coarse_nodes;
         D.coarse_m = m;
-        D.row_major = (int32_t)(el.reserved & VBA_ELIMINATION_ROW_MAJOR);
+        D.row_major = row_major;
         if (el.structure_id != R.elim_structure || R.structure_id != el.structure_id || R.n != (int32_t)n ||
             R.num_edges != (int32_t)E) {
             // validate the structure and build the pair index

@@ -71,7 +71,6 @@ pub const VBA_GNC_GEMAN_MCCLURE: u32 = 0;
 pub const VBA_GNC_TRUNCATED_LEAST_SQUARES: u32 = 1;
 
 pub const VBA_DENSE_NOALLOC_MAX_N: u32 = 1024;
-pub const VBA_ELIMINATION_ROW_MAJOR: u32 = 1;
 
 #[repr(C)]
 #[derive(Clone, Copy, Debug)]
@@ -377,6 +376,8 @@ extern "C" {
                              iterations: *mut u32) -> i32;
     pub fn vba_reduced_eliminate(ctx: *mut vba_context, elimination: *const vba_point_elimination,
                                  run_blocks: *mut f64, coarse_sums: *mut f64) -> i32;
+    pub fn vba_reduced_eliminate_row_major(ctx: *mut vba_context, elimination: *const vba_point_elimination,
+                                           run_blocks: *mut f64, coarse_sums: *mut f64) -> i32;
 }
 
 // ---- include/vba_io.h -----------------------------------------------------

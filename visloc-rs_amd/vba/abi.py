@@ -240,8 +240,6 @@ class ServerConfig(C.Structure):
     ]
 
 
-ELIMINATION_ROW_MAJOR = 1  # vba_point_elimination.reserved
-
 GNC_GEMAN_MCCLURE = 0
 GNC_TRUNCATED_LEAST_SQUARES = 1
 
@@ -365,6 +363,7 @@ SIGNATURES = {
     "vba_dense_solve_noalloc": (C.c_int32, [C.c_void_p, C.c_uint32, P64, P64, P64]),
     "vba_reduced_solve": (C.c_int32, [C.c_void_p, C.POINTER(ReducedSystem), P64, C.POINTER(C.c_uint32)]),
     "vba_reduced_eliminate": (C.c_int32, [C.c_void_p, C.POINTER(PointElimination), P64, P64]),
+    "vba_reduced_eliminate_row_major": (C.c_int32, [C.c_void_p, C.POINTER(PointElimination), P64, P64]),
     "vba_optimize_weighted": (
         C.c_int32,
         [C.c_void_p, C.POINTER(Problem), C.POINTER(Options), P64, C.c_uint64, P64, P64,

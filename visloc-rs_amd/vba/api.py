@@ -333,7 +333,7 @@ class PointEliminationInput:
     def view(self, row_major: bool = False):
         """(abi.PointElimination, arrays to keep alive while it is used):
         column-major copies of the blocks, or with row_major the blocks as
-        they are (abi.ELIMINATION_ROW_MAJOR)."""
+        they are (for vba_reduced_eliminate_row_major)."""
         def blocks(m, r, c):
             m = np.asarray(m, np.float64).reshape(-1, r, c)
             return np.ascontiguousarray(m if row_major else np.swapaxes(m, -1, -2))
@@ -361,7 +361,6 @@ class PointEliminationInput:
         v.num_points = len(arrs["point_off"]) - 1
         v.num_extra = len(arrs["extra_edge"])
         v.num_run_edges = len(arrs["run_edges"])
-        v.reserved = abi.ELIMINATION_ROW_MAJOR if row_major else 0
         if self.coarse is not None:
             v.coarse_group, v.coarse_nodes = int(self.coarse[0]), int(self.coarse[1])
         ptr = {np.dtype(np.uint32): abi.PU32, np.dtype(np.uint64): abi.PU64, np.dtype(np.uint8): abi.PU8,
@@ -562,7 +561,7 @@ class Device:
         return step, int(its.value)
 
     def reduced_eliminate(self, elim: "PointEliminationInput"):
-        """vba_reduced_eliminate, `ReducedSolveAccelerator::eliminate`
+        """vba_reduced_eliminate_row_major, `ReducedSolveAccelerator::eliminate`
         (pipelines/slam/src/ba_accel.rs:150-156): returns (run_blocks
         (len(run_edges), 6, 6), coarse_sums (m, m, 6, 6) or None), row-major
         6x6 here, or None where the trait returns None. The blocks stay on
@@ -572,13 +571,13 @@ class Device:
         runs = np.empty((max(1, len(elim.run_edges)), 36))
         m = elim.coarse_aggregates()
         coarse = np.empty((max(1, m * m), 36))
-        st = self.lib.vba_reduced_eliminate(self.ctx, C.byref(view), runs.ctypes.data_as(abi.P64),
-                                            coarse.ctypes.data_as(abi.P64))
+        st = self.lib.vba_reduced_eliminate_row_major(self.ctx, C.byref(view), runs.ctypes.data_as(abi.P64),
+                                                      coarse.ctypes.data_as(abi.P64))
         del keep
         if st == abi.DECLINED:
             return None
         if st != abi.OK:
-            raise RuntimeError(f"vba_reduced_eliminate: {st} {self.last_error()}")
+            raise RuntimeError(f"vba_reduced_eliminate_row_major: {st} {self.last_error()}")
         rb = runs[:len(elim.run_edges)].reshape(-1, 6, 6)
         cs = coarse[:m * m].reshape(m, m, 6, 6) if m else None
         return rb, cs
