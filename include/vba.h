@@ -278,7 +278,8 @@ typedef struct vba_context vba_context;
 /* ---- lifecycle (the reference's *_abi_version/_create/_destroy/_last_error) */
 uint32_t vba_abi_version(void);
 /* Create a context on a HIP device ordinal. NULL on failure (see
- * vba_last_error(NULL)). */
+ * vba_last_error(NULL)). A solve polls for the device's results: its calling
+ * thread keeps a core busy while it waits. */
 struct vba_context* vba_create(int32_t device);
 void vba_destroy(struct vba_context* ctx);
 /* Last error message of ctx, or of the calling thread when ctx is NULL. */
@@ -455,7 +456,7 @@ void vba_prepared_batch_free(vba_context* ctx, vba_prepared_batch* batch);
  * (matrix-free, large dense) are solved one per submap stream. Admission
  * keeps the estimated device footprint of running work within
  * hbm_budget_bytes. A result equals the one vba_optimize gives the request
- * alone. */
+ * alone. Each lane that is solving keeps a host core busy. */
 typedef struct vba_server_config {
     int32_t device;
     uint32_t max_window_batch;    /* windows per device batch */
