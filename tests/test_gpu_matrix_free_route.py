@@ -51,8 +51,8 @@ def solve_on_both_operators(device, problem, o):
     return out, state
 
 
-def compare(device, problem, extent, o):
-    out, (poses, _) = solve_on_both_operators(device, problem, o)
+def compare(device, problem, extent, o, solve=solve_on_both_operators):
+    out, (poses, _) = solve(device, problem, o)
     ro = vba.default_options()
     for f, _ in abi.Options._fields_:
         setattr(ro, f, getattr(o, f))
@@ -98,18 +98,36 @@ def test_lenses_per_camera(device):
     compare(device, s.problem, s.scene_extent, o)
 
 
-def test_long_tracks_stay_on_the_edges(device):
-    """Every landmark in every camera: more terms an edge than the lists may
-    take, so the product stays on the edges."""
-    s = vba.synthesize(abi.SYNTH_CIRCLE, num_cameras=40, num_landmarks=2000, seed=2)
-    o = options(abi.PRECISION_FP64, robust_kernel=abi.KERNEL_NONE)
-    pp = device.prepare(s.problem, o)
+def solve_on_the_edges(device, problem, o):
+    pp = device.prepare(problem, o)
     device.profile(True)
     out = pp.solve(o)
     device.profile(False, reset=False)
-    assert out.status == abi.OK and out.result.total_pcg_iterations > 0
+    assert out.status == abi.OK, out.message
+    assert device.profile_query("schur_apply")["launches"] > 0
     assert device.profile_query("explicit_apply")["launches"] == 0
+    state = pp.state()
     pp.free()
+    return out, state
+
+
+@pytest.mark.parametrize("precision", [abi.PRECISION_FP64, abi.PRECISION_MIXED])
+@pytest.mark.parametrize("policy", [abi.PCG_MAXIT_ACCEPT_ITERATE, abi.PCG_MAXIT_REJECT])
+def test_long_tracks_stay_on_the_edges(device, precision, policy):
+    """Every landmark in every camera: more terms an edge than the lists may
+    take, so the product stays on the edges. (A second fixed camera holds the
+    scale, along which the precisions would part.)"""
+    s = vba.synthesize(abi.SYNTH_CIRCLE, num_cameras=40, num_landmarks=2000, seed=2)
+    p = s.problem.copy()
+    p.pose_fixed[[0, 13]] = 1
+    o = options(precision, policy, iterations=12, robust_kernel=abi.KERNEL_HUBER)
+    compare(device, p, s.scene_extent, o, solve_on_the_edges)
+
+
+@pytest.mark.parametrize("precision", [abi.PRECISION_FP64, abi.PRECISION_MIXED])
+def test_the_iterate_at_the_cap_stays_on_the_edges(device, precision):
+    s = loop()
+    compare(device, s.problem, s.scene_extent, options(precision, abi.PCG_MAXIT_ACCEPT_ITERATE), solve_on_the_edges)
 
 
 @pytest.mark.parametrize("cams,lms", [(3, 60), (31, 2000), (32, 2000), (33, 2000), (65, 4000)])

@@ -43,6 +43,11 @@ def test_schedules_give_identical_results(device, solver, precision, max_pcg):
     outs = solve_all(device, pp, o)
     (ref, (p0, l0)) = outs[0]
     assert ref.result.total_pcg_iterations > 0
+    device.profile(True)
+    assert pp.solve(o).status == abi.OK
+    device.profile(False, reset=False)
+    product = "schur_apply" if solver == abi.SOLVER_MATRIX_FREE else "explicit_apply"
+    assert [n for n in ("schur_apply", "explicit_apply") if device.profile_query(n)["launches"]] == [product]
     for out, (p, l) in outs[1:]:
         assert out.iterations == ref.iterations
         assert out.result.final_cost == ref.result.final_cost
