@@ -601,8 +601,8 @@ int32_t vba_dense_solve_noalloc(vba_context* ctx, uint32_t n, const double* h, c
  *   M = ceil(coarse_nodes / coarse_group);
  * - structure_id: identifies `edges` across calls (0: unknown); while it
  *   stays the same the library reuses the edge index it derived.
- * The point elimination hook (`ReducedSolveAccelerator::eliminate`) is not
- * offered: blocks always come in offdiag. */
+ * - offdiag NULL with edges: the blocks that the point elimination below left
+ *   on the device. */
 typedef struct vba_reduced_system {
     uint64_t structure_id;
     uint32_t num_nodes;

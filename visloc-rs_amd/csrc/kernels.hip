@@ -1054,8 +1054,8 @@ __device__ void dense_solve_small(const DenseRows& io, double* S, double* work, 
 
 // ---------------------------------------------------------------------------
 // The same solve across the whole device, for systems larger than one
-// work-group holds: a right-looking Cholesky over 64-column panels, two
-// launches per panel, and a back substitution of one launch per panel.
+// work-group holds: a right-looking Cholesky over 64-column panels, a
+// launch per panel, and a back substitution of one launch per panel.
 //
 // k_chol_step, one launch per panel. Its first work-groups own 64 panel rows
 // each: they take the previous panel's part from the 64 x 64 diagonal block

@@ -327,13 +327,13 @@ void launch_dense_assemble(const DevProblem& P, const DensePairs& D, double* S, 
 // Solve S x = b (Cholesky, then an LU fallback with allow_lu, else singular)
 // for the variable poses; writes x and sets status[0] (0 ok, 1 singular);
 // status holds two words (the second records a failed pivot). S is
-// overwritten; `work` holds dense_work_size(n) doubles. Systems of more than kDenseOneGroupMax
-// unknowns are factored across the device (two launches per 64 columns, a
-// copy of S for the LU fallback in `work`), smaller ones by one work-group
-// that reads S and overwrites it only in the LU fallback.
-// Returns the error of the copy or of a launch.
-// The same solve for a plain system: S row-major n x n (overwritten), b and x
-// n long, always with the LU fallback.
+// overwritten; `work` holds dense_work_size(n) doubles. Systems of more than
+// kDenseOneGroupMax unknowns are factored across the device (a launch per 64
+// columns, a copy of S for the LU fallback in `work`), smaller ones by one
+// work-group that reads S and overwrites it only in the LU fallback.
+// Returns the error of the copy or of a launch. launch_dense_solve_plain is
+// the same for a plain system: S row-major n x n (overwritten), b and x n
+// long, always with the LU fallback.
 constexpr int32_t kDenseOneGroupMax = 256;
 // Doubles of `work`: the copy, then three vectors.
 constexpr size_t dense_work_size(size_t n) { return n * n + 3 * n; }
