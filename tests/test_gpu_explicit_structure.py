@@ -61,7 +61,9 @@ def test_the_lists_scratch_is_given_back(device):
     handle.free()
     terms, blocks = matrix_sizes(problem)
     lists = 12 * terms + blocks * (4 + 288) + (blocks + 16000) / 2 * 20 + 16000 * 60
-    assert used <= 1.02 * lists + (12 << 20)  # (allocations' granularity)
+    # the rest is the allocations' granularity and what the runtime takes for itself, 8 MB at a time (11 to 19 MB
+    # seen; 44 with the bitmaps)
+    assert used <= 1.02 * lists + (24 << 20)
 
 
 def test_structure_built_on_the_host(device):
@@ -86,6 +88,26 @@ def test_structure_built_on_the_host(device):
     assert device.profile_query("explicit_apply")["launches"] == 0
     assert again.iterations == a.iterations
     handle.free()
+
+
+@pytest.mark.parametrize("precision", [abi.PRECISION_FP64, abi.PRECISION_MIXED])
+@pytest.mark.parametrize("cameras,landmarks", [(65, 200), (66, 3000), (3000, 6000), (3001, 6000), (3003, 120000)])
+def test_few_and_many_rows_short_and_long_lists(device, cameras, landmarks, precision):
+    """Products with four waves a row (up to 3,000 rows) and with one, lists of
+    up to 40 terms a block summed by eight lanes and longer ones by a wave, the
+    last work-group not full: the steps are those of the product over the edges
+    (both to 1e-8, at a damping that lets CG get there)."""
+    problem = scene(cameras, landmarks)
+    kw = dict(precision=precision, max_iterations=3, initial_lambda=1e4, max_lambda=1e10,
+              pcg_maxit_policy=abi.PCG_MAXIT_ACCEPT_ITERATE)
+    a = device.optimize(problem, options(abi.SOLVER_MATRIX_FREE, **kw))
+    b = device.optimize(problem, options(abi.SOLVER_PCG_EXPLICIT, **kw))
+    assert a.status == b.status == abi.OK and a.accepted == b.accepted
+    step = np.linalg.norm(a.poses - problem.poses)
+    for x, y in zip(a.iterations, b.iterations):
+        assert 0 < x["pcg_iterations"] < 500 and 0 < y["pcg_iterations"] < 500
+        assert abs(x["max_pose_step"] - y["max_pose_step"]) <= 1e-6 * x["max_pose_step"]
+    assert np.linalg.norm(a.poses - b.poses) <= 1e-6 * max(step, 1e-3)
 
 
 def test_fixed_poses_do_not_count_against_the_lists(device):

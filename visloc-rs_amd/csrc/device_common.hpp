@@ -305,6 +305,21 @@ __device__ __forceinline__ int wave_entry36(int lane) {
     return ((lane & 32) ? 18 : 0) + ((lane & 16) ? 9 : 0) + w;
 }
 
+// The same over the 8 lanes of a group: lane g of it gets entries g, g + 8, ...
+// (five of them, or four where g > 3) in s.
+__device__ __forceinline__ void octet_sum36(const double v[36], int lane, double s[5]) {
+    double a[20], b[10];  // entries 8 m + (0..3 or 4..7), then 8 m + (0, 1 or 2, 3 of those)
+#pragma unroll
+    for (int i = 0; i < 20; ++i) {
+        const int e = 8 * (i / 4) + i % 4;
+        a[i] = halve_dpp<0x141>(v[e], e + 4 < 36 ? v[e + 4] : 0.0, lane & 4);  // row_half_mirror
+    }
+#pragma unroll
+    for (int i = 0; i < 10; ++i) b[i] = halve_dpp<0x4E>(a[4 * (i / 2) + i % 2], a[4 * (i / 2) + i % 2 + 2], lane & 2);  // quad_perm [2,3,0,1]
+#pragma unroll
+    for (int m = 0; m < 5; ++m) s[m] = halve_dpp<0xB1>(b[2 * m], b[2 * m + 1], lane & 1);  // quad_perm [1,0,3,2]
+}
+
 // Block b of sum_l W_p V_l^-1 W_q^T over its term list (landmark l, edge of
 // p, edge of q), W_p V_l^-1 W_q^T = [[C, -C K], [K C, -K C K]] with
 // C = G_p V_l^-1 G_q and K = [X_l]x, by one wave: entry wave_entry36(lane)
@@ -325,10 +340,10 @@ __device__ __forceinline__ int wave_entry36(int lane) {
 // With F32 the sum is of the mixed operator's blocks, its FP32-stored G and the
 // V^-1 that it pairs with them: G rounded as it loads gives the same values.
 template <bool F32>
-__device__ __forceinline__ double schur_block_wave(const DevProblem& P, const DensePairs& D, int b, int lane) {
+__device__ __forceinline__ void schur_block_terms(const DevProblem& P, const DensePairs& D, int b, int lane, int lanes,
+                                                  double acc[36]) {
     const double* const Vinv = F32 ? P.VinvM : P.Vinv64;
     auto stored = [](double2 v) { return F32 ? make_double2((float)v.x, (float)v.y) : v; };
-    double acc[36];
 #pragma unroll
     for (int i = 0; i < 36; ++i) acc[i] = 0.0;
     const int end = D.block_ptr[b + 1];
@@ -345,7 +360,7 @@ __device__ __forceinline__ double schur_block_wave(const DevProblem& P, const De
             const double2 p01 = stored(a2[0]), p23 = stored(a2[1]), p45 = stored(a2[2]);
             const double2 q01 = stored(b2[0]), q23 = stored(b2[1]), q45 = stored(b2[2]);
             const double x0 = X[0], x1 = X[1], x2 = X[2];
-            k += 64;
+            k += lanes;
             const int32_t* tn = D.terms + 3 * (size_t)min(k, end - 1);
             l = tn[0];
             ep = tn[1];
@@ -387,6 +402,14 @@ __device__ __forceinline__ double schur_block_wave(const DevProblem& P, const De
             if (k >= end) break;
         }
     }
+}
+
+// The block's sum by one wave: entry wave_entry36(lane) (row-major 6x6) in
+// each lane.
+template <bool F32>
+__device__ __forceinline__ double schur_block_wave(const DevProblem& P, const DensePairs& D, int b, int lane) {
+    double acc[36];
+    schur_block_terms<F32>(P, D, b, lane, 64, acc);
     return wave_sum36(acc, lane);
 }
 

@@ -7,10 +7,11 @@
 // one assembly per LM iteration each PCG product reads 36 values per stored
 // block instead of streaming every edge's G.
 //
-// Assembly: one wave per upper block sums the block's term list (one term per
-// landmark the two poses share, in landmark order) in a fixed order, then
-// writes S_pq and its transpose S_qp. Products: four waves per block row, 48
-// lanes of each as 6 rows x 8 column-block groups.
+// Assembly: one wave per upper block (an eighth of one where the lists are
+// short) sums the block's term list (one term per landmark the two poses share,
+// in landmark order) in a fixed order, then writes S_pq and its transpose S_qp.
+// Products: four waves per block row, or one where there are many rows, 48 lanes
+// of each as 6 rows x 8 column-block groups.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -266,32 +267,51 @@ __global__ __launch_bounds__(64) void k_explicit_fill(DevProblem P, ExplicitBuil
     }
 }
 
-// One upper block per wave: S_pq = [p == q](U_p + lambda I) - sum of its
-// terms, stored row-major at block_pos[2b] and transposed at
-// block_pos[2b + 1]. The diagonal block keeps its upper triangle and mirrors
-// it, so that it is exactly symmetric.
-template <bool F32>
+// One upper block per kLanes lanes (a wave, or an eighth of one): S_pq =
+// [p == q](U_p + lambda I) - sum of its terms, stored row-major at
+// block_pos[2b] and transposed at block_pos[2b + 1]. The diagonal block keeps
+// its upper triangle and mirrors it, so that it is exactly symmetric.
+template <bool F32, int kLanes>
 __global__ __launch_bounds__(kBlock, 4) void k_explicit_assemble(DevProblem P, DensePairs D, ExplicitDev X,
                                                                  double lambda) {
-    const int b = block_of_wave(D.num_blocks);
-    if (b >= D.num_blocks) return;
-    const int lane = threadIdx.x & 63;
-    double v = -schur_block_wave<F32>(P, D, b, lane);
-    const int sp = D.block_pq[2 * b], sq = D.block_pq[2 * b + 1];
-    const int pos = X.block_pos[2 * b], idx = wave_entry36(lane);
-    if (idx < 0) return;
-    const int i = idx / 6, j = idx % 6, tidx = 6 * j + i;
-    int pos_t = X.block_pos[2 * b + 1];
-    if (sp == sq) {
-        if (i > j) return;
-        v = P.U[21 * (size_t)sp + up6(i, j)] + (i == j && lambda > 0.0 ? lambda : 0.0) + v;
-        pos_t = i < j ? pos : -1;
+    constexpr int kPer = 64 / kLanes;  // blocks a wave
+    const int lane = threadIdx.x & 63, wave_block = kPer * block_of_wave((D.num_blocks + kPer - 1) / kPer);
+    if (wave_block >= D.num_blocks) return;
+    const int b = min(wave_block + lane / kLanes, D.num_blocks - 1);
+    double s[5];  // (minus) the sums of entries first, first + 8, ...
+    int first, count;
+    if constexpr (kLanes == 64) {
+        s[0] = -schur_block_wave<F32>(P, D, b, lane);
+        first = wave_entry36(lane);
+        count = first < 0 ? 0 : 1;
+    } else {
+        double acc[36];
+        schur_block_terms<F32>(P, D, b, lane % kLanes, kLanes, acc);
+        octet_sum36(acc, lane, s);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) s[i] = -s[i];
+        first = lane % kLanes;
+        count = wave_block + lane / kLanes < D.num_blocks ? (first > 3 ? 4 : 5) : 0;
     }
-    X.S64[36 * (size_t)pos + idx] = v;
-    if (X.S32) X.S32[36 * (size_t)pos + idx] = (float)v;
-    if (pos_t >= 0) {
-        X.S64[36 * (size_t)pos_t + tidx] = v;
-        if (X.S32) X.S32[36 * (size_t)pos_t + tidx] = (float)v;
+    const int sp = D.block_pq[2 * b], sq = D.block_pq[2 * b + 1];
+    const int pos = X.block_pos[2 * b], other = X.block_pos[2 * b + 1];
+#pragma unroll
+    for (int e = 0; e < (kLanes == 64 ? 1 : 5); ++e) {
+        if (e >= count) break;
+        const int idx = first + 8 * e, i = idx / 6, j = idx % 6, tidx = 6 * j + i;
+        double v = s[e];
+        int pos_t = other;
+        if (sp == sq) {
+            if (i > j) continue;
+            v = P.U[21 * (size_t)sp + up6(i, j)] + (i == j && lambda > 0.0 ? lambda : 0.0) + v;
+            pos_t = i < j ? pos : -1;
+        }
+        X.S64[36 * (size_t)pos + idx] = v;
+        if (X.S32) X.S32[36 * (size_t)pos + idx] = (float)v;
+        if (pos_t >= 0) {
+            X.S64[36 * (size_t)pos_t + tidx] = v;
+            if (X.S32) X.S32[36 * (size_t)pos_t + tidx] = (float)v;
+        }
     }
 }
 
@@ -315,40 +335,56 @@ __global__ __launch_bounds__(kBlock) void k_explicit_precond(DevProblem P, Expli
     for (int i = 0; i < 36; ++i) out[i] = inv[i];
 }
 
-// A block row's product by kRowWaves waves, two rows a work-group. Lane 8i + g
-// of wave w takes row i of the blocks 8 w + g, 8 w + g + 32, ... of the row,
-// kRowBlocks of them at a time.
+// A block row's product by kWaves waves. Lane 8i + g of wave w takes row i of
+// the blocks 8 w + g, 8 (w + kWaves) + g, ... of the row, kBlocks of them at a
+// time.
 //
-// The matrix is small (288 bytes a block; a loop's 60 blocks a row make 14 MB
-// for 800 poses) and stays in the L2s, so the product is bound by its chain of
-// dependent loads (row bounds, columns, vectors) and by the launch. A block a
-// lane and pass makes two passes of a row of 64 blocks, and the inputs of the
-// PCG scalars load with the first one. (Two blocks a lane: more registers and
-// the same time; eight waves a row: 8 to 20 % slower.) One wave a row, four
-// blocks at a time after the scalars, took 8.9 us at 210 poses (FP64 blocks)
-// and 11.1 us at 800 (FP32 blocks) by the trace; 5.6 and 8.7 us here.
-constexpr int kRowWaves = 4, kRowBlocks = 1;
-constexpr int kRowThreads = 64 * kRowWaves * kExplicitRows;
+// Few rows (explicit_group_rows): the matrix is small (288 bytes a block; a
+// loop's 60 blocks a row make 14 MB for 800 poses) and stays in the L2s, so the
+// product is bound by its chain of dependent loads (row bounds, columns,
+// vectors) and by the launch. Four waves a row and a block a lane and pass make
+// two passes of a row of 64 blocks, and the inputs of the PCG scalars load with
+// the first one. (Two blocks a lane: more registers and the same time; eight
+// waves a row: 8 to 20 % slower.) One wave a row, four blocks at a time after
+// the scalars, took 8.9 us at 210 poses (FP64 blocks) and 11.1 us at 800 (FP32
+// blocks) by the trace; 5.6 and 8.7 us here.
+//
+// Many rows fill the device by themselves, and every wave derives the PCG
+// scalars from all partials, so a row gets one wave, two blocks a lane, its
+// scalars first (fewer registers), and a work-group four rows (half the
+// partials that the step kernel's waves sum). Product and step with FP64
+// blocks, four waves a row against this: 24.1 and 23.1 us at 2,000 poses, 28.0
+// and 29.8 at 2,500, 30.6 and 30.1 at 3,000, 36.0 and 35.0 at 4,000, 58.3 and
+// 53.7 at 8,000, 96 and 75 at 16,000 with 56 blocks a row.
+template <int kWaves, int kBlocks, int kRows, bool kEarly>
+struct RowSplit {
+    static constexpr int waves = kWaves, blocks = kBlocks, rows = kRows, threads = 64 * kWaves * kRows;
+    static constexpr bool early = kEarly;      // the PCG scalars before the row's loads
+    static constexpr int stride = 8 * kWaves;  // blocks apart that a lane takes
+};
+using FewRows = RowSplit<4, 1, kExplicitFewRows, false>;
+using ManyRows = RowSplit<1, 2, kExplicitManyRows, true>;
 
 // Work-groups' rows: neighbouring rows on one XCD, whose L2 then holds their
 // part of the matrix and of the vectors they share.
+template <typename Split>
 __device__ __forceinline__ int row_groups(const DevProblem& P) {
-    return (P.num_pose_slots + kExplicitRows - 1) / kExplicitRows;
+    return (P.num_pose_slots + Split::rows - 1) / Split::rows;
 }
 
-template <typename TS>
+template <typename TS, int kBlocks>
 struct RowLoads {
-    int q[kRowBlocks];
-    TS s[kRowBlocks][6];
+    int q[kBlocks];
+    TS s[kBlocks][6];
 };
-// Blocks t, t + 32, ... of the row (clamped to its last block, whose product
-// the caller drops) and their columns.
-template <typename TS>
+// Blocks t, t + stride, ... of the row (clamped to its last block, whose
+// product the caller drops) and their columns.
+template <typename Split, typename TS>
 __device__ __forceinline__ void load_row_blocks(const ExplicitDev& X, const TS* __restrict__ S, int t, int last, int i,
-                                                RowLoads<TS>* r) {
+                                                RowLoads<TS, Split::blocks>* r) {
 #pragma unroll
-    for (int u = 0; u < kRowBlocks; ++u) {
-        const int tc = max(min(t + 8 * kRowWaves * u, last), 0);
+    for (int u = 0; u < Split::blocks; ++u) {
+        const int tc = max(min(t + Split::stride * u, last), 0);
         r->q[u] = X.col[tc];
         load6(S + 36 * (size_t)tc + 6 * i, r->s[u]);
     }
@@ -361,48 +397,54 @@ __device__ __forceinline__ double group8_sum(double v) {
     return v + dpp_partner<0x141>(v);  // row_half_mirror
 }
 
-// (S v)_p for v = v1 + beta v2 (v2 may be null) over blocks t, t + 32, ...
+// (S v)_p for v = v1 + beta v2 (v2 may be null) over blocks t, t + stride, ...
 // from the loaded ones on; `beta` is called once the vectors' loads are out
 // and false ends the launch (the same in every wave). The row's sum of row
 // component c is valid in lanes c < 6 of the row's wave 0.
-template <typename TS, typename Beta>
+template <typename Split, typename TS, typename Beta>
 __device__ __forceinline__ bool row_product(const ExplicitDev& X, const TS* __restrict__ S, int begin, int end,
                                             const double* __restrict__ v1, const double* __restrict__ v2, Beta beta,
                                             int lane, int wave, double (*sum)[8], double* y) {
     const int i = min(lane >> 3, 5), g = lane & 7, last = end - 1;
     int base = begin + 8 * wave, t = base + g;
-    RowLoads<TS> r;
-    load_row_blocks(X, S, t, last, i, &r);
+    RowLoads<TS, Split::blocks> r;
     double acc = 0.0, bt = 0.0;
+    if (Split::early && !beta(&bt)) return false;
+    load_row_blocks<Split>(X, S, t, last, i, &r);
     for (bool first = true;; first = false) {
-        double v[kRowBlocks][6], w[kRowBlocks][6];
+        double v[Split::blocks][6], w[Split::blocks][6];
 #pragma unroll
-        for (int u = 0; u < kRowBlocks; ++u) {
+        for (int u = 0; u < Split::blocks; ++u) {
             load6(v1 + 6 * (size_t)r.q[u], v[u]);
             if (v2) load6(v2 + 6 * (size_t)r.q[u], w[u]);
         }
-        if (first && !beta(&bt)) return false;
+        if (!Split::early && first && !beta(&bt)) return false;
 #pragma unroll
-        for (int u = 0; u < kRowBlocks; ++u)
-            if (t + 8 * kRowWaves * u < end)
+        for (int u = 0; u < Split::blocks; ++u)
+            if (t + Split::stride * u < end)
 #pragma unroll
                 for (int j = 0; j < 6; ++j)
                     acc = fma((double)r.s[u][j], v2 ? fma(bt, w[u][j], v[u][j]) : v[u][j], acc);
-        base += 8 * kRowWaves * kRowBlocks;
+        base += Split::stride * Split::blocks;
         t = base + g;
         if (base >= end) break;  // no lane of the wave has a block left
-        load_row_blocks(X, S, t, last, i, &r);
+        load_row_blocks<Split>(X, S, t, last, i, &r);
     }
     acc = group8_sum(acc);
     if (lane < 48 && g == 0) sum[wave][i] = acc;
     __syncthreads();
     *y = 0.0;
-    if (wave == 0 && lane < 6) *y = ((sum[0][lane] + sum[1][lane]) + sum[2][lane]) + sum[3][lane];
+    if (wave == 0 && lane < 6) {
+        *y = sum[0][lane];
+#pragma unroll
+        for (int w = 1; w < Split::waves; ++w) *y += sum[w][lane];
+    }
     return true;
 }
 
 // Sums (over lanes 0..5 of each row's wave 0, then over the work-group's
 // rows) into the work-group's partial.
+template <typename Split>
 __device__ __forceinline__ void rows_to_partial(double v0, double v1, bool head, int row, double (*lds)[2],
                                                 double* out) {
     if (head) {
@@ -416,23 +458,23 @@ __device__ __forceinline__ void rows_to_partial(double v0, double v1, bool head,
     __syncthreads();
     if (threadIdx.x < 2) {
         double a = lds[0][threadIdx.x];
-        for (int r = 1; r < kExplicitRows; ++r) a += lds[r][threadIdx.x];
+        for (int r = 1; r < Split::rows; ++r) a += lds[r][threadIdx.x];
         out[threadIdx.x] = a;
     }
 }
 
 // d_new = z + beta d_old and q = S d_new; d.q partials per work-group. The
 // work-groups first derive the iteration's scalars.
-template <typename TS>
-__global__ __launch_bounds__(kRowThreads) void k_pcg_explicit(DevProblem P, ExplicitDev X, const TS* __restrict__ S,
+template <typename TS, typename Split>
+__global__ __launch_bounds__(Split::threads) void k_pcg_explicit(DevProblem P, ExplicitDev X, const TS* __restrict__ S,
                                                               const double* __restrict__ d_old,
                                                               double* __restrict__ d_new, int k, int fresh) {
-    __shared__ double sum[kExplicitRows][kRowWaves][8], lds[kExplicitRows][2];
+    __shared__ double sum[Split::rows][Split::waves][8], lds[Split::rows][2];
     const PrologueIn pin = pcg_prologue_load(P, k);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int row = wv / kRowWaves, wave = wv % kRowWaves;
-    const int group = xcd_tile(blockIdx.x, row_groups(P)), p = group * kExplicitRows + row;
-    if (group >= row_groups(P)) return;
+    const int row = wv / Split::waves, wave = wv % Split::waves;
+    const int group = xcd_tile(blockIdx.x, row_groups<Split>(P)), p = group * Split::rows + row;
+    if (group >= row_groups<Split>(P)) return;
     const int pc = min(p, P.num_pose_slots - 1);
     const bool var = p < P.num_pose_slots && P.pose_var[pc] >= 0;
     const size_t kk = 6 * (size_t)pc + (lane < 6 ? lane : 0);
@@ -440,7 +482,7 @@ __global__ __launch_bounds__(kRowThreads) void k_pcg_explicit(DevProblem P, Expl
     double beta = 0.0, y;
     // (the first product of a solve or restart has d = z and d_old = 0, so
     // the term that beta = 0 multiplies is finite)
-    if (!row_product<TS>(X, S, X.row_ptr[pc], X.row_ptr[pc + 1], P.z, d_old,
+    if (!row_product<Split, TS>(X, S, X.row_ptr[pc], X.row_ptr[pc + 1], P.z, d_old,
                          [&](double* b) {
                              const bool go = pcg_prologue_finish(P, k, fresh, pin, &beta);
                              *b = beta;
@@ -455,24 +497,25 @@ __global__ __launch_bounds__(kRowThreads) void k_pcg_explicit(DevProblem P, Expl
         P.q[kk] = y;
         dq = dc * y;
     }
-    rows_to_partial(dq, 0.0, wave == 0, row, lds, P.bpart + 2 * (size_t)group);
+    rows_to_partial<Split>(dq, 0.0, wave == 0, row, lds, P.bpart + 2 * (size_t)group);
 }
 
 // r_t = b - S64 x; with restart r = r_t, z = M^-1 r_t, d = 0. Partials
 // (r_t.r_t, r_t.z) per work-group, as the implicit operator's check.
-__global__ __launch_bounds__(kRowThreads) void k_explicit_true_pose(DevProblem P, ExplicitDev X, int restart) {
-    __shared__ double sum[kExplicitRows][kRowWaves][8], lds[kExplicitRows][2];
+template <typename Split>
+__global__ __launch_bounds__(Split::threads) void k_explicit_true_pose(DevProblem P, ExplicitDev X, int restart) {
+    __shared__ double sum[Split::rows][Split::waves][8], lds[Split::rows][2];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int row = wv / kRowWaves, wave = wv % kRowWaves;
-    const int group = xcd_tile(blockIdx.x, row_groups(P)), p = group * kExplicitRows + row;
-    if (group >= row_groups(P)) return;
+    const int row = wv / Split::waves, wave = wv % Split::waves;
+    const int group = xcd_tile(blockIdx.x, row_groups<Split>(P)), p = group * Split::rows + row;
+    if (group >= row_groups<Split>(P)) return;
     const int pc = min(p, P.num_pose_slots - 1);
     const bool var = p < P.num_pose_slots && P.pose_var[pc] >= 0;
     const int c = lane < 6 ? lane : 0;
     const size_t k = 6 * (size_t)pc + c;
     const double bc = P.b[k];
     double y;
-    (void)row_product<double>(X, X.S64, X.row_ptr[pc], X.row_ptr[pc + 1], P.x, nullptr, [](double*) { return true; },
+    (void)row_product<Split, double>(X, X.S64, X.row_ptr[pc], X.row_ptr[pc + 1], P.x, nullptr, [](double*) { return true; },
                               lane, wave, sum[row], &y);
     double v[2] = {0.0, 0.0};
     if (var && wave == 0) {
@@ -489,7 +532,7 @@ __global__ __launch_bounds__(kRowThreads) void k_explicit_true_pose(DevProblem P
             }
         }
     }
-    rows_to_partial(v[0], v[1], wave == 0, row, lds, P.bpart + 2 * (size_t)group);
+    rows_to_partial<Split>(v[0], v[1], wave == 0, row, lds, P.bpart + 2 * (size_t)group);
 }
 
 }  // namespace
@@ -514,29 +557,42 @@ void launch_explicit_lists(const DevProblem& P, const ExplicitBuild& B, int32_t 
 void launch_explicit_assemble(const DevProblem& P, const DensePairs& D, const ExplicitDev& X, bool f32, double lambda,
                               hipStream_t s) {
     if (!D.num_blocks) return;
-    const auto kernel = f32 ? k_explicit_assemble<true> : k_explicit_assemble<false>;
-    hipLaunchKernelGGL(kernel, dim3(block_grid(D.num_blocks)), dim3(kBlock), 0, s, P, D, X, lambda);
+    const auto kernel = X.short_lists ? (f32 ? k_explicit_assemble<true, 8> : k_explicit_assemble<false, 8>)
+                                      : (f32 ? k_explicit_assemble<true, 64> : k_explicit_assemble<false, 64>);
+    const int waves = X.short_lists ? blocks_for(D.num_blocks, 8) : D.num_blocks;
+    hipLaunchKernelGGL(kernel, dim3(block_grid(waves)), dim3(kBlock), 0, s, P, D, X, lambda);
 }
 
 void launch_explicit_precond(const DevProblem& P, const ExplicitDev& X, hipStream_t s) {
     hipLaunchKernelGGL(k_explicit_precond, dim3(blocks_for(P.num_pose_slots, kBlock)), dim3(kBlock), 0, s, P, X);
 }
 
+namespace {
+template <typename TS>
+void launch_product(const DevProblem& P, const ExplicitDev& X, const TS* S, const double* d_old, double* d_new,
+                    int32_t pcg_iter, int32_t fresh, hipStream_t s) {
+    const int rows = explicit_group_rows(P.num_pose_slots);
+    const bool few = rows == FewRows::rows;
+    const auto kernel = few ? k_pcg_explicit<TS, FewRows> : k_pcg_explicit<TS, ManyRows>;
+    hipLaunchKernelGGL(kernel, dim3(xcd_grid(blocks_for(P.num_pose_slots, rows))),
+                       dim3(few ? FewRows::threads : ManyRows::threads), 0, s, P, X, S, d_old, d_new, (int)pcg_iter,
+                       (int)fresh);
+}
+}  // namespace
+
 void launch_pcg_explicit(const DevProblem& P, const ExplicitDev& X, bool fp32, const double* d_old, double* d_new,
                          int32_t pcg_iter, int32_t fresh, hipStream_t s) {
-    const dim3 grid(xcd_grid(blocks_for(P.num_pose_slots, kExplicitRows)));
-    if (fp32)
-        hipLaunchKernelGGL(k_pcg_explicit<float>, grid, dim3(kRowThreads), 0, s, P, X, (const float*)X.S32, d_old, d_new,
-                           (int)pcg_iter, (int)fresh);
-    else
-        hipLaunchKernelGGL(k_pcg_explicit<double>, grid, dim3(kRowThreads), 0, s, P, X, (const double*)X.S64, d_old, d_new,
-                           (int)pcg_iter, (int)fresh);
+    if (fp32) launch_product(P, X, (const float*)X.S32, d_old, d_new, pcg_iter, fresh, s);
+    else launch_product(P, X, (const double*)X.S64, d_old, d_new, pcg_iter, fresh, s);
 }
 
 void launch_explicit_true_residual(const DevProblem& P, const ExplicitDev& X, int32_t restart,
                                    const Post<PcgState>& post, hipStream_t s) {
-    hipLaunchKernelGGL(k_explicit_true_pose, dim3(xcd_grid(blocks_for(P.num_pose_slots, kExplicitRows))), dim3(kRowThreads), 0, s, P,
-                       X, (int)restart);
+    const int rows = explicit_group_rows(P.num_pose_slots);
+    const bool few = rows == FewRows::rows;
+    const auto kernel = few ? k_explicit_true_pose<FewRows> : k_explicit_true_pose<ManyRows>;
+    hipLaunchKernelGGL(kernel, dim3(xcd_grid(blocks_for(P.num_pose_slots, rows))),
+                       dim3(few ? FewRows::threads : ManyRows::threads), 0, s, P, X, (int)restart);
     launch_pcg_true_finish(P, restart, post, s);
 }
 

@@ -259,10 +259,22 @@ struct ExplicitDev {
     const int32_t* diag_pos;   // full position of S_pp per pose slot (-1: fixed pose)
     double* S64;               // 36 per full position
     float* S32;                // FP32 copy for the mixed-precision matvec (null in FP64)
+    bool short_lists;          // kExplicitShortList
 };
-// Block rows a work-group of the explicit products takes: each leaves one
-// partial in bpart.
-constexpr int kExplicitRows = 2;
+// Block rows a work-group of the explicit products takes (each leaves one
+// partial in bpart) with at most kExplicitFewPoses rows, and with more.
+constexpr int32_t kExplicitFewPoses = 3000;
+constexpr int kExplicitFewRows = 2, kExplicitManyRows = 4;
+constexpr int explicit_group_rows(int32_t poses) {
+    return poses <= kExplicitFewPoses ? kExplicitFewRows : kExplicitManyRows;
+}
+constexpr int32_t explicit_bparts(int32_t poses) {
+    return (poses + explicit_group_rows(poses) - 1) / explicit_group_rows(poses);
+}
+// Terms a block on average below which its list is short: an assembly by eight
+// lanes a block is then faster than by 64 (133 and 120 us at 38 terms, 784 and
+// 630 us at 31, 436 and 182 us at 5; 545 and 580 us at 57, 67 and 87 us at 56).
+constexpr int64_t kExplicitShortList = 40;
 // Building the explicit matrix's structure on the device from the problem's
 // edges: lpose is the pose of each l-order edge, bits the row bitmaps (nw
 // words a row) of the variable poses a pose shares a landmark with, itself

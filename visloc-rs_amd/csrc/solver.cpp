@@ -812,7 +812,7 @@ DevProblem bind(const Context& ctx, Prepared& pr, const vba_options& o, bool mix
         P.num_bpart = (int32_t)((NP + (kBlock / 64) - 1) / (kBlock / 64));
         P.num_cpart = (int32_t)((NP + (kBlock / 64) * kPosesPerWave - 1) / ((kBlock / 64) * kPosesPerWave));
         // (sized for the explicit product's work-groups too, which are more)
-        const size_t bparts = std::max<size_t>(P.num_bpart, (NP + kExplicitRows - 1) / kExplicitRows);
+        const size_t bparts = std::max(P.num_bpart, explicit_bparts((int32_t)NP));
         P.bpart = (double*)ensure(pr, B_BPART, 2 * std::max<size_t>(bparts, 1) * sizeof(double));
         P.cpart = (double*)ensure(pr, B_CPART, 2 * (size_t)std::max(P.num_cpart, 1) * sizeof(double));
         P.pcg = (PcgState*)ensure(pr, B_PCG, sizeof(PcgState));
@@ -942,6 +942,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
             D.terms = buf<int32_t>(pr, B_X_TERMS);
             X.num_blocks = pr.x_num_blocks;
             X.num_full = pr.x_num_full;
+            X.short_lists = count_terms(pr) < kExplicitShortList * X.num_blocks;
             X.block_pos = buf<int32_t>(pr, B_X_BLOCK_POS);
             X.row_ptr = buf<int32_t>(pr, B_X_ROW_PTR);
             X.col = buf<int32_t>(pr, B_X_COL);
@@ -956,7 +957,7 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         // P as the matrix's kernels take it: their partials, and the direction `d`
         auto over_matrix = [&](double* d) {
             DevProblem Px = P;
-            Px.num_bpart = (int32_t)((NP + kExplicitRows - 1) / kExplicitRows);
+            Px.num_bpart = explicit_bparts(P.num_pose_slots);
             Px.d = d;
             return Px;
         };
