@@ -1041,10 +1041,10 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         // Whether a matrix-free solve may change to the explicit matrix: only
         // where each step it takes is a converged one. The iterate of a solve
         // that is stopped at its cap unconverged hangs on the operator's
-        // rounding, FP64 rounding too: with ACCEPT_ITERATE, 163-camera submaps
-        // ended up to 10 % of the landmarks away (1 of 48; most within 1e-6)
-        // where one weak landmark decided whether a step was accepted. With
-        // REJECT, 110 loops ended within 2.6e-8.
+        // rounding, FP64 rounding too: with ACCEPT_ITERATE, 3 of 72 submaps of
+        // 100 to 300 cameras moved by 10 to 35 % of the landmarks (most by
+        // 1e-6), where one weak landmark decided whether a step was accepted.
+        // With REJECT, 110 loops ended within 2.6e-8.
         bool ask = matrix_free && !xplicit && !accept_iterate;
         const int32_t max_pcg = (int32_t)o.max_pcg_iterations;
         auto push = [&](const vba_iteration_stats& st) {
