@@ -1041,8 +1041,8 @@ int32_t run(Context& ctx, Prepared& pr, const vba_options& o, vba_iteration_stat
         // Whether a matrix-free solve may change to the explicit matrix: only
         // where each step it takes is a converged one. The iterate of a solve
         // that is stopped at its cap unconverged hangs on the operator's
-        // rounding, FP64 rounding too: with ACCEPT_ITERATE, 3 of 72 submaps of
-        // 100 to 300 cameras moved by 10 to 35 % of the landmarks (most by
+        // rounding, FP64 rounding too: with ACCEPT_ITERATE, 2 of 72 submaps of
+        // 100 to 300 cameras moved by 10 and 35 % of the landmarks (most by
         // 1e-6), where one weak landmark decided whether a step was accepted.
         // With REJECT, 110 loops ended within 2.6e-8.
         bool ask = matrix_free && !xplicit && !accept_iterate;
